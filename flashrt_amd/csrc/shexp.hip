@@ -9,6 +9,7 @@
 //     (h = g / (1 + exp(-g)) * u), or the down product. Q8_0 weights take Q8_0 activations (x and
 //     h quantized per 32 as the CPU path does, q8_0 . q8_0 per block as an exact integer dot, then
 //     scaled by d_w d_a); the other types take the fp32 activations.
+//     Taken up to 8 tokens; more go to k_shexp_mm, the same products on the matrix cores.
 //   - the layer with such a shared expert: router logits -> route_topk -> the routed experts as
 //     per-slot outputs (moe_hits for windows of up to 8 tokens, moe_q2::run for prefill chunks) ->
 //     the shared expert -> k_slot_combine (the routed slots in ascending expert id, then the shared
@@ -176,6 +177,305 @@ __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ 
     }
 }
 
+// ---- the same products for more tokens, on the matrix cores
+//
+// A workgroup takes 64 weight rows (DUAL: 32 gate rows and the same 32 up rows) against 16 NC tokens;
+// its four waves split K in quarters and add their sums in LDS as (q0 + q1) + (q2 + q3), so that a
+// chunk of a few hundred tokens still has several waves per SIMD and no wave runs a long serial K loop.
+// Operands go straight from global memory (each weight row is read by one wave; the activations come
+// from L2) into registers, one K-step ahead; no LDS and no barrier in the K loop.
+//   F32, F16, BF16 weights: the fp32 activations are split exactly into three bf16 planes
+//     (k_split3: 8 + 8 + 8 significant bits by truncation), the weights into one (BF16), two (F16) or
+//     three (F32), and every pair of parts is one v_mfma_f32_16x16x32_bf16 into one fp32 accumulator:
+//     exact products, fp32 sums, as the fmaf chains of k_shexp_mv.
+//   Q8_0 weights: v_mfma_i32_16x16x32_i8 per 32-block, an exact integer dot, then + float(s) * (d_w d_a),
+//     the terms of k_shexp_mv.
+// What bounds it: the L1 reads of the operands (six activation fragments and four weight fragments of
+// 1 KB per 24 matrix instructions), then the matrix cores. Measured (n = 2560, ff = 640; k_shexp_mv
+// before): see kShMmMinT.
+typedef short bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16v __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef int intx4 __attribute__((ext_vector_type(4)));
+
+// v = hi + mid + lo exactly, each with at most 8 significant bits (truncations: no part overflows);
+// an infinity or a NaN stays in hi alone
+__device__ __forceinline__ void split3(float v, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+    const uint32_t b = __float_as_uint(v);
+    hi = b & 0xffff0000u;
+    const float r = v - __uint_as_float(hi);
+    mid = __float_as_uint(r) & 0xffff0000u;
+    lo = __float_as_uint(r - __uint_as_float(mid));
+    if ((b & 0x7f800000u) == 0x7f800000u) {
+        if (b & 0x007fffffu) hi |= 0x00400000u;
+        mid = lo = 0;
+    }
+}
+// the upper halves of two floats' bits as one dword (a below b)
+__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+
+// planes [3][count] bf16 of count floats (a multiple of 8)
+__global__ void __launch_bounds__(256) k_split3(const float* __restrict__ x, size_t count, uint16_t* __restrict__ planes) {
+    const size_t i = (size_t(blockIdx.x) * 256 + threadIdx.x) * 8;
+    if (i >= count) return;
+    uint32_t w[3][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        uint32_t a[3], b[3];
+        split3(x[i + 2 * q], a[0], a[1], a[2]);
+        split3(x[i + 2 * q + 1], b[0], b[1], b[2]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) w[p][q] = pack_hi(a[p], b[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<uint4*>(planes + p * count + i) = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+}
+
+template <int TYPE>
+struct ShDense {
+    static constexpr int parts = TYPE == FRT_GGML_F32 ? 3 : TYPE == FRT_GGML_F16 ? 2 : 1;
+    static constexpr int words = TYPE == FRT_GGML_F32 ? 8 : 4;   // dwords of 8 weights
+    // the bf16 parts of 8 weights held as raw dwords
+    static __device__ __forceinline__ void split(const uint32_t (&raw)[words], bf16x8 (&out)[parts]) {
+        uint32_t w[parts][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if constexpr (TYPE == FRT_GGML_BF16) {
+                w[0][q] = raw[q];
+            } else {
+                float a, b;
+                if constexpr (TYPE == FRT_GGML_F32) {
+                    a = __uint_as_float(raw[2 * q]);
+                    b = __uint_as_float(raw[2 * q + 1]);
+                } else {
+                    a = h2f(uint16_t(raw[q] & 0xffffu));
+                    b = h2f(uint16_t(raw[q] >> 16));
+                }
+                uint32_t pa[3], pb[3];
+                split3(a, pa[0], pa[1], pa[2]);   // (fp16: 11 significant bits, the third part is 0)
+                split3(b, pb[0], pb[1], pb[2]);
+#pragma unroll
+                for (int p = 0; p < parts; ++p) w[p][q] = pack_hi(pa[p], pb[p]);
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < parts; ++p) out[p] = __builtin_bit_cast(bf16x8, make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]));
+    }
+};
+
+// out (DUAL): dense types the three planes [3][T][rows] of h = silu(gate) * up, Q8_0 its codes hq [T][rows]
+// and scales hd [T][rows / 32]; else of [T][rows] fp32. aq / ad or ap (planes [3][T][cols]): the input.
+template <int TYPE, bool DUAL, int NC>
+__global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1, const uint8_t* __restrict__ W2, int rows,
+                                                  int cols, const uint16_t* __restrict__ ap, const int8_t* __restrict__ aq,
+                                                  const float* __restrict__ ad, int T, float* __restrict__ of,
+                                                  uint16_t* __restrict__ op, int8_t* __restrict__ hq,
+                                                  float* __restrict__ hd) {
+    constexpr bool Q8 = TYPE == FRT_GGML_Q8_0;
+    __shared__ __align__(16) floatx4 part[4][NC][4][64];
+    __shared__ __align__(16) float s_dw[Q8 ? 4 : 1][4][2][16];   // per wave: the row tiles' block scales
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+    const int t0 = blockIdx.y * 16 * NC;
+    const int r0 = blockIdx.x * (DUAL ? 32 : 64);
+    int tok[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) tok[c] = min(t0 + 16 * c + li, T - 1);   // past the end: the last token again, not written
+    floatx4 acc[4][NC];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[i][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (Q8) {
+        // K-steps of 64: a pair of Q8_0 blocks, 68 bytes of a row. Lane group lg takes codes 8 lg .. 8 lg + 7
+        // of each block: bytes 2 + 8 lg (dwords 2 lg .. 2 lg + 2, shifted by two bytes) and 36 + 8 lg.
+        const size_t rb = size_t(cols / kQ8) * 34;
+        const int steps = cols / 64, s0 = steps * wave / 4, s1 = steps * (wave + 1) / 4;
+        const uint8_t* row[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            row[i] = DUAL ? (i < 2 ? W1 : W2) + size_t(r0 + 16 * (i & 1) + li) * rb : W1 + size_t(r0 + 16 * i + li) * rb;
+        struct Step {
+            uint32_t a[4][5];
+            uint2 b[NC][2];
+            float2 d[NC];
+        };
+        auto load = [&](int st, Step& s) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t* p = reinterpret_cast<const uint32_t*>(row[i] + size_t(st) * 68);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) s.a[i][q] = p[2 * lg + q];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) s.a[i][3 + q] = p[9 + 2 * lg + q];
+            }
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int8_t* x = aq + size_t(tok[c]) * cols + st * 64 + 8 * lg;
+                s.b[c][0] = *reinterpret_cast<const uint2*>(x);
+                s.b[c][1] = *reinterpret_cast<const uint2*>(x + 32);
+                s.d[c] = *reinterpret_cast<const float2*>(ad + size_t(tok[c]) * (cols / kQ8) + 2 * st);
+            }
+        };
+        auto mac = [&](const Step& s) {
+            // d_w of the pair's blocks by row: the first's in dword 0 (lane group 0), the second's in the
+            // upper half of dword 8 (lane group 3), through the wave's LDS to the lanes of rows 4 lg ..
+            float* sw = &s_dw[wave][0][0][0];
+            asm volatile("" ::: "memory");   // (a wave's LDS operations complete in order)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (lg == 0) sw[(i * 2) * 16 + li] = h2f(uint16_t(s.a[i][0] & 0xffffu));
+                if (lg == 3) sw[(i * 2 + 1) * 16 + li] = h2f(uint16_t(s.a[i][2] >> 16));
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const long a0 = __builtin_bit_cast(long, make_uint2(__builtin_amdgcn_alignbyte(s.a[i][1], s.a[i][0], 2),
+                                                                    __builtin_amdgcn_alignbyte(s.a[i][2], s.a[i][1], 2)));
+                const long a1 = __builtin_bit_cast(long, make_uint2(s.a[i][3], s.a[i][4]));
+                const float4 d0 = *reinterpret_cast<const float4*>(sw + (i * 2) * 16 + 4 * lg);
+                const float4 d1 = *reinterpret_cast<const float4*>(sw + (i * 2 + 1) * 16 + 4 * lg);
+                const float w0[4] = {d0.x, d0.y, d0.z, d0.w}, w1[4] = {d1.x, d1.y, d1.z, d1.w};
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const intx4 z = {0, 0, 0, 0};
+                    const intx4 v0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a0, __builtin_bit_cast(long, s.b[c][0]), z, 0, 0, 0);
+                    const intx4 v1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a1, __builtin_bit_cast(long, s.b[c][1]), z, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        acc[i][c][r] = fmaf(float(v0[r]), w0[r] * s.d[c].x, acc[i][c][r]);
+                        acc[i][c][r] = fmaf(float(v1[r]), w1[r] * s.d[c].y, acc[i][c][r]);
+                    }
+                }
+            }
+        };
+        Step a, b;
+        if (s0 < s1) load(s0, a);
+        for (int st = s0; st < s1; st += 2) {
+            load(min(st + 1, s1 - 1), b);
+            mac(a);
+            if (st + 1 < s1) {
+                load(min(st + 2, s1 - 1), a);
+                mac(b);
+            }
+        }
+    } else {
+        using D = ShDense<TYPE>;
+        constexpr int es = TYPE == FRT_GGML_F32 ? 4 : 2;   // bytes per weight
+        const int steps = cols / 32, s0 = steps * wave / 4, s1 = steps * (wave + 1) / 4;
+        const uint8_t* row[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            row[i] = (DUAL ? (i < 2 ? W1 : W2) + size_t(r0 + 16 * (i & 1) + li) * cols * es
+                           : W1 + size_t(r0 + 16 * i + li) * cols * es) + 8 * lg * es;
+        const size_t plane = size_t(T) * cols;
+        const uint16_t* xp[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) xp[c] = ap + size_t(tok[c]) * cols + 8 * lg;
+        struct Step {
+            uint32_t a[4][D::words];
+            bf16x8 b[NC][3];
+        };
+        auto load = [&](int st, Step& s) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int q = 0; q < D::words / 4; ++q) {
+                    const uint4 v = reinterpret_cast<const uint4*>(row[i] + size_t(st) * 32 * es)[q];
+                    s.a[i][4 * q] = v.x;
+                    s.a[i][4 * q + 1] = v.y;
+                    s.a[i][4 * q + 2] = v.z;
+                    s.a[i][4 * q + 3] = v.w;
+                }
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int p = 0; p < 3; ++p) s.b[c][p] = *reinterpret_cast<const bf16x8*>(xp[c] + p * plane + st * 32);
+        };
+        auto mac = [&](const Step& s) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                bf16x8 a[D::parts];
+                D::split(s.a[i], a);
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+#pragma unroll
+                    for (int pa = D::parts - 1; pa >= 0; --pa)   // the small products first
+#pragma unroll
+                        for (int pb = 2; pb >= 0; --pb)
+                            acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16v, a[pa]),
+                                                                                __builtin_bit_cast(bf16v, s.b[c][pb]),
+                                                                                acc[i][c], 0, 0, 0);
+            }
+        };
+        Step a, b;
+        if (s0 < s1) load(s0, a);
+        for (int st = s0; st < s1; st += 2) {
+            load(min(st + 1, s1 - 1), b);
+            mac(a);
+            if (st + 1 < s1) {
+                load(min(st + 2, s1 - 1), a);
+                mac(b);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[wave][c][i][lane] = acc[i][c];
+    __syncthreads();
+    if (wave >= NC) return;
+    // wave c finishes token column c: lane (token li, rows 16 i + 4 lg + r)
+    const int c = wave, t = t0 + 16 * c + li;
+    floatx4 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = (part[0][c][i][lane] + part[1][c][i][lane]) + (part[2][c][i][lane] + part[3][c][i][lane]);
+    if constexpr (!DUAL) {
+        if (t < T)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                *reinterpret_cast<floatx4*>(of + size_t(t) * rows + r0 + 16 * i + 4 * lg) = v[i];
+        return;
+    }
+    float h[2][4];
+    float am = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float g = v[i][r], u = v[2 + i][r];
+            h[i][r] = g / (1.0f + expf(-g)) * u;
+            am = fmaxf(am, fabsf(h[i][r]));
+        }
+    if constexpr (Q8) {   // the 32 rows are one Q8_0 block of h: its maximum over the four lanes of a token
+        am = fmaxf(am, __shfl_xor(am, 16, 64));
+        am = fmaxf(am, __shfl_xor(am, 32, 64));
+        const float d = q8_scale(am), id = q8_inv(d);
+        if (t < T) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                uint32_t q = 0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) q |= uint32_t(uint8_t(int8_t(q8_code(h[i][r], id)))) << (8 * r);
+                *reinterpret_cast<uint32_t*>(hq + size_t(t) * rows + r0 + 16 * i + 4 * lg) = q;
+            }
+            if (lg == 0) hd[size_t(t) * (rows / kQ8) + r0 / 32] = f16_round(d);
+        }
+    } else if (t < T) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            uint32_t p[4][3];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) split3(h[i][r], p[r][0], p[r][1], p[r][2]);
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                *reinterpret_cast<uint2*>(op + (size_t(q) * T + t) * rows + r0 + 16 * i + 4 * lg) =
+                    make_uint2(pack_hi(p[0][q], p[1][q]), pack_hi(p[2][q], p[3][q]));
+        }
+    }
+}
+
 // hit lists of moe_hits from routing ids: hit_ptr[t][k] = arena + ids[t][k] * stride for k < K, and,
 // with a shared blob, hit_ptr[t][K] = shared; hit_n[t] = the slots per token (K or K + 1)
 __global__ void k_hits_from_ids(const int32_t* __restrict__ ids, int T, int K, const uint8_t* arena, size_t stride,
@@ -210,17 +510,32 @@ __global__ void __launch_bounds__(256) k_slot_combine(int T, int K, int S, int n
     }
     __syncthreads();
     const float g = 1.0f / (1.0f + expf(-gate[t]));
-    for (int i = blockIdx.x * 256 + tid; i < n; i += gridDim.x * 256) {
-        float acc = 0.0f;
-        for (int r = 0; r < K; ++r) {
-            const float p = s_w[r] * Y[(size_t(t) * S + s_ord[r]) * n + i];
-            acc = acc + p;
-        }
-        const float p = sh[size_t(t) * sh_stride + i] * g;
-        float o = acc + p;
-        if (resid) o = resid[size_t(t) * n + i] + o;
-        out[size_t(t) * n + i] = o;
+    const int i = (blockIdx.x * 256 + tid) * 2;   // (n is even)
+    if (i >= n) return;
+    const float2 s = *reinterpret_cast<const float2*>(sh + size_t(t) * sh_stride + i);
+    float a0 = 0.0f, a1 = 0.0f;
+    for (int r0 = 0; r0 < K; r0 += 8) {   // eight slots' rows in flight
+        float2 y[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            y[q] = *reinterpret_cast<const float2*>(Y + (size_t(t) * S + s_ord[min(r0 + q, K - 1)]) * n + i);
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (r0 + q < K) {
+                const float w = s_w[r0 + q];
+                const float p0 = w * y[q].x, p1 = w * y[q].y;
+                a0 = a0 + p0;
+                a1 = a1 + p1;
+            }
     }
+    const float p0 = s.x * g, p1 = s.y * g;
+    float o0 = a0 + p0, o1 = a1 + p1;
+    if (resid) {
+        o0 = resid[size_t(t) * n + i] + o0;
+        o1 = resid[size_t(t) * n + i + 1] + o1;
+    }
+    out[size_t(t) * n + i] = o0;
+    out[size_t(t) * n + i + 1] = o1;
 }
 
 }  // namespace
@@ -258,8 +573,47 @@ static int shexp_mv(int type, bool dual, const void* W1, const void* W2, int row
 int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16* xhi, _Float16* xlo,
                 hipStream_t stream);
 
+// Calls of at least this many tokens run on the matrix cores (k_shexp_mm).
+constexpr int kShMmMinT = 9;
+
 size_t shexp_ws_bytes(int T, int n, int ffs) {
-    return up256(size_t(T) * ffs * 4) + up256(size_t(T) * ffs) + up256(size_t(T) * (ffs / kQ8) * 4);
+    const size_t mv = up256(size_t(T) * ffs * 4) + up256(size_t(T) * ffs) + up256(size_t(T) * (ffs / kQ8) * 4);
+    if (T < kShMmMinT) return mv;
+    const size_t mm = up256(size_t(T) * n * 6) + up256(size_t(T) * ffs * 6);   // the bf16 planes of x and h
+    return mv > mm ? mv : mm;
+}
+
+template <int TYPE, bool DUAL>
+static void shexp_mm(const uint8_t* W1, const uint8_t* W2, int rows, int cols, const uint16_t* ap, const int8_t* aq,
+                     const float* ad, int T, float* of, uint16_t* op, int8_t* hq, float* hd, hipStream_t stream) {
+    const int gx = rows / (DUAL ? 32 : 64);
+    // 32 tokens per workgroup halve the weights' L1 reads, where that leaves two workgroups per CU
+    if (gx * ((T + 31) / 32) >= 512)
+        k_shexp_mm<TYPE, DUAL, 2><<<dim3(gx, (T + 31) / 32), 256, 0, stream>>>(W1, W2, rows, cols, ap, aq, ad, T, of, op, hq, hd);
+    else
+        k_shexp_mm<TYPE, DUAL, 1><<<dim3(gx, (T + 15) / 16), 256, 0, stream>>>(W1, W2, rows, cols, ap, aq, ad, T, of, op, hq, hd);
+}
+
+template <int TYPE>
+static int shexp_run_mm(const void* g, const void* u, const void* d, int n, int ffs, const float* x, const int8_t* xq,
+                        const float* xd, int T, float* sh, void* ws, hipStream_t stream) {
+    const uint8_t *wg = static_cast<const uint8_t*>(g), *wu = static_cast<const uint8_t*>(u), *wd = static_cast<const uint8_t*>(d);
+    uint8_t* p = static_cast<uint8_t*>(ws);
+    if (TYPE == FRT_GGML_Q8_0) {
+        int8_t* hq = reinterpret_cast<int8_t*>(p);
+        float* hd = reinterpret_cast<float*>(p + up256(size_t(T) * ffs));
+        shexp_mm<TYPE, true>(wg, wu, ffs, n, nullptr, xq, xd, T, nullptr, nullptr, hq, hd, stream);
+        shexp_mm<TYPE, false>(wd, nullptr, n, ffs, nullptr, hq, hd, T, sh, nullptr, nullptr, nullptr, stream);
+    } else {
+        uint16_t* xp = reinterpret_cast<uint16_t*>(p);
+        uint16_t* hp = reinterpret_cast<uint16_t*>(p + up256(size_t(T) * n * 6));
+        const size_t count = size_t(T) * n;
+        k_split3<<<unsigned((count / 8 + 255) / 256), 256, 0, stream>>>(x, count, xp);
+        shexp_mm<TYPE, true>(wg, wu, ffs, n, xp, nullptr, nullptr, T, nullptr, hp, nullptr, nullptr, stream);
+        shexp_mm<TYPE, false>(wd, nullptr, n, ffs, hp, nullptr, nullptr, T, sh, nullptr, nullptr, nullptr, stream);
+    }
+    FRT_LAUNCHED("shared expert");
+    return kOk;
 }
 
 // sh [T][n] = the shared expert of type `type` on u [T][n]; uq/ud: u's Q8_0 (Q8_0 type only; may be
@@ -268,6 +622,12 @@ int shexp_run(int type, const void* g, const void* u, const void* d, int n, int 
               const float* xd, int T, float* sh, void* ws, hipStream_t stream) {
     if (!shexp_type_ok(type)) return set_error(kErrShape, "shared expert: ggml type %d (F32, F16, BF16 or Q8_0)", type);
     if (!shexp_shape_ok(n, ffs)) return set_error(kErrShape, "shared expert: n=%d ffs=%d", n, ffs);
+    if (T >= kShMmMinT) switch (type) {
+        case FRT_GGML_F32: return shexp_run_mm<FRT_GGML_F32>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
+        case FRT_GGML_F16: return shexp_run_mm<FRT_GGML_F16>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
+        case FRT_GGML_BF16: return shexp_run_mm<FRT_GGML_BF16>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
+        default: return shexp_run_mm<FRT_GGML_Q8_0>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
+    }
     uint8_t* p = static_cast<uint8_t*>(ws);
     float* h = reinterpret_cast<float*>(p);
     p += up256(size_t(T) * ffs * 4);
@@ -294,7 +654,7 @@ int hits_from_ids(const int32_t* ids, int T, int K, const uint8_t* arena, size_t
 int slot_combine(int T, int K, int S, int n, const int32_t* ids, const float* wts, const float* Y, const float* sh,
                  size_t sh_stride, const float* gate, const float* resid, float* out, hipStream_t stream) {
     if (K < 1 || K > 32) return set_error(kErrShape, "combine: K=%d", K);
-    const dim3 grid((n + 255) / 256 < 8 ? (n + 255) / 256 : 8, T);
+    const dim3 grid((n + 511) / 512, T);
     k_slot_combine<<<grid, 256, 0, stream>>>(T, K, S, n, ids, wts, Y, sh, sh_stride, gate, resid, out);
     FRT_LAUNCHED("combine");
     return kOk;

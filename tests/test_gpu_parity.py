@@ -1289,6 +1289,47 @@ def test_layer_dense_shared_expert(F, gtype, T):
     assert err <= H.OUT_REL
 
 
+@pytest.mark.parametrize("gtype", [H.GGML_Q8_0, H.GGML_F16, H.GGML_BF16, H.GGML_F32])
+@pytest.mark.parametrize("T,n,ffs", [(9, 512, 64), (16, 512, 64), (17, 1024, 192), (33, 512, 128), (700, 2560, 640)])
+def test_shared_expert_many_tokens(F, gtype, T, n, ffs):
+    """The dense shared expert on the matrix cores (from 9 tokens): edges of the 16- and 32-token and
+    32-row tiles, one to ten K-steps per wave, against float64 on the weights' exact values. The routed
+    experts have zero scales, so the layer gives sigmoid(gate) * shared. The dense types' products are
+    exact and summed in fp32: n and ffs terms in two products, 4 (n + ffs) 2^-24 of the rows' sizes covers
+    their roundings many times over. Q8_0 rounds h to codes, so a code may move by one step of its block
+    (1/127 of the block's largest value, one of ffs terms): 2e-3."""
+    E, K, ff = 16, 2, 128
+    rng = np.random.default_rng(T + gtype)
+    eb = F.expert_bytes(n, ff)
+    stride = (eb + 4095) // 4096 * 4096
+    arena = torch.zeros(E * stride, dtype=torch.uint8, device="cuda")
+    router = torch.from_numpy((rng.standard_normal((E, n)) * 0.02).astype(np.float32)).cuda()
+    gate = (rng.standard_normal(n) * 0.02).astype(np.float32)
+    raw = [H.dense_tensor(gtype, r, c, rng) for r, c in ((ffs, n), (ffs, n), (n, ffs))]
+    dv = [torch.from_numpy(a).cuda() for a in raw]
+    gate_d = torch.from_numpy(gate).cuda()
+    ml = F.MoeLayer(arena.data_ptr(), stride, E, 0, router, gate_d, n, ff, K)
+    ml.set_shared_dense(gtype, *dv, ffs)
+    x = rng.standard_normal((T, n)).astype(np.float32)
+    out = torch.full((T, n), float("nan"), dtype=torch.float32, device="cuda")
+    ml.forward(torch.from_numpy(x).cuda(), out, T=T)
+    torch.cuda.synchronize()
+    g, u, d = (H.dense_values(gtype, a, r, c) for a, (r, c) in zip(raw, ((ffs, n), (ffs, n), (n, ffs))))
+    xx = x.astype(np.float64)
+    if gtype == H.GGML_Q8_0:
+        q, s = O.quantize_q8(x)
+        xx = (q.reshape(T, n // 32, 32) * s.reshape(T, n // 32, 1).astype(np.float64)).reshape(T, n)
+    gg = xx @ g.T
+    h = gg / (1 + np.exp(-gg)) * (xx @ u.T)
+    if gtype == H.GGML_Q8_0:
+        q, s = O.quantize_q8(h.astype(np.float32))
+        h = (q.reshape(T, ffs // 32, 32) * s.reshape(T, ffs // 32, 1).astype(np.float64)).reshape(T, ffs)
+    ref = (h @ d.T) / (1 + np.exp(-(x.astype(np.float64) @ gate)))[:, None]
+    err = H.out_rel(out.cpu().numpy(), ref)
+    print(f"type {gtype} T {T} n {n} ffs {ffs}: {err:.2e}")
+    assert err <= (2e-3 if gtype == H.GGML_Q8_0 else 4 * (n + ffs) * 2.0 ** -24)
+
+
 def test_layer_dense_shared_expert_stack_norm(F):
     """Config 2 layers (RMS norm, Zipf bias, residual) with a Q8_0 shared expert of ff 512, chained
     by a two-layer stack call (layer by layer: the persistent kernels take only the Q2_0 blob), each
