@@ -28,6 +28,7 @@ constexpr int kChunk = 256;    // slots per dispatch chunk (one wave of k_pf_pla
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 namespace {
 
@@ -259,31 +260,34 @@ __global__ void __launch_bounds__(64) k_pf_place(const int32_t* __restrict__ ids
 // Codes 4..7 of each half are shifted down by 8 first. Per pair of weights: one v_and_or_b32,
 // one v_pk_add_f16 and one v_pk_mul_f16 (plus one shift per 16 weights).
 //
-// k_pf_gemm<SMALL>: the gate/up GEMM. A tile's A rows are ff rows f0 .. of gate and the same rows of
-// up; wave w owns 32 of them (2 gate + 2 up tiles of 16), so SwiGLU and the Q8_0 of a 32-row block
-// of h (quant/q2_0/moe_cpu.cpp:43-61) are lane-local; h = code * d is written as fp16 for the down
-// GEMM. Two shapes:
-//   SMALL = false: 256 threads (4 waves), 64 tokens x 128 ff rows, activation stages of K = 64 (a
-//                  48 KB ring), so two workgroups share a CU and one computes while the other waits
-//                  for its loads; the tile classes of 2-4 token columns (one branch-free variant per
-//                  column count).
-//   SMALL = true:  256 threads, 16 tokens x 128 ff rows, stages of K = 256 in a ring of 2, for the tiles of one
-//                  token column (half of them under skewed routing): a quarter of the LDS and of the
-//                  registers, so 4 workgroups share a CU.
-// Every activation fragment read from LDS feeds 4 MFMAs, every dequantized weight fragment NC NP.
+// k_pf_gemm<DOWN, SMALL>: 256 threads, 64 weight rows (A) per wave against the tokens (B) of one tile.
+// Gate/up: wave w takes ff rows f0 + 32 w .. of gate and the same 32 of up, so SwiGLU and the Q8_0 of a
+// 32-row block of h (quant/q2_0/moe_cpu.cpp:43-61) stay in the wave; h = code * d is written as fp16
+// for the down GEMM. Down: wave w takes output rows r0 + 64 w .., K = ff.
+//   SMALL = false: tiles of 17-64 tokens, v_mfma_f32_32x32x16_f16 (two row tiles x one or two token
+//                  columns of 32), activation stages of K = 64. A 32x32 product holds the matrix core
+//                  32 cycles and the issue port about 10, so five of the dequantization's VALU
+//                  instructions hide behind each (a 16x16 one: 16 and 9, two); both measured with
+//                  chains of independent products and VALU instructions. In the kernel the two add up
+//                  all the same: MFMA 47% and VALU 43% of the SIMD cycles at 2048 tokens.
+//   SMALL = true:  tiles of up to 16 tokens, v_mfma_f32_16x16x32_f16 (four row tiles), stages of
+//                  K = 256; bound by the dequantization (26 VALU instructions per 16 x 64 weights).
 //
-// K order (perm256_pos): within each 256-element stretch, MFMA lane group g takes block g of the
-// stretch. So the weights go straight from HBM into registers: lane (row i, group g) loads the
-// 16-byte code chunk of block g of its row, and the 4 lanes of a row read 64 contiguous bytes (a
-// weight row is a separate 512-byte stretch of HBM; one lane per row and 16-byte chunk would make
-// every lane a separate cache-line request). Each wave loads only its own rows, one stretch ahead,
-// into a second register set.
+// K order (perm256_pos): within each 256-element stretch, MFMA lane group g (16x16: four groups; 32x32:
+// two, of blocks 2 p + g for p = 0, 1) takes one block's 16-byte code chunk, dword by dword.
 //
-// Activations go through LDS: stages of 64 or 128 K in a ring of 3 slots
-// filled by direct global-to-LDS loads (global_load_lds: each lane's 16 bytes land at the wave's LDS
-// base + 16 lane, no registers), issued 2 stages ahead; one workgroup barrier per stage. Slot layout:
-//   [NP][tokens][cpt chunks of 8 fp16], chunk kc of token j at j * cpt + (kc ^ (j % cpt)), so that the
-//   lanes of a 128-bit read phase (one chunk of 8 tokens) hit distinct bank groups.
+// Weights go through the wave's own LDS (no barrier): 64 rows x 64 bytes of codes and 64 x 4 scales per
+// stretch by direct global-to-LDS loads whose four consecutive lanes read one row's 64 bytes. Loaded
+// straight into the MFMA's registers, each lane of a quad is another row, and the L1 takes one clock
+// per lane instead of one per 64 bytes: 17 against 59 bytes per clock and CU (measured, L2-resident
+// rows). Chunk c of row r sits at c ^ ((r >> 2) & 3), so that the sixteen lanes of a read phase hit
+// distinct banks. A stretch's weights are read
+// into registers at its start; the next stretch's then load into the same LDS.
+//
+// Activations go through LDS too: stages in a ring of slots filled by direct global-to-LDS loads
+// (global_load_lds: each lane's 16 bytes land at the wave's LDS base + 16 lane, no registers), issued
+// `ahead` stages ahead; one workgroup barrier per stage. Slot layout:
+//   [NP][tokens][cpt chunks of 8 fp16], chunk kc of token j at j * cpt + (kc ^ swz(j)) (GemmShape).
 // Issue order of k_pf_gemm's loads, as stages s of the same pattern: stage s issues the weights of
 // stretch s / sps + 1 when s is a stretch's first (s % sps == 0: "A"), then the activations of stage
 // s + ahead ("B"). The prologue is the stages s = -max(ahead, sps) .. -1 of that pattern (A of
@@ -319,22 +323,27 @@ constexpr bool gu_waits_ok(int ahead, int sps, int kDB, int kDA) {
         if (gu_after_b(st, ahead, sps, kDB, kDA) != gu_wait(gu_mod(st, sps), ahead, sps, kDB, kDA)) return false;
     return true;
 }
-template <bool SMALL>
-struct GuShape {
-    static constexpr int threads = 256;
+template <bool DOWN, bool SMALL>
+struct GemmShape {
+    static constexpr int parts = DOWN ? 1 : 2;            // activation parts (h as one fp16 value, x as hi and lo)
     static constexpr int tokens = SMALL ? 16 : kTN;       // activation rows in LDS
-    static constexpr int ff_rows = threads / 2;           // ff rows per workgroup (32 per wave)
+    static constexpr int rows = DOWN ? 256 : 128;         // output rows (down) / ff rows (gate/up) per workgroup
     static constexpr int stage_k = SMALL ? 256 : 64;      // K per activation stage
     static constexpr int sps = 256 / stage_k;             // stages per weight stretch
-    static constexpr int ksps = stage_k / 32;             // MFMA K-steps per stage
     static constexpr int cpt = stage_k / 8;               // 16-byte chunks per token per stage
     static constexpr int slot_b = tokens * stage_k * 2;   // bytes per part per slot
-    static constexpr int stages = SMALL ? 2 : 3;          // activation ring slots
+    static constexpr int stages = SMALL ? 2 : DOWN ? 4 : 2;   // activation ring slots
     static constexpr int ahead = stages - 1;              // stages issued ahead
-    static constexpr int smem = stages * 2 * slot_b;
-    static constexpr int dma = tokens * cpt / threads;    // activation loads per lane per part
-    static constexpr int min_waves = SMALL ? 4 : 2;       // per SIMD (SMALL: 4 workgroups per CU)
-    static_assert(sps <= 4 && gu_waits_ok(ahead, sps, dma * 2, 8), "the wait counts of k_pf_gemm");
+    static constexpr int ring_b = stages * parts * slot_b;
+    static constexpr int wave_a = 64 * 64 + 64 * 16;      // a wave's weights: codes of one stretch, scales of two
+    static constexpr int smem = ring_b + 4 * wave_a;
+    // chunk kc of token j sits at kc ^ swz(j): the sixteen tokens of a 256-byte read phase (64 banks) take
+    // sixteen different 16-byte columns (two tokens of 128 bytes share a row of the banks when cpt = 8)
+    static __device__ __forceinline__ int swz(int j) { return (cpt == 8 ? j >> 1 : j) & (cpt - 1); }
+    static constexpr int dma = tokens * cpt / 256;        // activation loads per lane per part
+    static constexpr int kDB = dma * parts, kDA = 6;      // loads per stage (activations) and stretch (weights)
+    static_assert(sps <= 4 && gu_waits_ok(ahead, sps, kDB, kDA), "the wait counts of k_pf_gemm");
+    static_assert(!DOWN || tokens * (256 + 4) * (SMALL ? 4 : 2) <= smem, "the down epilogue's staging");
 };
 
 
@@ -343,6 +352,10 @@ typedef const __attribute__((address_space(1))) void* gbl_ptr_t;
 // direct global -> LDS load of 16 bytes per lane to lds_base + 16 lane (lds_base uniform)
 __device__ __forceinline__ void ldsdma16(const void* g, void* lds_base) {
     __builtin_amdgcn_global_load_lds((gbl_ptr_t)g, (lds_ptr_t)lds_base, 16, 0, 0);
+}
+// the same with 4 bytes per lane, to lds_base + 4 lane
+__device__ __forceinline__ void ldsdma4(const void* g, void* lds_base) {
+    __builtin_amdgcn_global_load_lds((gbl_ptr_t)g, (lds_ptr_t)lds_base, 4, 0, 0);
 }
 // A workgroup barrier that does not wait for outstanding global loads (__syncthreads' release fence
 // would wait for all of them, the ring's later stages included): this wave's LDS accesses complete,
@@ -353,6 +366,14 @@ __device__ __forceinline__ void ring_barrier() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0); vmcnt and expcnt not waited for
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+// this wave's LDS reads have returned, before anything after this is issued (direct global-to-LDS loads
+// may then overwrite what they read)
+__device__ __forceinline__ void lds_reads_done() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 }
@@ -410,242 +431,13 @@ __device__ __forceinline__ int lane_xor32(int v) {
 __device__ __forceinline__ floatx4 mfma_acc(half8 a, half8 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ floatx16 mfma_acc(half8 a, half8 b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
 
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
 
-template <bool SMALL>
-__global__ void __launch_bounds__(GuShape<SMALL>::threads, GuShape<SMALL>::min_waves)
-k_pf_gemm(const uint8_t* __restrict__ arena, size_t stride, int E, const uint8_t* __restrict__ shared_blob, int n,
-          int np, int hblk, int ff, const _Float16* __restrict__ bhi, const _Float16* __restrict__ blo,
-          const int32_t* __restrict__ tok_of, const int32_t* __restrict__ bounds, const int2* __restrict__ tiles,
-          const int32_t* __restrict__ n_tiles, _Float16* __restrict__ hout) {
-    using Sh = GuShape<SMALL>;
-    constexpr int NP = 2;
-    constexpr int kDB = Sh::dma * NP;   // activation loads per lane per stage
-    constexpr int kDA = 8;              // weight loads per lane per stretch (4 code chunks + 4 scales)
-    // A 1-D grid of gx ff-slices x tiles (tiles rounded up to a multiple of 8). Workgroup L runs on
-    // XCD L % 8, so the slices of a tile are placed 8 apart: they run on the same XCD at about the same
-    // time, and the tile's activations come into that XCD's L2 once.
-    const int gx = ff / Sh::ff_rows;
-    const int ffp = (ff + 255) & ~255;   // h row length
-    const int L = blockIdx.x, r8 = L >> 3;
-    const int slice = r8 % gx, t = (L & 7) + 8 * (r8 / gx);
-    // n_tiles[0]: tiles in all; n_tiles[1]: the first tile of one token column (the list is ordered
-    // longest first). The small shape takes those, the other the rest.
-    const int ti = SMALL ? n_tiles[1] + t : t;
-    if (ti >= (SMALL ? n_tiles[0] : n_tiles[1])) return;
-    extern __shared__ __align__(16) uint8_t smem[];
-    __shared__ int sRow[Sh::tokens];
-    const int2 tile = tiles[ti];
-    const int grp = tile.x;
-    const int row0 = bounds[grp] + tile.y;
-    const int cnt = min(Sh::tokens, bounds[grp + 1] - row0);
-    const uint8_t* blob = grp < E ? arena + size_t(grp) * stride : shared_blob;
-    const int nbk = n / kBlock;   // weight blocks per row
-    const size_t mb = mat_bytes(ff, n);
-    const int rbase = slice * Sh::ff_rows;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int li = lane & 15, lg = lane >> 4;
-    // activation row of each tile token; past the group's end the first repeats (never written)
-    if (tid < Sh::tokens) sRow[tid] = tok_of[row0 + min(tid, cnt - 1)];
-    __syncthreads();
-
-    // this lane's weight rows: ff row rbase + 32 wave + 16 (i & 1) + li of gate (i < 2) and up;
-    // rows past the end load any row and are never stored. aoff = row * nbk: the chunk and scale
-    // index of the row's block 0. K runs to np (n rounded up to 512, the activations zero past n):
-    // a block past the row's last is read as its last, whose finite products with zeros are 0.
-    const uint8_t* const mG = blob;
-    const uint8_t* const mU = blob + mb;
-    const size_t scale_off = size_t(ff) * nbk * 16;
-    uint32_t aoff[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) aoff[i] = uint32_t(min(rbase + 32 * wave + 16 * i + li, ff - 1)) * nbk;
-    struct ARegs {
-        uint4 cw[4];
-        uint32_t sc[4];
-    };
-    auto load_a = [&](int q, ARegs& a) {   // stretch q (blocks 4q + lg)
-        const int bq = min(4 * q + lg, nbk - 1);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint8_t* m = i < 2 ? mG : mU;
-            const size_t o = size_t(aoff[i & 1]) + bq;
-            a.cw[i] = gld_u4(m + o * 16);
-            a.sc[i] = gld<uint16_t>(m + scale_off + o * 2);
-        }
-    };
-    // this thread's activation chunks of a stage: LDS positions P = threads p + tid (token P / 16)
-    uint32_t boff[Sh::dma];   // element offsets (rows * n stays below 2^31)
-#pragma unroll
-    for (int p = 0; p < Sh::dma; ++p) {
-        const int P = Sh::threads * p + tid, j = P / Sh::cpt, kc = (P % Sh::cpt) ^ (j & (Sh::cpt - 1));
-        boff[p] = uint32_t(sRow[j]) * np + kc * 8;
-    }
-    auto issue_b = [&](int st, int slot) {
-        uint8_t* b = smem + slot * NP * Sh::slot_b;
-#pragma unroll
-        for (int p = 0; p < Sh::dma; ++p) {
-            ldsdma16(bhi + boff[p] + size_t(st) * Sh::stage_k, b + p * Sh::threads * 16 + wave * 1024);
-            ldsdma16(blo + boff[p] + size_t(st) * Sh::stage_k, b + Sh::slot_b + p * Sh::threads * 16 + wave * 1024);
-        }
-    };
-    floatx4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[i][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    const DqMagic mg = dq_magic();
-
-    // K-step t of stage st (K-step tt of the stretch whose weights are in a), by token column: column
-    // 0's activations are read first, the 4 A fragments dequantized while they land, then each
-    // column's MFMAs run while the next column's activations are read (two column buffers).
-    auto kstep = [&](auto nc, int st, int t, const ARegs& a, int tt) {
-        constexpr int NC = decltype(nc)::value;
-        const half8* sb = reinterpret_cast<const half8*>(smem + (st % Sh::stages) * NP * Sh::slot_b);
-        auto rd = [&](int c, half8(&b)[NP]) {
-            const int j = c * 16 + li, kc = t * 4 + lg;
-#pragma unroll
-            for (int part = 0; part < NP; ++part) b[part] = sb[part * (Sh::slot_b / 16) + j * Sh::cpt + (kc ^ (j & (Sh::cpt - 1)))];
-        };
-        half8 b0[NP], b1[NP];
-        rd(0, b0);
-        half8 av[4];
-        const int d = tt >> 1;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint4 w = a.cw[i];
-            const uint32_t cw = d == 0 ? w.x : d == 1 ? w.y : d == 2 ? w.z : w.w;
-            const _Float16 sc = __builtin_bit_cast(_Float16, uint16_t(a.sc[i]));
-            av[i] = dequant8((tt & 1) ? cw >> 8 : cw, half2v{sc, sc}, mg);
-        }
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            half8(&cur)[NP] = (c & 1) ? b1 : b0;
-            half8(&nxt)[NP] = (c & 1) ? b0 : b1;
-            if (c + 1 < NC) rd(c + 1, nxt);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int part = 0; part < NP; ++part) acc[i][c] = mfma_acc(av[i], cur[part], acc[i][c]);
-        }
-    };
-
-    // Stage st (K = stage_k st ..) is part h = st % sps of stretch st / sps. Per stage st, after its
-    // barrier: A stretch st / sps + 1 (first stage of a stretch, h = 0), then B stage st + ahead (the
-    // issue pattern of gu_wait). Waiting for B stage st (vmcnt: the loads issued after it may stay
-    // outstanding) covers everything issued before it, A stretch st / sps included. The pattern is
-    // the same for every stage: past the end, the last stretch / stage is loaded again (into
-    // registers / a slot nothing reads any more), so the wait counts are constants and the
-    // compiler's own waits for the weight registers never see a path without later loads (at such
-    // a merge it would wait for every load in flight).
-    const int nst = np / Sh::stage_k;   // stages
-    const int nq = np / 256;            // stretches (even)
-    auto run = [&](auto nc) {
-        ARegs a0, a1;   // stretches of even / odd index (named, so they stay in registers)
-        // the loads of stages -max(ahead, sps) .. -1 of the steady-state pattern below
-#pragma unroll
-        for (int s = -(Sh::ahead > Sh::sps ? Sh::ahead : Sh::sps); s < 0; ++s) {
-            if (gu_mod(s, Sh::sps) == 0 && s >= -Sh::sps) load_a(0, a0);
-            if (s >= -Sh::ahead) issue_b(min(s + Sh::ahead, nst - 1), s + Sh::ahead);
-        }
-        // the two stages of stretch q, whose weights are in cur; the next stretch loads into nxt
-        auto stretch = [&](int q, const ARegs& cur, ARegs& nxt) {
-#pragma unroll
-            for (int h = 0; h < Sh::sps; ++h) {
-                const int st = Sh::sps * q + h;
-                // loads issued after B stage st (by stages st - ahead + 1 .. st - 1) may stay outstanding
-                switch (h) {
-                    case 0: wait_vm<gu_wait(0, Sh::ahead, Sh::sps, kDB, kDA)>(); break;
-                    case 1: wait_vm<gu_wait(1, Sh::ahead, Sh::sps, kDB, kDA)>(); break;
-                    case 2: wait_vm<gu_wait(2, Sh::ahead, Sh::sps, kDB, kDA)>(); break;
-                    default: wait_vm<gu_wait(3, Sh::ahead, Sh::sps, kDB, kDA)>(); break;
-                }
-                ring_barrier();   // stage st is in LDS for every wave; every wave is done with stage st - 1
-                if (h == 0) load_a(min(q + 1, nq - 1), nxt);
-                issue_b(min(st + Sh::ahead, nst - 1), (st + Sh::ahead) % Sh::stages);   // into stage st - 1's slot
-#pragma unroll
-                for (int t = 0; t < Sh::ksps; ++t) kstep(nc, st, t, cur, Sh::ksps * h + t);
-            }
-        };
-        for (int q = 0; q < nq; q += 2) {   // nq is even
-            stretch(q, a0, a1);
-            stretch(q + 1, a1, a0);
-        }
-    };
-    if constexpr (SMALL) {
-        run(std::integral_constant<int, 1>{});
-    } else {
-        switch ((cnt + 15) / 16) {   // token columns with at least one real token (2..4 here)
-            case 2: run(std::integral_constant<int, 2>{}); break;
-            case 3: run(std::integral_constant<int, 3>{}); break;
-            default: run(std::integral_constant<int, 4>{}); break;
-        }
-    }
-
-    // lane: token column c*16 + li; ff rows f = rbase + 32 wave + 16 i + 4 lg + r (i = 0, 1) for gate
-    // (acc[i]) and up (acc[2 + i]). The 32 rows of the wave are one Q8_0 block of h.
-    const int fbase = rbase + 32 * wave;
-#pragma unroll
-    for (int c = 0; c < (SMALL ? 1 : 4); ++c) {
-        const int col = c * 16 + li;
-        float hv[2][4];
-        float am = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                hv[i][r] = silu_mul(acc[i][c][r], acc[2 + i][c][r]);
-                am = fmaxf(am, fabsf(hv[i][r]));
-            }
-        am = fmaxf(am, __builtin_bit_cast(float, lane_xor16(__builtin_bit_cast(int, am))));
-        am = fmaxf(am, __builtin_bit_cast(float, lane_xor32(__builtin_bit_cast(int, am))));
-        if (hblk == 64) {   // ff rows 64 m .. 64 m + 63 are waves 2m' and 2m' + 1 (rbase is a multiple of 128)
-            wait_vm<0>();      // the ring's last direct-to-LDS loads (repeats past the end) have landed
-            __syncthreads();   // (uniform: hblk is a kernel argument) every wave is past its last LDS read
-            float* sam = reinterpret_cast<float*>(smem);
-            if (lg == 0) sam[wave * 16 + li] = am;
-            __syncthreads();
-            am = fmaxf(am, sam[(wave ^ 1) * 16 + li]);
-        }
-        const float d = q8_scale(am);
-        const float id = q8_inv(d);
-        const float dr = f16_round(d);
-        if (col < cnt && fbase < ff) {
-            const size_t row = size_t(row0 + col);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int f = fbase + 16 * i + 4 * lg + r;
-                    const float a = float(q8_code(hv[i][r], id)) * dr;
-                    hout[row * ffp + (f & ~255) + perm256_pos(f & 255)] = _Float16(a);
-                }
-        }
-    }
-    // h rows are ffp = ff rounded up to 256 long (whole perm256 stretches for the down GEMM); the
-    // slice holding the last rows also writes zeros at the pad's positions, so that the down GEMM's
-    // products there are 0 (its weights for the pad are any finite values of the row)
-    if (ffp > ff && rbase + Sh::ff_rows >= ff) {
-        const int np = ffp - ff;   // pad elements per row: f = ff .. ffp - 1
-        for (int i = tid; i < cnt * np; i += Sh::threads) {
-            const int col = i / np, f = ff + i % np;
-            hout[size_t(row0 + col) * ffp + (f & ~255) + perm256_pos(f & 255)] = _Float16(0.0f);
-        }
-    }
-}
-
-// k_pf_down: the down GEMM, one workgroup (256 threads) per tile. The tile's activations (h of 64
-// dispatched rows, all of K = ffp = ff rounded up to 256, perm256 order, zeros in the pad) are loaded
-// into LDS once (64 tokens x ffp fp16; chunk kc of token j at j * ffp / 8 + (kc ^ (j & 15))), then
-// the workgroup walks all n output rows in blocks
-// of 256 (wave w: rows 64 w + 16 i + li of the block), streaming the weights straight into
-// registers with three stretches of lookahead (four register sets). No barrier after the
-// activation load: each wave reads only its own weights. Two workgroups share a CU (64 KB of LDS
-// each for ff = 512), so one computes while the other waits for loads. NQ = ffp / 256 stretches per
-// row block; a weight block past the row's last (the pad) is read as the row's last block, whose
-// finite products with the pad's zeros are 0. TAIL: the stretch count is not a multiple of 4, and
-// the last round of 4 steps has steps past the end (loads repeated, no products).
 // 4 consecutive per-slot outputs as float, fp16 or bf16 (round to nearest even)
 __device__ __forceinline__ void store4(float* p, floatx4 v) { *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]); }
 __device__ __forceinline__ void store4(_Float16* p, floatx4 v) {
@@ -653,17 +445,6 @@ __device__ __forceinline__ void store4(_Float16* p, floatx4 v) {
     const half4v h = {_Float16(v[0]), _Float16(v[1]), _Float16(v[2]), _Float16(v[3])};
     *reinterpret_cast<half4v*>(p) = h;
 }
-// (chunked down: fp32 only; the chunks run one after another on the stream)
-__device__ __forceinline__ void add4(float* p, floatx4 v) {
-    float4 o = *reinterpret_cast<float4*>(p);
-    o.x += v[0];
-    o.y += v[1];
-    o.z += v[2];
-    o.w += v[3];
-    *reinterpret_cast<float4*>(p) = o;
-}
-template <typename T>
-__device__ __forceinline__ void add4(T*, floatx4) {}
 __device__ __forceinline__ void store4(__hip_bfloat16* p, floatx4 v) {
     p[0] = __float2bfloat16(v[0]);
     p[1] = __float2bfloat16(v[1]);
@@ -671,149 +452,308 @@ __device__ __forceinline__ void store4(__hip_bfloat16* p, floatx4 v) {
     p[3] = __float2bfloat16(v[3]);
 }
 
-// ff above 1024 runs in chunks of K = 1024 (the tile's activations of one chunk in LDS): chunk k0 .. k0
-// + 256 NQ - 1 of h (rows hstride long) against weight blocks k0 / 64 .. of each row, the chunk's
-// products added to yd (fp32) after the first chunk (accumulate).
-// SMALL: the one-column tiles (16 tokens; the list's n_tiles[1] .. n_tiles[0] - 1) with a quarter of
-// the LDS and at most 168 registers, so 3 workgroups share a CU; otherwise the tiles before them
-// (2-4 columns). Measured on configs[3]: the layer 542 -> 522 us against one kernel for all tiles.
-template <int NQ, bool TAIL, typename OutT, bool SMALL>
-__global__ void __launch_bounds__(256, SMALL ? 3 : 2) k_pf_down(const uint8_t* __restrict__ arena, size_t stride, int E,
-                                                 const uint8_t* __restrict__ shared_blob, int n, int ff,
-                                                 const _Float16* __restrict__ h, const int32_t* __restrict__ bounds,
-                                                 const int2* __restrict__ tiles, const int32_t* __restrict__ n_tiles,
-                                                 OutT* __restrict__ yd, const int32_t* __restrict__ slot_of, int k0,
-                                                 int hstride, int accumulate) {
-    constexpr int ffp = NQ * 256;      // the chunk's h length
-    const int nbk = ff / kBlock;       // weight blocks per row
-    const int b0 = k0 / kBlock;        // the chunk's first weight block
-    const int nbc = min(nbk - b0, ffp / kBlock);   // weight blocks of the chunk
-    constexpr int cpt = ffp / 8;       // 16-byte activation chunks per token
-    constexpr int TN = SMALL ? 16 : kTN;   // tokens per tile
-    constexpr int MC = TN / 16;              // token columns at most
-    constexpr int kDB = TN * cpt / 256;      // activation loads per lane
-    static_assert(TN * cpt % 256 == 0, "whole activation loads per lane");
-    const int ti = SMALL ? n_tiles[1] + int(blockIdx.y) : int(blockIdx.y);
-    if (ti >= n_tiles[SMALL ? 0 : 1]) return;
-    extern __shared__ __align__(16) uint8_t smem[];
-    __shared__ int sRow[TN];
-    const int2 tile = tiles[ti];
+// One workgroup's part of one tile: row slice `slice` of tile `tile`.
+template <bool DOWN, bool SMALL, typename OutT>
+__device__ __forceinline__ void pf_tile(uint8_t* smem, int* sRow, const int2 tile, int slice, const uint8_t* __restrict__ arena,
+                                        size_t stride, int E, const uint8_t* __restrict__ shared_blob, int n, int kp, int hblk,
+                                        int ff, const _Float16* __restrict__ bh, const _Float16* __restrict__ bl,
+                                        const int32_t* __restrict__ row_of, const int32_t* __restrict__ bounds,
+                                        OutT* __restrict__ out) {
+    using Sh = GemmShape<DOWN, SMALL>;
+    constexpr int NP = Sh::parts;
     const int grp = tile.x;
     const int row0 = bounds[grp] + tile.y;
-    const int cnt = min(TN, bounds[grp + 1] - row0);
+    const int cnt = min(Sh::tokens, bounds[grp + 1] - row0);
     const uint8_t* blob = grp < E ? arena + size_t(grp) * stride : shared_blob;
-    const uint8_t* const md = blob + 2 * mat_bytes(ff, n);   // down [n][ff]
-    const size_t scale_off = size_t(n) * nbk * 16;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int li = lane & 15, lg = lane >> 4;
-    if (tid < TN) sRow[tid] = row0 + min(tid, cnt - 1);   // past the group's end: repeat a row
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < kDB; ++p) {
-        const int P = 256 * p + tid, j = P / cpt, kc = (P % cpt) ^ (j & 15);
-        ldsdma16(h + size_t(sRow[j]) * hstride + k0 + kc * 8, smem + P * 16 - lane * 16);
+    const int nbk = (DOWN ? ff : n) / kBlock;   // weight blocks per row (even: n and ff are multiples of 128)
+    const int mrows = DOWN ? n : ff;            // rows of the matrix
+    const size_t mb = mat_bytes(ff, n);
+    const int rbase = slice * Sh::rows;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    // the activation row of each tile token (gate/up: its token's; down: its own); past the group's end
+    // the last repeats (never written)
+    if (tid < Sh::tokens) {
+        const int r = row0 + min(tid, cnt - 1);
+        sRow[tid] = DOWN ? r : row_of[r];
     }
+    __syncthreads();
 
-    uint32_t aoff[4];   // this lane's row in its row block, for tile i
-#pragma unroll
-    for (int i = 0; i < 4; ++i) aoff[i] = uint32_t(64 * wave + 16 * i + li);
-    struct ARegs {
-        uint4 cw[4];
-        uint32_t sc[4];
+    // weight loads of stretch q: lane l takes chunk position l % 4 of rows 16 p + l / 4, p = 0..3 (codes).
+    // Scales come for two stretches at a time (16 bytes a row: block pair l % 4 of row 16 p + l / 4), half
+    // of the rows with each stretch before. Wave rows: gate/up 0..31 gate, 32..63 up; down: 64
+    // consecutive rows (past the matrix's end the last repeats, never written). K runs to kp; a block
+    // past the row's last is read as its last, whose finite products with the zeros are 0.
+    uint8_t* const sA = smem + Sh::ring_b + wave * Sh::wave_a;
+    const uint8_t* const mat = DOWN ? blob + 2 * mb : blob;
+    const uint32_t scale_off = uint32_t(mrows) * nbk * 16;
+    auto row_at = [&](int rl) {   // (matrix offset, row) of wave row rl
+        return DOWN ? min(rbase + 64 * wave + rl, mrows - 1) : rbase + 32 * wave + (rl & 31);
     };
-    const int nsx = ((n + 255) / 256) * NQ;   // stretches in all (a multiple of 4 unless TAIL)
-    // stretch s: row block s / NQ, blocks 4 (s % NQ) + lg; rows past n (a last block of 128 rows)
-    // read row n - 1 and are never stored
-    auto load_a = [&](int s, ARegs& a) {
-        const int rb = s / NQ;
-        const uint32_t blk = b0 + min(4 * (s % NQ) + lg, nbc - 1);
+    uint32_t coff[4], soff[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const size_t o = size_t(min(rb * 256 + int(aoff[i]), n - 1)) * nbk + blk;
-            a.cw[i] = gld_u4(md + o * 16);
-            a.sc[i] = gld<uint16_t>(md + scale_off + o * 2);
+    for (int p = 0; p < 4; ++p) {
+        const uint32_t m = !DOWN && p >= 2 ? uint32_t(mb) : 0u, r = uint32_t(row_at(16 * p + (lane >> 2))) * nbk;
+        coff[p] = m + r * 16;
+        soff[p] = m + scale_off + r * 2;
+    }
+    const int cchunk = (lane & 3) ^ ((lane >> 4) & 3);   // the chunk at this lane's position: c ^ ((row >> 2) & 3)
+    auto issue_scales = [&](int pair, int half) {
+        const uint32_t so = uint32_t(min(4 * pair + (lane & 3), nbk / 2 - 1)) * 4;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) ldsdma4(mat + ((half ? soff[2 + p] : soff[p]) + so), sA + 4096 + half * 512 + p * 256);
+    };
+    auto issue_a = [&](int q) {   // stretch q's codes; half the rows' scales of the pair of stretches after q's
+        const uint32_t bo = uint32_t(min(4 * q + cchunk, nbk - 1)) * 16;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) ldsdma16(mat + (coff[p] + bo), sA + p * 1024);
+        issue_scales((q + 1) >> 1, (q & 1) ^ 1);
+    };
+    // this thread's activation chunks of a stage: LDS positions P = 256 p + tid (token P / cpt)
+    size_t boff[Sh::dma];   // element offsets
+#pragma unroll
+    for (int p = 0; p < Sh::dma; ++p) {
+        const int P = 256 * p + tid, j = P / Sh::cpt, kc = (P % Sh::cpt) ^ Sh::swz(j);
+        boff[p] = size_t(sRow[j]) * kp + kc * 8;
+    }
+    auto issue_b = [&](int st, int slot) {
+        uint8_t* b = smem + slot * NP * Sh::slot_b + wave * 1024;
+#pragma unroll
+        for (int p = 0; p < Sh::dma; ++p) {
+            ldsdma16(bh + boff[p] + size_t(st) * Sh::stage_k, b + p * 4096);
+            if constexpr (NP == 2) ldsdma16(bl + boff[p] + size_t(st) * Sh::stage_k, b + Sh::slot_b + p * 4096);
         }
     };
-    const DqMagic mg = dq_magic();
-
-    size_t yslot[MC];   // yd row of this lane's token column c (loaded before the weight stream)
+    // the MFMA shape: RT row tiles of MR rows, lanes (row or token lr, group lg), PG blocks per lane and stretch
+    constexpr int MR = SMALL ? 16 : 32, RT = 64 / MR, MC = Sh::tokens / MR, PG = SMALL ? 1 : 2;
+    const int lr = lane & (MR - 1), lg = lane / MR;
+    using Acc = std::conditional_t<SMALL, floatx4, floatx16>;
+    Acc acc[RT][MC];
 #pragma unroll
-    for (int c = 0; c < MC; ++c) yslot[c] = size_t(slot_of[row0 + min(c * 16 + li, cnt - 1)]) * n;
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int c = 0; c < MC; ++c)
+#pragma unroll
+            for (int r = 0; r < MR * MR / 64; ++r) acc[i][c][r] = 0.0f;
+    const DqMagic mg = dq_magic();
+    half8 cw[RT][PG];        // (read as the activations are: bits of code dwords)
+    _Float16 sc[RT][PG], sc1[RT][PG];   // scales of this stretch and, in an even one, of the next
+    auto read_a = [&](bool even) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int p = 0; p < PG; ++p) {
+                const int rl = MR * i + lr, c = (SMALL ? 0 : 2 * p) + lg;
+                cw[i][p] = reinterpret_cast<const half8*>(sA)[rl * 4 + (c ^ ((rl >> 2) & 3))];
+                sc[i][p] = sc1[i][p];
+                if (even) {
+                    sc[i][p] = reinterpret_cast<const _Float16*>(sA + 4096)[rl * 8 + c];
+                    sc1[i][p] = reinterpret_cast<const _Float16*>(sA + 4096)[rl * 8 + 4 + c];
+                }
+            }
+    };
+
+    // Stage st (K = stage_k st ..) is part h = st % sps of stretch st / sps. Per stage st, after its
+    // barrier: A stretch st / sps + 1 (first stage of a stretch, h = 0, once the current stretch's
+    // weights are in registers), then B stage st + ahead (the issue pattern of gu_wait). Waiting for B
+    // stage st (vmcnt: the loads issued after it may stay outstanding) covers everything issued before
+    // it, A stretch st / sps included. The pattern is the same for every stage: past the end, the last
+    // stretch / stage is loaded again (into LDS that nothing reads any more), so the wait counts are
+    // constants.
+    const int nst = kp / Sh::stage_k;   // stages
+    const int nq = kp / 256;            // stretches
     auto run = [&](auto nc) {
         constexpr int NC = decltype(nc)::value;
-        ARegs a0, a1, a2, a3;
-        floatx4 acc[4][NC];
-        load_a(0, a0);
-        load_a(min(1, nsx - 1), a1);
-        load_a(min(2, nsx - 1), a2);
-        wait_vm<3 * 8>();   // the activations (issued first) are in LDS for this wave ...
-        __syncthreads();    // ... and for every wave
+        // K-step t of the stage in slot sb (t: its 32-deep chunk group), block pair half p (32x32 only)
+        auto rd = [&](const half8* sb, int t, int p, half8(&b)[NC][NP]) {
+            const int kc = t * 4 + (SMALL ? 0 : 2 * p) + lg;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int c = 0; c < NC; ++c) {
+                const int j = c * MR + lr;
 #pragma unroll
-            for (int c = 0; c < NC; ++c) acc[i][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-        const half8* sb = reinterpret_cast<const half8*>(smem);
-        // stretch s with weights in cur; the stretch three ahead loads into nxt (the last one again
-        // past the end, so every stretch has the same loads in flight)
-        auto step = [&](int s, int q, const ARegs& cur, ARegs& nxt) {
-            load_a(min(s + 3, nsx - 1), nxt);
-            if (TAIL && s >= nsx) return;   // past the end (uniform)
-#pragma unroll
-            for (int tt = 0; tt < 8; ++tt) {
-                half8 bv[4];
-#pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    const int j = c * 16 + li, kc = (q * 8 + tt) * 4 + lg;
-                    bv[c] = sb[j * cpt + (kc ^ (j & 15))];
-                }
-                const int d = tt >> 1;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint4 w = cur.cw[i];
-                    const uint32_t cw = d == 0 ? w.x : d == 1 ? w.y : d == 2 ? w.z : w.w;
-                    const _Float16 sc = __builtin_bit_cast(_Float16, uint16_t(cur.sc[i]));
-                    const half8 av = dequant8((tt & 1) ? cw >> 8 : cw, half2v{sc, sc}, mg);
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) acc[i][c] = mfma_acc(av, bv[c], acc[i][c]);
-                }
-            }
-            if (q == NQ - 1) {   // row block s / NQ done: yd[slot][row], then a fresh block
-                const int rb = s / NQ;
-#pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    if (c * 16 + li < cnt) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int r = rb * 256 + 64 * wave + 16 * i + 4 * lg;
-                            if (r < n) {   // (n % 4 == 0)
-                                if (accumulate) add4(yd + yslot[c] + r, acc[i][c]);
-                                else store4(yd + yslot[c] + r, acc[i][c]);
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[i][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-                }
+                for (int part = 0; part < NP; ++part)
+                    b[c][part] = sb[part * (Sh::slot_b / 16) + j * Sh::cpt + (kc ^ Sh::swz(j))];
             }
         };
-        // the stretch's place in its row block: a constant per unrolled step when NQ divides 4
-        auto qof = [&](int s, int i) { return 4 % NQ == 0 ? i % NQ : s % NQ; };
-        for (int s = 0; s < nsx; s += 4) {
-            step(s, qof(s, 0), a0, a3);
-            step(s + 1, qof(s + 1, 1), a1, a0);
-            step(s + 2, qof(s + 2, 2), a2, a1);
-            step(s + 3, qof(s + 3, 3), a3, a2);
+        // the loads of stages -max(ahead, sps) .. -1 of the steady-state pattern below
+#pragma unroll
+        for (int s = -(Sh::ahead > Sh::sps ? Sh::ahead : Sh::sps); s < 0; ++s) {
+            if (gu_mod(s, Sh::sps) == 0 && s >= -Sh::sps) {
+                issue_scales(0, 0);
+                issue_a(0);   // (with the other half's scales)
+            }
+            if (s >= -Sh::ahead) issue_b(min(s + Sh::ahead, nst - 1), s + Sh::ahead);
+        }
+        int slot = 0, slot_in = Sh::ahead;   // the slots of stages st and st + ahead
+        for (int q = 0; q < nq; ++q) {
+#pragma unroll
+            for (int h = 0; h < Sh::sps; ++h) {
+                const int st = Sh::sps * q + h;
+                // loads issued after B stage st (by stages st - ahead + 1 .. st - 1) may stay outstanding
+                switch (h) {
+                    case 0: wait_vm<gu_wait(0, Sh::ahead, Sh::sps, Sh::kDB, Sh::kDA)>(); break;
+                    case 1: wait_vm<gu_wait(1, Sh::ahead, Sh::sps, Sh::kDB, Sh::kDA)>(); break;
+                    case 2: wait_vm<gu_wait(2, Sh::ahead, Sh::sps, Sh::kDB, Sh::kDA)>(); break;
+                    default: wait_vm<gu_wait(3, Sh::ahead, Sh::sps, Sh::kDB, Sh::kDA)>(); break;
+                }
+                ring_barrier();   // stage st is in LDS for every wave; every wave is done with stage st - 1
+                if (h == 0) {
+                    read_a((q & 1) == 0);
+                    lds_reads_done();   // the wave's weights are in registers: their LDS may be written
+                    issue_a(min(q + 1, nq - 1));
+                }
+                issue_b(min(st + Sh::ahead, nst - 1), slot_in);   // into stage st - 1's slot
+                const half8* sb = reinterpret_cast<const half8*>(smem + slot * NP * Sh::slot_b);
+                slot = slot + 1 == Sh::stages ? 0 : slot + 1;
+                slot_in = slot_in + 1 == Sh::stages ? 0 : slot_in + 1;
+                constexpr int steps = Sh::stage_k / 32 * PG;
+                half8 b[2][NC][NP];
+                rd(sb, 0, 0, b[0]);
+#pragma unroll
+                for (int u = 0; u < steps; ++u) {
+                    const int tt = Sh::stage_k / 32 * h + u / PG, p = u % PG;   // the step's place in the stretch
+                    if (u + 1 < steps) rd(sb, (u + 1) / PG, (u + 1) % PG, b[(u + 1) & 1]);
+#pragma unroll
+                    for (int i = 0; i < RT; ++i) {
+                        const uint32_t x = __builtin_bit_cast(u32x4_t, cw[i][p])[tt >> 1];
+                        const half8 av = dequant8((tt & 1) ? x >> 8 : x, half2v{sc[i][p], sc[i][p]}, mg);
+#pragma unroll
+                        for (int c = 0; c < NC; ++c)
+#pragma unroll
+                            for (int part = 0; part < NP; ++part) acc[i][c] = mfma_acc(av, b[u & 1][c][part], acc[i][c]);
+                    }
+                }
+            }
         }
     };
     if constexpr (SMALL) {
         run(std::integral_constant<int, 1>{});
     } else {
-        switch ((cnt + 15) / 16) {   // token columns with at least one real token (2..4 here)
-            case 2: run(std::integral_constant<int, 2>{}); break;
-            case 3: run(std::integral_constant<int, 3>{}); break;
-            default: run(std::integral_constant<int, 4>{}); break;
+        if (cnt <= 32) run(std::integral_constant<int, 1>{});
+        else run(std::integral_constant<int, 2>{});
+    }
+    wait_vm<0>();      // the ring's last direct-to-LDS loads (repeats past the end) have landed
+    __syncthreads();   // and every wave is past its last LDS read
+
+    // Lane (token lr, group lg) holds MFMA rows 4 lg + 8 a + b (32x32: a, b = 0..3) or 4 lg + b (16x16) of
+    // each row tile, as register 4 a + b.
+    if constexpr (DOWN) {
+        // through LDS, a column of tokens at a time, so that each token's 256 outputs leave in one run
+        constexpr int ld = 256 + 4;
+        float* sy = reinterpret_cast<float*>(smem);
+#pragma unroll
+        for (int c = 0; c < MC; ++c) {
+            if (c * MR >= cnt) break;   // (uniform)
+            if (c) __syncthreads();
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int a = 0; a < MR * MR / 256; ++a)
+                    *reinterpret_cast<floatx4*>(sy + lr * ld + 64 * wave + MR * i + 8 * a + 4 * lg) =
+                        floatx4{acc[i][c][4 * a], acc[i][c][4 * a + 1], acc[i][c][4 * a + 2], acc[i][c][4 * a + 3]};
+            __syncthreads();
+            for (int j = wave; j < min(MR, cnt - c * MR); j += 4) {
+                const int r = rbase + 4 * lane;
+                if (r < n)   // (n % 4 == 0)
+                    store4(out + size_t(row_of[row0 + c * MR + j]) * n + r, *reinterpret_cast<const floatx4*>(sy + j * ld + 4 * lane));
+            }
+        }
+    } else {
+        // ff rows fbase .. fbase + 31 (one Q8_0 block of h) of token column c: gate in the first half of
+        // the row tiles, up in the second
+        const int ffp = (ff + 255) & ~255;   // h row length
+        const int fbase = rbase + 32 * wave;
+        constexpr int HT = RT / 2, NR = MR * MR / 64;   // gate row tiles; values per lane of each
+#pragma unroll
+        for (int c = 0; c < MC; ++c) {
+            const int col = c * MR + lr;
+            float hv[HT][NR];
+            float am = 0.0f;
+#pragma unroll
+            for (int i = 0; i < HT; ++i)
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    hv[i][r] = silu_mul(acc[i][c][r], acc[HT + i][c][r]);
+                    am = fmaxf(am, fabsf(hv[i][r]));
+                }
+            if (SMALL) am = fmaxf(am, __builtin_bit_cast(float, lane_xor16(__builtin_bit_cast(int, am))));
+            am = fmaxf(am, __builtin_bit_cast(float, lane_xor32(__builtin_bit_cast(int, am))));
+            if (hblk == 64) {   // ff rows 64 m .. 64 m + 63 are waves 2m' and 2m' + 1 (rbase is a multiple of 128)
+                float* sam = reinterpret_cast<float*>(smem);
+                if (c) __syncthreads();   // (uniform: hblk is a kernel argument)
+                if (lg == 0) sam[wave * MR + lr] = am;
+                __syncthreads();
+                am = fmaxf(am, sam[(wave ^ 1) * MR + lr]);
+            }
+            const float d = q8_scale(am);
+            const float id = q8_inv(d);
+            const float dr = f16_round(d);
+            if (col < cnt) {
+                // f = fbase + 16 s + 4 e + b: 16x16 s = i, e = lg; 32x32 s = a / 2, e = 2 (a % 2) + lg. In
+                // perm256 order (s, b / 2) are the four consecutive values at the position of (s = 0, e, b % 2).
+                _Float16* dst = out + size_t(row0 + col) * ffp + (fbase & ~255);
+#pragma unroll
+                for (int e = 0; e < (SMALL ? 1 : 2); ++e)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        _Float16 v[4];
+#pragma unroll
+                        for (int s = 0; s < 2; ++s)
+#pragma unroll
+                            for (int u = 0; u < 2; ++u) {
+                                const float x = SMALL ? hv[s % HT][(b + 2 * u) % NR] : hv[0][(4 * (2 * s + e) + b + 2 * u) % NR];
+                                v[2 * s + u] = _Float16(float(q8_code(x, id)) * dr);
+                            }
+                        typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+                        const int f = (fbase & 255) + 4 * (SMALL ? lg : 2 * e + lg) + b;
+                        *reinterpret_cast<half4v*>(dst + perm256_pos(f)) = half4v{v[0], v[1], v[2], v[3]};
+                    }
+            }
+        }
+        // h rows are ffp = ff rounded up to 256 long (whole perm256 stretches for the down GEMM); the
+        // slice holding the last rows also writes zeros at the pad's positions, so that the down GEMM's
+        // products there are 0 (its weights for the pad are any finite values of the row)
+        if (ffp > ff && rbase + Sh::rows >= ff) {
+            const int np = ffp - ff;   // pad elements per row: f = ff .. ffp - 1
+            for (int i = tid; i < cnt * np; i += 256) {
+                const int col = i / np, f = ff + i % np;
+                out[size_t(row0 + col) * ffp + (f & ~255) + perm256_pos(f & 255)] = _Float16(0.0f);
+            }
         }
     }
+}
+
+// DOWN: bh is h [S][kp] (kp = ff rounded up to 256, zeros in the pad), out is yd [slot][n]. Gate/up: bh and
+// bl are the x pairs [T][kp] (kp = n rounded up to 512, zeros past n), out is h.
+// Both tile shapes in one launch, in an order that mixes them: the small tiles stream weights from HBM
+// (each expert's once), the larger ones are bound by the matrix cores, and side by side each fills what
+// the other leaves idle.
+template <bool DOWN, typename OutT>
+__global__ void __launch_bounds__(256, 3)
+k_pf_gemm(const uint8_t* __restrict__ arena, size_t stride, int E, const uint8_t* __restrict__ shared_blob, int n,
+          int kp, int hblk, int ff, const _Float16* __restrict__ bh, const _Float16* __restrict__ bl,
+          const int32_t* __restrict__ row_of, const int32_t* __restrict__ bounds, const int2* __restrict__ tiles,
+          const int32_t* __restrict__ n_tiles, OutT* __restrict__ out) {
+    // A 1-D grid of gx row slices x tiles (tiles rounded up to a multiple of 8). Workgroup L runs on
+    // XCD L % 8, so the slices of a tile are placed 8 apart: they run on the same XCD at about the same
+    // time, and the tile's activations come into that XCD's L2 once.
+    const int gx = DOWN ? (n + 255) / 256 : ff / GemmShape<DOWN, false>::rows;
+    const int L = blockIdx.x, r8 = L >> 3;
+    const int slice = r8 % gx, t = (L & 7) + 8 * (r8 / gx);
+    // n_tiles[0]: tiles in all; n_tiles[1] = B: the first tile of up to 16 tokens (the list is ordered
+    // longest first). The first M places of the order hold the B large tiles evenly spread, the rest
+    // are small, so that the launch ends on short tiles.
+    const int N = n_tiles[0], B = n_tiles[1];
+    if (t >= N) return;
+    const int M = max(1, B + (N - B) * 3 / 4);
+    const int before = t < M ? int(int64_t(t) * B / M) : B, upto = t < M ? int(int64_t(t + 1) * B / M) : B;
+    const bool big = upto > before;
+    const int2 tile = tiles[big ? before : B + t - before];
+    extern __shared__ __align__(16) uint8_t smem[];
+    __shared__ int sRow[kTN];
+    if (big)
+        pf_tile<DOWN, false, OutT>(smem, sRow, tile, slice, arena, stride, E, shared_blob, n, kp, hblk, ff, bh, bl, row_of, bounds, out);
+    else
+        pf_tile<DOWN, true, OutT>(smem, sRow, tile, slice, arena, stride, E, shared_blob, n, kp, hblk, ff, bh, bl, row_of, bounds, out);
 }
 
 // ---------------------------------------------------------------- combine
@@ -921,71 +861,38 @@ int pf_check(int T, int K, int n, int ff, int E) {
     return kOk;
 }
 
-template <bool SMALL>
-static int pf_gemm_attr() {
+template <bool DOWN, typename OutT>
+static int pf_gemm(const char* name, const uint8_t* arena, size_t stride, int E, const uint8_t* shared_blob, int n, int kp,
+                   int ff, int blk, const _Float16* bh, const _Float16* bl, const int32_t* row_of, const PfWs& w, int mt,
+                   OutT* out, hipStream_t stream) {
+    constexpr int big = GemmShape<DOWN, false>::smem, small = GemmShape<DOWN, true>::smem, smem = big > small ? big : small;
+    static_assert(3 * (smem + 4 * kTN) <= 160 * 1024, "three workgroups per CU");
     static bool done = false;   // per process; the attribute is a property of the kernel
     if (!done) {
-        FRT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_gemm<SMALL>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, GuShape<SMALL>::smem));
+        FRT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_gemm<DOWN, OutT>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, smem));
         done = true;
     }
+    const unsigned grid = unsigned(DOWN ? (n + 255) / 256 : ff / GemmShape<DOWN, false>::rows) * unsigned((mt + 7) / 8 * 8);
+    launch_timed(name, k_pf_gemm<DOWN, OutT>, dim3(grid), dim3(256), smem, stream, arena, stride, E, shared_blob, n, kp, blk,
+                 ff, bh, bl, row_of, (const int32_t*)w.bounds, (const int2*)w.tiles, (const int32_t*)w.n_tiles, out);
     return kOk;
 }
 
-template <int NQ, bool TAIL, typename OutT, bool SMALL>
-static int pf_down_attr(size_t lds) {
-    static bool done = false;
-    if (!done) {
-        FRT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_down<NQ, TAIL, OutT, SMALL>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-        done = true;
-    }
-    return kOk;
-}
-
-// The two grouped GEMMs: gate/up (k_pf_gemm) on the exact x pairs, SwiGLU and Q8_0 of h in the
-// epilogue; down (k_pf_down) on h -> yd per slot as OutT.
+// The two grouped GEMMs: gate/up on the exact x pairs, SwiGLU and Q8_0 of h in the epilogue; down on
+// h -> yd per slot as OutT.
 template <typename OutT>
 static int pf_expert_gemms(const uint8_t* arena, size_t stride, int E, const uint8_t* shared_blob, int n, int ff,
                            int blk, const PfWs& w, int mt, OutT* ydf, hipStream_t stream) {
-    if (int rc = pf_gemm_attr<false>()) return rc;
-    if (int rc = pf_gemm_attr<true>()) return rc;
-    // tiles of 2-4 token columns, then those of one (the tile list is ordered longest first)
-    const int mt8 = (mt + 7) / 8 * 8;
-    launch_timed("pf_gateup", k_pf_gemm<false>, dim3(ff / GuShape<false>::ff_rows * mt8), dim3(GuShape<false>::threads),
-                 GuShape<false>::smem, stream, arena, stride, E, shared_blob, n, pf_np(n), blk, ff, (const _Float16*)w.xhi,
-                 (const _Float16*)w.xlo, (const int32_t*)w.tok_of, (const int32_t*)w.bounds, (const int2*)w.tiles,
-                 (const int32_t*)w.n_tiles, w.h16);
-    launch_timed("pf_gateup1", k_pf_gemm<true>, dim3(ff / GuShape<true>::ff_rows * mt8), dim3(GuShape<true>::threads),
-                 GuShape<true>::smem, stream, arena, stride, E, shared_blob, n, pf_np(n), blk, ff, (const _Float16*)w.xhi,
-                 (const _Float16*)w.xlo, (const int32_t*)w.tok_of, (const int32_t*)w.bounds, (const int2*)w.tiles,
-                 (const int32_t*)w.n_tiles, w.h16);
-    timing_mark(stream, "pf_gateup");
     const int ffp = (ff + 255) / 256 * 256;   // h row length
-    // ff up to 1024: one pass over the whole h row; beyond, chunks of 1024 added up in fp32 yd
     if (ffp > 1024 && !std::is_same<OutT, float>::value)
         return set_error(kErrShape, "prefill: ff=%d above 1024 needs fp32 per-slot outputs", ff);
-    for (int k0 = 0; k0 < ffp; k0 += 1024) {
-        const int nq = (ffp - k0 < 1024 ? ffp - k0 : 1024) / 256;   // stretches of this chunk
-        const size_t down_lds = size_t(kTN) * nq * 256 * 2;         // the tile's activations (SMALL: a quarter)
-        const bool tail = ((n + 255) / 256) * nq % 4 != 0;
-        const int acc = k0 > 0 ? 1 : 0;
-#define FRT_PF_DOWN(NQV, TL)                                                                                 \
-    if (nq == NQV && tail == TL) {                                                                           \
-        if (int rc = pf_down_attr<NQV, TL, OutT, false>(down_lds)) return rc;                                \
-        if (int rc = pf_down_attr<NQV, TL, OutT, true>(down_lds / 4)) return rc;                             \
-        launch_timed("pf_down", k_pf_down<NQV, TL, OutT, false>, dim3(1, mt), dim3(256), down_lds, stream, arena, \
-                     stride, E, shared_blob, n, ff, (const _Float16*)w.h16, (const int32_t*)w.bounds,            \
-                     (const int2*)w.tiles, (const int32_t*)w.n_tiles, ydf, (const int32_t*)w.slot_of, k0, ffp, acc); \
-        launch_timed("pf_down1", k_pf_down<NQV, TL, OutT, true>, dim3(1, mt), dim3(256), down_lds / 4, stream, arena, \
-                     stride, E, shared_blob, n, ff, (const _Float16*)w.h16, (const int32_t*)w.bounds,            \
-                     (const int2*)w.tiles, (const int32_t*)w.n_tiles, ydf, (const int32_t*)w.slot_of, k0, ffp, acc); \
-    }
-        FRT_PF_DOWN(1, false) FRT_PF_DOWN(1, true) FRT_PF_DOWN(2, false) FRT_PF_DOWN(2, true)
-        FRT_PF_DOWN(3, false) FRT_PF_DOWN(3, true) FRT_PF_DOWN(4, false) FRT_PF_DOWN(4, true)
-#undef FRT_PF_DOWN
-    }
-    return kOk;
+    if (int rc = pf_gemm<false>("pf_gateup", arena, stride, E, shared_blob, n, pf_np(n), ff, blk,
+                                (const _Float16*)w.xhi, (const _Float16*)w.xlo, (const int32_t*)w.tok_of, w, mt, w.h16, stream))
+        return rc;
+    timing_mark(stream, "pf_gateup");
+    return pf_gemm<true>("pf_down", arena, stride, E, shared_blob, n, ffp, ff, blk, (const _Float16*)w.h16,
+                         (const _Float16*)nullptr, (const int32_t*)w.slot_of, w, mt, ydf, stream);
 }
 
 // The grouped expert products for routed ids (+ optionally the shared expert as group E).

@@ -733,6 +733,30 @@ def test_moe_q2_run_shapes(F, n, ff, T, K, E):
             assert err <= H.OUT_REL, (t, k, err)
 
 
+@pytest.mark.parametrize("n,ff", [(128, 128), (384, 256), (640, 384), (512, 640)])
+def test_moe_q2_run_tile_edges(F, n, ff):
+    """Groups of every size class of the grouped GEMMs' tiles (16 tokens; 17-32 and 33-64 in the 32x32 shape;
+    full tiles with a rest) in one call, each row against the oracle's expert."""
+    sizes = [1, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 80, 81, 128, 0, 2]
+    rng = np.random.default_rng(n + ff)
+    ids = np.repeat(np.arange(len(sizes)), sizes).astype(np.int32)
+    rng.shuffle(ids)
+    T, E = ids.size, len(sizes)
+    eb = F.expert_bytes(n, ff)
+    arena = torch.empty(E * eb, dtype=torch.uint8, device="cuda")
+    F.gen.experts(arena, eb, 7, 0, 0, E, n, ff)
+    x = rng.standard_normal((T, n)).astype(np.float32)
+    nb = F.moe_q2.workspace_bytes(T, 1, n, ff, E)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    yd = torch.full((T, n), float("nan"), dtype=torch.float32, device="cuda")
+    F.moe_q2.run(arena.data_ptr(), eb, E, n, ff, torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda(), T, 1, yd, ws, nb)
+    torch.cuda.synchronize()
+    y, ah = yd.cpu().numpy(), arena.cpu().numpy().reshape(E, eb)
+    for t in range(T):
+        ref = O.expert_ffn(ah[ids[t]], n, ff, x[t])
+        assert H.out_rel(y[t][None], ref) <= H.OUT_REL, (t, ids[t])
+
+
 def test_moe_q2_run_shape_errors(F, w0):
     """The grouped GEMMs' shape limits (n and ff multiples of 128, ff up to 4096) fail loudly."""
     T, K = 4, 2
