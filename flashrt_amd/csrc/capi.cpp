@@ -73,7 +73,8 @@ int router_gemm(const float* x, int T, const float* W, const float* bias, const 
 size_t router_gemm_ws_bytes(int T, int E, bool gate);
 int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16* xhi, _Float16* xlo,
                 hipStream_t stream);
-int quantize_pairs(const float* x, int rows, int n, int np, int blk, _Float16* xhi, _Float16* xlo, hipStream_t stream);
+int quantize_pairs(const float* x, int rows, int n, int np, int blk, _Float16* xhi, _Float16* xlo, int8_t* xq, float* xd,
+                   hipStream_t stream);
 int router_gemm_topk(const float* x, int T, const float* W, const float* bias, const float* gate_w, int E, int n,
                      float* logits, float* gate, float* part, int K, int32_t* ids, float* wts, uint32_t* counts,
                      hipStream_t stream);
@@ -134,10 +135,12 @@ extern int g_dec1_grid_cap;
 // prefill.hip
 size_t pf_workspace_bytes(int T, int K, int n, int ff, int E, bool shared, bool own_yd);
 int pf_run(const uint8_t* experts, size_t stride, int E, int n, int ff, const float* x, const int32_t* ids, int T, int K,
-           void* yd, void* ws, size_t ws_bytes, hipStream_t stream, int block64, int yd_bf16);
+           void* yd, void* ws, size_t ws_bytes, hipStream_t stream, int block64, int yd_bf16, bool pairs_done);
 int pf_moe(const uint8_t* arena, size_t stride, int E, const uint8_t* shared_blob, int n, int ff, const float* x,
            const int32_t* ids, const float* wts, const float* gate, int T, int K, const float* resid, float* out,
-           void* ws, size_t ws_bytes, hipStream_t stream);
+           void* ws, size_t ws_bytes, bool pairs_done, hipStream_t stream);
+int pf_pairs(const float* x, int T, int K, int n, int ff, int E, bool shared, bool own_yd, void* ws, size_t ws_bytes,
+             float* norm_u, int8_t* xq, float* xd, hipStream_t stream);
 int pf_dispatch(const int32_t* ids, int T, int K, int E, int32_t* bounds, int32_t* tok_of, int32_t* slot_of, void* ws,
                 size_t ws_bytes, hipStream_t stream);
 size_t pf_dispatch_ws_bytes(int T, int K, int E);
@@ -283,8 +286,16 @@ static int dense_layer(const frt_moe_layer& L, const LayerWs& lw, const DenseWs&
     if (!small)
         if (int rc = pf_check(T, K, n, ff, E)) return rc;
     const float* u = x;
-    if (L.flags & FRT_LAYER_NORM_INPUT) {
+    const bool norm = (L.flags & FRT_LAYER_NORM_INPUT) != 0;
+    if (!small) {   // the GEMMs' x pairs, and Q8_0 of the input where the shared expert takes it
+        const bool q8 = dense && L.shared_type == FRT_GGML_Q8_0;
+        if (int rc = pf_pairs(x, T, K, n, ff, E, false, false, w.rws, w.rws_bytes, norm ? w.u : nullptr,
+                              q8 ? w.xq : nullptr, q8 ? w.xd : nullptr, s))
+            return rc;
+    } else if (norm) {
         if (int rc = rmsnorm(x, T, n, w.u, s)) return rc;
+    }
+    if (norm) {
         u = w.u;
         timing_mark(s, "rmsnorm");
     }
@@ -300,7 +311,7 @@ static int dense_layer(const frt_moe_layer& L, const LayerWs& lw, const DenseWs&
                                              w.part, K, ids, wts, counts, s)) {
             return rc;
         }
-        if (small || (dense && L.shared_type == FRT_GGML_Q8_0))
+        if (small)
             if (int rc = quantize_q8(u, T, n, w.xq, w.xd, nullptr, nullptr, s)) return rc;
     }
     timing_mark(s, "router");
@@ -317,7 +328,7 @@ static int dense_layer(const frt_moe_layer& L, const LayerWs& lw, const DenseWs&
                                   w.xd + size_t(t0) * (n / kQ8), n, ff, w.rws, w.Y + size_t(t0) * S * n, s, tn))
                 return rc;
         }
-    } else if (int rc = pf_run(L.experts, L.stride, E, n, ff, u, ids, T, K, w.Y, w.rws, w.rws_bytes, s, 0, 0)) {
+    } else if (int rc = pf_run(L.experts, L.stride, E, n, ff, u, ids, T, K, w.Y, w.rws, w.rws_bytes, s, 0, 0, true)) {
         return rc;
     }
     const float* sh = w.Y + size_t(K) * n;   // the Q2_0 shared expert: slot K of each token
@@ -530,7 +541,7 @@ int frt_quantize_q8(void* stream, const float* x, int rows, int n, int8_t* xq, f
 int frt_quantize_pairs(void* stream, const float* x, int rows, int n, int block, uint16_t* xhi, uint16_t* xlo) {
     if (!x || !xhi || !xlo) return set_error(kErrNull, "quantize_pairs: null pointer");
     return quantize_pairs(x, rows, n, (n + 511) & ~511, block, reinterpret_cast<_Float16*>(xhi),
-                          reinterpret_cast<_Float16*>(xlo), static_cast<hipStream_t>(stream));
+                          reinterpret_cast<_Float16*>(xlo), nullptr, nullptr, static_cast<hipStream_t>(stream));
 }
 
 size_t frt_moe_dispatch_workspace_bytes(int T, int K, int E) { return pf_dispatch_ws_bytes(T, K, E); }
@@ -546,7 +557,7 @@ size_t frt_moe_q2_workspace_bytes(int T, int K, int n, int ff, int E) {
 int frt_moe_q2_run(const uint8_t* experts, size_t stride, int E, int n, int ff, const float* x, const int32_t* ids,
                    int T, int K, void* yd, void* ws, size_t ws_bytes, void* stream, int block64, int yd_bf16) {
     return pf_run(experts, stride, E, n, ff, x, ids, T, K, yd, ws, ws_bytes, static_cast<hipStream_t>(stream), block64,
-                  yd_bf16);
+                  yd_bf16, false);
 }
 
 size_t frt_moe_hits_scratch_bytes(int K, int ff, int T) { return hits_bytes(K, ff, T, kHitsMaxN); }
@@ -631,7 +642,8 @@ int frt_moe_layer_forward(const frt_moe_layer* L, const float* x, int T, const f
     if (int rc = pf_check(T, K, n, ff, E)) return rc;
     const float* xin = x;
     if (norm) {
-        if (int rc = rmsnorm(x, T, n, w.u, s)) return rc;
+        // u and the GEMMs' pairs of it in one launch
+        if (int rc = pf_pairs(x, T, K, n, ff, E, true, true, w.rest, w.rest_bytes, w.u, nullptr, nullptr, s)) return rc;
         xin = w.u;
         timing_mark(s, "rmsnorm");
     }
@@ -642,7 +654,7 @@ int frt_moe_layer_forward(const frt_moe_layer* L, const float* x, int T, const f
         return rc;
     timing_mark(s, "route_topk");
     return pf_moe(L->experts, L->stride, E, L->shared, n, ff, xin, ids_o, wts_o, w.gate, T, K, resid, out, w.rest,
-                  w.rest_bytes, s);
+                  w.rest_bytes, norm != 0, s);
 }
 
 size_t frt_noalloc_scratch_bytes(void) { return kNoAllocScratchBytes; }

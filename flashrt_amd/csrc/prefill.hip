@@ -242,6 +242,108 @@ __global__ void __launch_bounds__(64) k_pf_place(const int32_t* __restrict__ ids
     }
 }
 
+// The whole dispatch of a short chunk in one workgroup: up to 256 slots per wave (kSmallSlots in all), E <=
+// 1024 (a thread per expert). Wave w ranks its slots in order by ballots against its own histogram
+// (hist [16][E]), the histograms are summed over the waves per expert, one scan gives the groups' first
+// rows and the tiles, and each slot goes to its place: the same bounds, tiles and rows as the four
+// kernels above. What bounds either is launches and latency: 21 -> 9 us for 370 slots. (Longer chunks keep
+// the four kernels: one workgroup would walk them serially, 36 against 24 us at 20480 slots.)
+constexpr int kSmallSlots = 4096;
+__global__ void __launch_bounds__(1024) k_pf_dispatch1(const int32_t* __restrict__ ids, int S, int K, int E, int id_bits, int T,
+                                                       int shared, int32_t* __restrict__ bounds, int2* __restrict__ tiles,
+                                                       int32_t* __restrict__ n_tiles, int32_t* __restrict__ tok_of,
+                                                       int32_t* __restrict__ slot_of) {
+    extern __shared__ int32_t hist[];
+    __shared__ int s_row[1024];
+    __shared__ int ws[17 * 5];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    int32_t* const h = hist + wave * E;
+    for (int e = lane; e < E; e += 64) h[e] = 0;
+    const int nb = (S + 1023) / 1024;   // batches of 64 slots per wave (1..4)
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    int ex[4], pos[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const int s = (wave * nb + b) * 64 + lane;
+        ex[b] = b < nb && s < S ? ids[s] : -1;
+        if (unsigned(ex[b]) >= unsigned(E)) ex[b] = -1;   // ids outside [0, E) are dropped
+    }
+    asm volatile("" ::: "memory");   // (a wave's LDS operations complete in order)
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        pos[b] = 0;
+        if (b >= nb) break;
+        const bool valid = ex[b] >= 0;
+        const int e = valid ? ex[b] : 0;
+        uint64_t peers = __ballot(valid);
+        for (int bit = 0; bit < id_bits; ++bit) {
+            const bool on = (e >> bit) & 1;
+            const uint64_t m = __ballot(on);
+            peers &= on ? m : ~m;
+        }
+        const int rank = __popcll(peers & lt);
+        const int seen = h[e];
+        pos[b] = seen + rank;
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        if (valid && rank == 0) h[e] = seen + __popcll(peers);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    int rows = 0;
+    if (tid < E)
+        for (int w = 0; w < 16; ++w) {
+            const int c = hist[w * E + tid];
+            hist[w * E + tid] = rows;
+            rows += c;
+        }
+    // tiles per class (as pf_scan_body counts them) and rows, scanned together
+    const int full = rows / kTN, rest = rows % kTN, kr = rest ? tile_class(rest) : 0;
+    const int v[5] = {rows, int(kr == 1), int(kr == 2), int(kr == 3), full + int(kr == 4)};
+    int r[5], tot[5];
+    block_excl_scan_v<5>(v, r, tot, ws);
+    const int sfull = shared ? T / kTN : 0, srest = shared ? T % kTN : 0, sk = srest ? tile_class(srest) : 0;
+    int base[5];   // first tile of each class; the shared group's tiles close each class
+    base[4] = 0;
+    base[3] = tot[4] + sfull + int(sk == 4);
+    base[2] = base[3] + tot[3] + int(sk == 3);
+    base[1] = base[2] + tot[2] + int(sk == 2);
+    if (tid < E) {
+        bounds[tid] = r[0];
+        s_row[tid] = r[0];
+        for (int i = 0; i < full; ++i) tiles[r[4] + i] = make_int2(tid, i * kTN);
+        if (kr) {
+            const int at = kr == 4 ? r[4] + full : (kr == 3 ? base[3] + r[3] : kr == 2 ? base[2] + r[2] : base[1] + r[1]);
+            tiles[at] = make_int2(tid, full * kTN);
+        }
+    }
+    if (tid == 0) {
+        bounds[E] = tot[0];
+        if (shared) {
+            bounds[E + 1] = tot[0] + T;
+            for (int i = 0; i < sfull; ++i) tiles[tot[4] + i] = make_int2(E, i * kTN);
+            if (sk) tiles[sk == 4 ? tot[4] + sfull : base[sk] + tot[sk]] = make_int2(E, sfull * kTN);
+        }
+        n_tiles[0] = base[1] + tot[1] + int(sk == 1);
+        n_tiles[1] = base[1];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+        if (b < nb && ex[b] >= 0) {
+            const int s = (wave * nb + b) * 64 + lane, row = s_row[ex[b]] + h[ex[b]] + pos[b];
+            tok_of[row] = s / K;
+            slot_of[row] = s;
+        }
+    if (shared)
+        for (int t = tid; t < T; t += 1024) {   // rows S + t (S = T K: every slot holds a valid id)
+            tok_of[S + t] = t;
+            slot_of[S + t] = S + t;
+        }
+}
+
 // ---------------------------------------------------------------- grouped GEMMs (gate + up, down)
 //
 // Operands enter the MFMA exactly, so the products are exact and only the fp32 accumulation rounds:
@@ -850,7 +952,10 @@ size_t pf_workspace_bytes(int T, int K, int n, int ff, int E, bool shared, bool 
     return pf_carve(nullptr, T, K, n, ff, E, shared, own_yd).bytes + 256;
 }
 
-int quantize_pairs(const float* x, int rows, int n, int np, int blk, _Float16* xhi, _Float16* xlo, hipStream_t stream);
+int quantize_pairs(const float* x, int rows, int n, int np, int blk, _Float16* xhi, _Float16* xlo, int8_t* xq, float* xd,
+                   hipStream_t stream);
+int norm_pairs(const float* x, int rows, int n, int np, float* u, _Float16* xhi, _Float16* xlo, int8_t* xq, float* xd,
+               hipStream_t stream);
 
 int pf_check(int T, int K, int n, int ff, int E) {
     if (T < 1 || K < 1 || K > 32 || E < 1 || E > 4096 || K > E) return set_error(kErrShape, "prefill: T=%d K=%d E=%d", T, K, E);
@@ -895,26 +1000,44 @@ static int pf_expert_gemms(const uint8_t* arena, size_t stride, int E, const uin
                          (const _Float16*)nullptr, (const int32_t*)w.slot_of, w, mt, ydf, stream);
 }
 
+// The dispatch of S = T K slots (and the shared group's T rows): bounds, tiles, tok_of and slot_of.
+static int pf_dispatch_run(const int32_t* ids, int T, int K, int E, bool shared, int32_t* cnt, int32_t* bounds, int2* tiles,
+                           int32_t* n_tiles, int32_t* tok_of, int32_t* slot_of, hipStream_t stream) {
+    int id_bits = 1;
+    while ((1 << id_bits) < E) ++id_bits;
+    const int S = T * K, nchunk = (S + kChunk - 1) / kChunk;
+    if (S <= kSmallSlots && E <= 1024) {
+        const size_t lds = size_t(16) * E * 4;
+        static bool done = false;   // per process; the attribute is a property of the kernel
+        if (!done) {
+            FRT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_dispatch1),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 16 * 1024 * 4));
+            done = true;
+        }
+        launch_timed("pf_dispatch1", k_pf_dispatch1, dim3(1), dim3(1024), lds, stream, ids, S, K, E, id_bits, T, shared ? 1 : 0,
+                     bounds, tiles, n_tiles, tok_of, slot_of);
+        return kOk;
+    }
+    launch_timed("pf_hist", k_pf_hist, dim3(nchunk), dim3(256), size_t(E) * 4, stream, ids, S, E, cnt);
+    launch_timed("pf_colscan", k_pf_colscan, dim3((E + 3) / 4), dim3(256), 0, stream, cnt, nchunk, E, bounds);
+    launch_timed("pf_scan", k_pf_scan, dim3(1), dim3(1024), 0, stream, E, T, shared ? 1 : 0, bounds, tiles, n_tiles);
+    launch_timed("pf_place", k_pf_place, dim3(nchunk + (shared ? (T + 63) / 64 : 0)), dim3(64), size_t(E) * 4, stream, ids, S,
+                 K, E, id_bits, (const int32_t*)cnt, (const int32_t*)bounds, tok_of, slot_of, shared ? T : 0);
+    return kOk;
+}
+
 // The grouped expert products for routed ids (+ optionally the shared expert as group E).
 // yd_kind: 0 float, 1 bf16 (moe_q2::run's yd_bf16), 2 fp16 (a whole layer's, combined here)
 static int pf_experts(const uint8_t* arena, size_t stride, int E, const uint8_t* shared_blob, int n, int ff,
                       const float* x, const int32_t* ids, int T, int K, void* yd, int yd_kind, int blk, const PfWs& w,
-                      hipStream_t stream) {
+                      bool pairs_done, hipStream_t stream) {
     const bool shared = shared_blob != nullptr;
     const int S = T * K + (shared ? T : 0);
     const int G = E + (shared ? 1 : 0);
-    const int nchunk = (T * K + kChunk - 1) / kChunk;
-    int id_bits = 1;
-    while ((1 << id_bits) < E) ++id_bits;
-    if (int rc = quantize_pairs(x, T, n, pf_np(n), blk, w.xhi, w.xlo, stream)) return rc;
+    if (!pairs_done)
+        if (int rc = quantize_pairs(x, T, n, pf_np(n), blk, w.xhi, w.xlo, nullptr, nullptr, stream)) return rc;
     timing_mark(stream, "pf_quant_x");
-    launch_timed("pf_hist", k_pf_hist, dim3(nchunk), dim3(256), size_t(E) * 4, stream, ids, T * K, E, w.cnt);
-    launch_timed("pf_colscan", k_pf_colscan, dim3((E + 3) / 4), dim3(256), 0, stream, w.cnt, nchunk, E, w.bounds);
-    launch_timed("pf_scan", k_pf_scan, dim3(1), dim3(1024), 0, stream, E, T, shared ? 1 : 0, w.bounds, w.tiles,
-                 w.n_tiles);
-    launch_timed("pf_place", k_pf_place, dim3(nchunk + (shared ? (T + 63) / 64 : 0)), dim3(64), size_t(E) * 4, stream,
-                 ids, T * K, K, E, id_bits, (const int32_t*)w.cnt, (const int32_t*)w.bounds, w.tok_of, w.slot_of,
-                 shared ? T : 0);
+    if (int rc = pf_dispatch_run(ids, T, K, E, shared, w.cnt, w.bounds, w.tiles, w.n_tiles, w.tok_of, w.slot_of, stream)) return rc;
     timing_mark(stream, "pf_dispatch");
     const int mt = pf_max_tiles(S, G);
     int rc = kOk;
@@ -927,33 +1050,46 @@ static int pf_experts(const uint8_t* arena, size_t stride, int E, const uint8_t*
     return kOk;
 }
 
+// The GEMMs' x pairs ahead of a pf_run (shared, own_yd false) or pf_moe (true) call on the same workspace
+// (its pairs_done): with norm_u, of x * rms scale, which also goes to norm_u. xq, xd (or null): the Q8_0
+// codes and scales of the same values.
+int pf_pairs(const float* x, int T, int K, int n, int ff, int E, bool shared, bool own_yd, void* ws, size_t ws_bytes,
+             float* norm_u, int8_t* xq, float* xd, hipStream_t stream) {
+    if (int rc = pf_check(T, K, n, ff, E)) return rc;
+    const PfWs w = pf_carve(ws, T, K, n, ff, E, shared, own_yd);
+    if (w.bytes > ws_bytes) return set_error(kErrWorkspace, "prefill: workspace %zu < %zu", ws_bytes, w.bytes);
+    if (norm_u) return norm_pairs(x, T, n, pf_np(n), norm_u, w.xhi, w.xlo, xq, xd, stream);
+    return quantize_pairs(x, T, n, pf_np(n), 32, w.xhi, w.xlo, xq, xd, stream);
+}
+
 // moe_q2::run (kernels/cuda/moe_q2.h:20-30): yd [T*K][n] per slot
 int pf_run(const uint8_t* experts, size_t stride, int E, int n, int ff, const float* x, const int32_t* ids, int T, int K,
-           void* yd, void* ws, size_t ws_bytes, hipStream_t stream, int block64, int yd_bf16) {
+           void* yd, void* ws, size_t ws_bytes, hipStream_t stream, int block64, int yd_bf16, bool pairs_done) {
     if (int rc = pf_check(T, K, n, ff, E)) return rc;
     if (!experts || !x || !ids || !yd || !ws) return set_error(kErrNull, "moe_q2::run: null pointer");
     const PfWs w = pf_carve(ws, T, K, n, ff, E, false, false);
     if (w.bytes > ws_bytes) return set_error(kErrWorkspace, "moe_q2::run: workspace %zu < %zu", ws_bytes, w.bytes);
     // block64: x and h quantized in Q8_0 blocks of 64 values rather than 32 (moe_q2.cu's AB = 64)
-    return pf_experts(experts, stride, E, nullptr, n, ff, x, ids, T, K, yd, yd_bf16 ? 1 : 0, block64 ? 64 : 32, w, stream);
+    return pf_experts(experts, stride, E, nullptr, n, ff, x, ids, T, K, yd, yd_bf16 ? 1 : 0, block64 ? 64 : 32, w, pairs_done,
+                      stream);
 }
 
 // The whole prefill layer after routing: ids/wts [T][K], gate [T] -> out [T][n] (+ resid)
 int pf_moe(const uint8_t* arena, size_t stride, int E, const uint8_t* shared_blob, int n, int ff, const float* x,
            const int32_t* ids, const float* wts, const float* gate, int T, int K, const float* resid, float* out,
-           void* ws, size_t ws_bytes, hipStream_t stream) {
+           void* ws, size_t ws_bytes, bool pairs_done, hipStream_t stream) {
     if (int rc = pf_check(T, K, n, ff, E)) return rc;
     const PfWs w = pf_carve(ws, T, K, n, ff, E, true, true);
     if (w.bytes > ws_bytes) return set_error(kErrWorkspace, "prefill: workspace %zu < %zu", ws_bytes, w.bytes);
     if (ff > 1024) {   // fp32 per-slot outputs
-        if (int rc = pf_experts(arena, stride, E, shared_blob, n, ff, x, ids, T, K, w.yd, 0, 32, w, stream)) return rc;
+        if (int rc = pf_experts(arena, stride, E, shared_blob, n, ff, x, ids, T, K, w.yd, 0, 32, w, pairs_done, stream)) return rc;
         launch_timed("pf_combine", k_pf_combine<float>, dim3((n + 1023) / 1024, T), dim3(256), 0, stream,
                      (const float*)w.yd, ids, wts, gate, T, K, n, 1, resid, out);
         timing_mark(stream, "pf_combine");
         FRT_LAUNCHED("prefill combine");
         return kOk;
     }
-    if (int rc = pf_experts(arena, stride, E, shared_blob, n, ff, x, ids, T, K, w.yd, 2, 32, w, stream)) return rc;
+    if (int rc = pf_experts(arena, stride, E, shared_blob, n, ff, x, ids, T, K, w.yd, 2, 32, w, pairs_done, stream)) return rc;
     launch_timed("pf_combine", k_pf_combine<_Float16>, dim3((n + 1023) / 1024, T), dim3(256), 0, stream,
                  (const _Float16*)w.yd, ids, wts, gate, T, K, n, 1, resid, out);
     timing_mark(stream, "pf_combine");
@@ -974,12 +1110,7 @@ int pf_dispatch(const int32_t* ids, int T, int K, int E, int32_t* bounds, int32_
     int2* tiles = reinterpret_cast<int2*>(p);
     p += up256(size_t(pf_max_tiles(T * K, E)) * 8);
     int32_t* n_tiles = reinterpret_cast<int32_t*>(p);
-    int id_bits = 1;
-    while ((1 << id_bits) < E) ++id_bits;
-    k_pf_hist<<<nchunk, 256, size_t(E) * 4, stream>>>(ids, T * K, E, cnt);
-    k_pf_colscan<<<(E + 3) / 4, 256, 0, stream>>>(cnt, nchunk, E, bounds);
-    k_pf_scan<<<1, 1024, 0, stream>>>(E, T, 0, bounds, tiles, n_tiles);
-    k_pf_place<<<nchunk, 64, size_t(E) * 4, stream>>>(ids, T * K, K, E, id_bits, cnt, bounds, tok_of, slot_of, 0);
+    if (int rc = pf_dispatch_run(ids, T, K, E, false, cnt, bounds, tiles, n_tiles, tok_of, slot_of, stream)) return rc;
     FRT_LAUNCHED("dispatch");
     return kOk;
 }

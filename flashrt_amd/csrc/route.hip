@@ -183,16 +183,17 @@ __global__ void k_quant_q8(const float* __restrict__ x, int n_blocks, int8_t* __
 // pairs go through LDS so that each lane then writes 4 consecutive positions (8 bytes) of each.
 // Same values as k_quant_q8 with xhi / xlo.
 // x [rows][n] -> the pairs [rows][np] (np >= n a multiple of 256; positions n .. np - 1 are zeros),
-// Q8_0 blocks of blk = 32 or 64 values (moe_q2::run's block64).
-__global__ void __launch_bounds__(256) k_quant_pairs(const float* __restrict__ x, int n, int np, int n_stretch, int blk,
-                                                     _Float16* __restrict__ xhi, _Float16* __restrict__ xlo) {
-    __shared__ _Float16 sp[4][2][256];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int st = blockIdx.x * 4 + wave;
-    if (st >= n_stretch) return;   // whole waves; no workgroup barrier below
-    const int spr = np / 256, row = st / spr, col = (st % spr) * 256 + lane * 4;   // n % 4 == 0
-    const float4 v4 = col < n ? *reinterpret_cast<const float4*>(x + size_t(row) * n + col) : make_float4(0, 0, 0, 0);
-    const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+// Q8_0 blocks of blk = 32 or 64 values (moe_q2::run's block64). xq / xd (or null; blk 32): the same
+// codes int8 [rows][n] and scales [rows][n / 32].
+struct PairsOut {
+    _Float16 *xhi, *xlo;
+    int8_t* xq;
+    float* xd;
+};
+// one wave's stretch: elements 256 col ..  of row `row`, v this lane's four
+__device__ __forceinline__ void quant_stretch(const float (&v)[4], int row, int col, int n, int np, int blk, _Float16 (&sp)[2][256],
+                                              const PairsOut& o) {
+    const int lane = threadIdx.x & 63;
     float am = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
     am = fmaxf(am, __shfl_xor(am, 1));
     am = fmaxf(am, __shfl_xor(am, 2));
@@ -202,20 +203,75 @@ __global__ void __launch_bounds__(256) k_quant_pairs(const float* __restrict__ x
     const float d = q8_scale(am);
     const float id = q8_inv(d);
     const float dr = f16_round(d);
+    uint32_t codes = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float a = float(q8_code(v[i], id)) * dr;
+        const int q = q8_code(v[i], id);
+        codes |= uint32_t(uint8_t(int8_t(q))) << (8 * i);
+        const float a = float(q) * dr;
         const _Float16 hi = _Float16(a);
         const int p = perm256_pos(lane * 4 + i);
-        sp[wave][0][p] = hi;
-        sp[wave][1][p] = _Float16(a - float(hi));
+        sp[0][p] = hi;
+        sp[1][p] = _Float16(a - float(hi));
     }
+    const int e = 256 * col + 4 * lane;
+    if (o.xq && e < n) {
+        *reinterpret_cast<uint32_t*>(o.xq + size_t(row) * n + e) = codes;
+        if (lane % 8 == 0) o.xd[size_t(row) * (n / kQ8) + e / kQ8] = dr;
+    }
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0xC07F);   // this wave's LDS writes are done (lgkmcnt(0))
     __builtin_amdgcn_wave_barrier();
-    const uint2 h = *reinterpret_cast<const uint2*>(&sp[wave][0][lane * 4]);
-    const uint2 l = *reinterpret_cast<const uint2*>(&sp[wave][1][lane * 4]);
-    *reinterpret_cast<uint2*>(xhi + size_t(st) * 256 + lane * 4) = h;
-    *reinterpret_cast<uint2*>(xlo + size_t(st) * 256 + lane * 4) = l;
+    const uint2 h = *reinterpret_cast<const uint2*>(&sp[0][lane * 4]);
+    const uint2 l = *reinterpret_cast<const uint2*>(&sp[1][lane * 4]);
+    const size_t at = size_t(row) * np + e;
+    *reinterpret_cast<uint2*>(o.xhi + at) = h;
+    *reinterpret_cast<uint2*>(o.xlo + at) = l;
+    asm volatile("" ::: "memory");   // (the next stretch's LDS writes stay after these reads)
+}
+__global__ void __launch_bounds__(256) k_quant_pairs(const float* __restrict__ x, int n, int np, int n_stretch, int blk, PairsOut o) {
+    __shared__ _Float16 sp[4][2][256];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int st = blockIdx.x * 4 + wave;
+    if (st >= n_stretch) return;   // whole waves; no workgroup barrier below
+    const int spr = np / 256, row = st / spr, c = st % spr, col = c * 256 + lane * 4;   // n % 4 == 0
+    const float4 v4 = col < n ? *reinterpret_cast<const float4*>(x + size_t(row) * n + col) : make_float4(0, 0, 0, 0);
+    const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+    quant_stretch(v, row, c, n, np, blk, sp[wave], o);
+}
+// The same of u = x * r (the canonical RMS scale, as k_rmsnorm), which is also written: a workgroup per
+// token, every wave forming the scale itself (the token's row comes from L1 after the first), then the
+// stretches wave, wave + 4, .. One launch for k_rmsnorm and k_quant_pairs: what bounds them at a few
+// hundred tokens is the launches (4.8 + 4.6 us at 37 tokens).
+template <int L>
+__global__ void __launch_bounds__(256) k_norm_pairs(const float* __restrict__ x, int np, float* __restrict__ u, PairsOut o) {
+    __shared__ _Float16 sp[4][2][256];
+    constexpr int n = 64 * L;
+    const int row = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const float* xr = x + size_t(row) * n;
+    float xc[L];
+#pragma unroll
+    for (int i = 0; i < L / 4; ++i) {
+        const float4 q = *reinterpret_cast<const float4*>(xr + lane * L + 4 * i);
+        xc[4 * i] = q.x;
+        xc[4 * i + 1] = q.y;
+        xc[4 * i + 2] = q.z;
+        xc[4 * i + 3] = q.w;
+    }
+    const float r = rms_scale_wave<L>(xc, n);
+    for (int c = wave; c < np / 256; c += 4) {   // (n is a multiple of 256: whole stretches)
+        const int col = c * 256 + lane * 4;
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (col < n) {
+            const float4 v4 = *reinterpret_cast<const float4*>(xr + col);
+            v[0] = v4.x * r;
+            v[1] = v4.y * r;
+            v[2] = v4.z * r;
+            v[3] = v4.w * r;
+            *reinterpret_cast<float4*>(u + size_t(row) * n + col) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+        quant_stretch(v, row, c, n, np, 32, sp[wave], o);
+    }
 }
 // (a zero block quantizes to codes 0 with d = 0: the pad reads as exact zeros)
 
@@ -328,12 +384,30 @@ int rmsnorm(const float* x, int T, int n, float* u, hipStream_t stream) {
 
 // The prefill GEMM's activation pairs alone: rows of np (a multiple of 256, >= n) in perm256 order,
 // Q8_0 blocks of blk (32 or 64) values.
-int quantize_pairs(const float* x, int rows, int n, int np, int blk, _Float16* xhi, _Float16* xlo, hipStream_t stream) {
-    if (rows < 1 || n % 128 || np % 256 || np < n || (blk != 32 && blk != 64))
+int quantize_pairs(const float* x, int rows, int n, int np, int blk, _Float16* xhi, _Float16* xlo, int8_t* xq, float* xd,
+                   hipStream_t stream) {
+    if (rows < 1 || n % 128 || np % 256 || np < n || (blk != 32 && blk != 64) || (xq && blk != 32))
         return set_error(kErrShape, "quantize_pairs: n=%d np=%d blk=%d", n, np, blk);
     const int ns = rows * (np / 256);
-    launch_timed("pf_quant_x", k_quant_pairs, dim3((ns + 3) / 4), dim3(256), 0, stream, x, n, np, ns, blk, xhi, xlo);
+    launch_timed("pf_quant_x", k_quant_pairs, dim3((ns + 3) / 4), dim3(256), 0, stream, x, n, np, ns, blk,
+                 PairsOut{xhi, xlo, xq, xd});
     FRT_LAUNCHED("quantize_pairs");
+    return kOk;
+}
+
+// rmsnorm (u) and quantize_pairs of u in one launch
+int norm_pairs(const float* x, int rows, int n, int np, float* u, _Float16* xhi, _Float16* xlo, int8_t* xq, float* xd,
+               hipStream_t stream) {
+    if (rows < 1 || np % 256 || np < n) return set_error(kErrShape, "norm_pairs: n=%d np=%d", n, np);
+    const PairsOut o{xhi, xlo, xq, xd};
+#define FRT_NP(LL) \
+    case LL: launch_timed("norm_pairs", k_norm_pairs<LL>, dim3(rows), dim3(256), 0, stream, x, np, u, o); break;
+    switch (n % 64 ? 0 : n / 64) {
+        FRT_NP(8) FRT_NP(16) FRT_NP(24) FRT_NP(32) FRT_NP(40) FRT_NP(48) FRT_NP(56) FRT_NP(64)
+        default: return set_error(kErrShape, "rmsnorm: n=%d", n);
+    }
+#undef FRT_NP
+    FRT_LAUNCHED("norm_pairs");
     return kOk;
 }
 
@@ -341,7 +415,7 @@ int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16
                 hipStream_t stream) {
     if (rows < 1 || n % 64) return set_error(kErrShape, "quantize_q8: n=%d not a multiple of 64", n);
     const int nb = rows * (n / kQ8);
-    if (xhi && xlo && !xq && !xd && n % 256 == 0) return quantize_pairs(x, rows, n, n, 32, xhi, xlo, stream);
+    if (xhi && xlo && !xq && !xd && n % 256 == 0) return quantize_pairs(x, rows, n, n, 32, xhi, xlo, nullptr, nullptr, stream);
     const int waves = (nb + 1) / 2;
     launch_timed("pf_quant_x", k_quant_q8, dim3((waves + 3) / 4), dim3(256), 0, stream, x, nb, xq, xd, xhi, xlo, n);
     FRT_LAUNCHED("quantize_q8");
@@ -609,34 +683,50 @@ __global__ void __launch_bounds__(256) k_router_combine(const float* __restrict_
 
 // k_router_combine and k_route_topk in one pass (E <= 512): wave w of a workgroup takes token
 // 4 blockIdx.x + w, sums its logits from the split's partials in k_router_combine's tree (writing the
-// logits and the gate as it does) into LDS, and selects from there with the same topk_wave.
+// logits and the gate as it does) into LDS, and selects from there by ballots (topk_wave_fast). Bound by
+// latency: with one logit's partials in flight and the bitonic selection 11.5 us at 37 tokens.
 __global__ void __launch_bounds__(256) k_route_topk_part(const float* __restrict__ part, int T, int E, int E1,
                                                          const float* __restrict__ bias, float* __restrict__ logits,
                                                          float* __restrict__ gate, int K, int32_t* __restrict__ ids,
                                                          float* __restrict__ wts, uint32_t* counts) {
     __shared__ __align__(16) float row[4][512];
-    __shared__ float cand_v[4][64];
-    __shared__ int cand_id[4][64];
+    __shared__ float cand_v[4][128];
+    __shared__ int cand_id[4][128];
     const int wave = threadIdx.x >> 6;
     const int t = blockIdx.x * 4 + wave, lane = threadIdx.x & 63;
     if (t >= T) return;   // (whole waves; no workgroup barrier below)
     const size_t N = size_t(T) * E1;
-    for (int e = lane; e < E1; e += 64) {
-        const size_t i = size_t(t) * E1 + e;
-        const float v = ((part[i] + part[N + i]) + (part[2 * N + i] + part[3 * N + i])) +
-                        ((part[4 * N + i] + part[5 * N + i]) + (part[6 * N + i] + part[7 * N + i]));
-        if (e < E) {
-            const float l = bias ? v + bias[e] : v;
-            logits[size_t(t) * E + e] = l;
-            row[wave][e] = l;
-        } else {
-            gate[t] = v;
+    const float* pt = part + size_t(t) * E1;
+    // four logits' partials (32 loads) in flight per lane; the gate's (column E) with the first
+    const bool has_gate = E1 > E && lane == 0;
+    float pg[8];
+#pragma unroll
+    for (int z = 0; z < 8; ++z) pg[z] = pt[z * N + (E1 - 1)];
+    for (int e0 = lane; e0 < E; e0 += 256) {
+        float p[4][8], b[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int e = min(e0 + 64 * q, E - 1);
+#pragma unroll
+            for (int z = 0; z < 8; ++z) p[q][z] = pt[z * N + e];
+            b[q] = bias ? bias[e] : 0.0f;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int e = e0 + 64 * q;
+            const float v = ((p[q][0] + p[q][1]) + (p[q][2] + p[q][3])) + ((p[q][4] + p[q][5]) + (p[q][6] + p[q][7]));
+            if (e < E) {
+                const float l = bias ? v + b[q] : v;
+                logits[size_t(t) * E + e] = l;
+                row[wave][e] = l;
+            }
         }
     }
+    if (has_gate) gate[t] = ((pg[0] + pg[1]) + (pg[2] + pg[3])) + ((pg[4] + pg[5]) + (pg[6] + pg[7]));
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int id = topk_wave<8>(row[wave], E, K, ids + size_t(t) * K, wts + size_t(t) * K, cand_v[wave], cand_id[wave]);
+    const int id = topk_wave_fast<8>(row[wave], E, K, ids + size_t(t) * K, wts + size_t(t) * K, cand_v[wave], cand_id[wave]);
     if (lane < K && counts) atomicAdd(counts + id, 1u);
 }
 

@@ -243,6 +243,24 @@ def test_dispatch_bit_exact(F, T, skew):
     assert np.array_equal(rs, np.argsort(ids.reshape(-1), kind="stable"))
 
 
+@pytest.mark.parametrize("T,E,K", [(1, 1, 1), (9, 3, 2), (37, 512, 10), (100, 1000, 32), (409, 1024, 10), (410, 512, 10),
+                                   (4096, 7, 1), (4097, 7, 1)])
+def test_dispatch_short_chunk(F, T, E, K):
+    """Either side of the one-workgroup dispatch's limits (4096 slots, 1024 experts; batches of 64 slots per
+    wave, empty waves): bounds, slots and tokens exactly those of the stable sort."""
+    rng = np.random.default_rng(T + E)
+    ids = np.stack([rng.permutation(E)[:K] for _ in range(T)]).astype(np.int32)
+    b = torch.empty(E + 1, dtype=torch.int32, device="cuda")
+    to = torch.empty(T * K, dtype=torch.int32, device="cuda")
+    so = torch.empty(T * K, dtype=torch.int32, device="cuda")
+    F.moe_dispatch(dev(ids), T, K, E, b, to, so)
+    torch.cuda.synchronize()
+    order = np.argsort(ids.reshape(-1), kind="stable")
+    assert np.array_equal(b.cpu().numpy(), np.concatenate([[0], np.cumsum(np.bincount(ids.reshape(-1), minlength=E))]))
+    assert np.array_equal(so.cpu().numpy(), order)
+    assert np.array_equal(to.cpu().numpy(), order // K)
+
+
 # ---------------------------------------------------------------- decode path (T <= 4)
 
 def test_layer_decode_config0(F, w0):
