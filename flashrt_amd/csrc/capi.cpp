@@ -87,8 +87,9 @@ int dec_moe(const float* logits, const float* gate, int T, int E, int K, const u
             const uint8_t* shared_blob, const int8_t* xq, const float* xd, int n, int ff, int32_t* ids, float* wts,
             uint32_t* counts, const float* resid, float* out, void* scratch, hipStream_t stream,
             const float* prefetch = nullptr);
-int dec_hits(const uint8_t* const* hit_ptr, const int32_t* hit_n, int K, const int8_t* xq, const float* xd, int n,
-             int ff, void* scratch, float* yh, hipStream_t stream, int T);
+int dec_hits(const uint8_t* const* hit_ptr, const int32_t* hit_n, int K, int8_t* xq, float* xd, int n,
+             int ff, void* scratch, float* yh, hipStream_t stream, int T, const float* x, int x_rows);
+float* dec_window_shared(void* scratch, int T, int K, int n);
 int dec_check(int T, int K, int n, int ff);
 size_t dec_window_bytes(int T, int K, int n, int ff);
 int dec_window_fits(int T, int K, int ff);
@@ -159,7 +160,7 @@ bool shexp_type_ok(int type);
 bool shexp_shape_ok(int n, int ffs);
 size_t shexp_ws_bytes(int T, int n, int ffs);
 int shexp_run(int type, const void* g, const void* u, const void* d, int n, int ffs, const float* x, const int8_t* xq,
-              const float* xd, int T, float* sh, void* ws, hipStream_t stream);
+              const float* xd, int T, float* sh, size_t sh_ld, void* ws, hipStream_t stream);
 int hits_from_ids(const int32_t* ids, int T, int K, const uint8_t* arena, size_t stride, const uint8_t* shared,
                   const uint8_t** hit_ptr, int32_t* hit_n, hipStream_t stream);
 int slot_combine(int T, int K, int S, int n, const int32_t* ids, const float* wts, const float* Y, const float* sh,
@@ -236,6 +237,12 @@ static bool dense_small(const frt_moe_layer& L, int T) {
     const int S = L.shared_dense ? L.top_k : L.top_k + 1;   // moe_hits slots per token
     return T <= 8 && S <= 32 && (dec_shape_templated(L.d_model, L.d_ff) || dec_shape_generic(L.d_model, L.d_ff));
 }
+// Such a layer's window on the window path's kernels: its routing and grouping in one launch, and its
+// combine in the down kernel, with the dense shared expert's rows written to its slots before.
+static bool dense_window(const frt_moe_layer& L, int T) {
+    return L.shared_dense && T <= 8 && dec_shape_templated(L.d_model, L.d_ff) && dec_window_fits(T, L.top_k, L.d_ff) &&
+           router_fused_fits(T, L.d_model);
+}
 // the slot path: a dense shared expert, or a window of a shape the templated decode kernels lack
 static bool slot_path(const frt_moe_layer& L, int T) {
     if (L.shared_dense) return true;
@@ -258,7 +265,9 @@ static DenseWs dense_carve(uint8_t* p0, uint8_t* p, const frt_moe_layer& L, int 
     w.Y = reinterpret_cast<float*>(take(size_t(T) * (K + 1) * n * 4));
     w.sh = reinterpret_cast<float*>(take(size_t(T) * n * 4));
     w.shws = take(shexp_ws_bytes(T, n, L.shared_ff > 0 ? L.shared_ff : 64));
-    if (dense_small(L, T)) {
+    if (dense_window(L, T)) {
+        w.rws_bytes = dec_window_bytes(T, K, n, ff);
+    } else if (dense_small(L, T)) {
         const int S = L.shared_dense ? K : K + 1;
         w.rws_bytes = dec_scratch_bytes(hits_chunk(T, S, ff), S, ff);
     } else {
@@ -292,8 +301,22 @@ static int dense_layer(const frt_moe_layer& L, const LayerWs& lw, const DenseWs&
         if (int rc = pf_pairs(x, T, K, n, ff, E, false, false, w.rws, w.rws_bytes, norm ? w.u : nullptr,
                               q8 ? w.xq : nullptr, q8 ? w.xd : nullptr, s))
             return rc;
-    } else if (norm) {
+    } else if (norm && !(dense_window(L, T) && L.shared_type == FRT_GGML_Q8_0)) {
         if (int rc = rmsnorm(x, T, n, w.u, s)) return rc;
+    }
+    if (dense_window(L, T)) {   // (a Q8_0 shared expert needs only the codes: the norm runs in the router kernel)
+        const bool q8 = L.shared_type == FRT_GGML_Q8_0;
+        const float* in = norm && !q8 ? w.u : x;
+        if (int rc = router_logits(in, T, L.router_w, L.router_bias, L.gate_w, E, n, lw.logits, lw.gate, s, norm && q8, w.xq,
+                                   w.xd))
+            return rc;
+        timing_mark(s, "router");
+        if (int rc = shexp_run(L.shared_type, L.shared_gate, L.shared_up, L.shared_down, n, ffs, in, w.xq, w.xd, T,
+                               dec_window_shared(w.rws, T, K, n), size_t(K + 1) * n, w.shws, s))
+            return rc;
+        timing_mark(s, "shared_expert");
+        return dec_window(lw.logits, E, ids, wts, counts, lw.gate, T, K, L.experts, L.stride, nullptr, w.xq, w.xd, n, ff,
+                          resid, out, w.rws, s);
     }
     if (norm) {
         u = w.u;
@@ -325,7 +348,7 @@ static int dense_layer(const frt_moe_layer& L, const LayerWs& lw, const DenseWs&
         for (int t0 = 0; t0 < T; t0 += tc) {
             const int tn = T - t0 < tc ? T - t0 : tc;
             if (int rc = dec_hits(w.hit_ptr + size_t(t0) * S, w.hit_n + t0, S, w.xq + size_t(t0) * n,
-                                  w.xd + size_t(t0) * (n / kQ8), n, ff, w.rws, w.Y + size_t(t0) * S * n, s, tn))
+                                  w.xd + size_t(t0) * (n / kQ8), n, ff, w.rws, w.Y + size_t(t0) * S * n, s, tn, nullptr, 0))
                 return rc;
         }
     } else if (int rc = pf_run(L.experts, L.stride, E, n, ff, u, ids, T, K, w.Y, w.rws, w.rws_bytes, s, 0, 0, true)) {
@@ -335,7 +358,7 @@ static int dense_layer(const frt_moe_layer& L, const LayerWs& lw, const DenseWs&
     size_t sh_stride = size_t(S) * n;
     if (dense) {
         if (int rc = shexp_run(L.shared_type, L.shared_gate, L.shared_up, L.shared_down, n, ffs, u, w.xq, w.xd, T, w.sh,
-                               w.shws, s))
+                               size_t(n), w.shws, s))
             return rc;
         timing_mark(s, "shared_expert");
         sh = w.sh;
@@ -574,11 +597,10 @@ int frt_moe_hits(const uint8_t* const* hit_ptr, const int32_t* hit_n, int K, con
     p += up256(size_t(T) * n);
     float* xd = reinterpret_cast<float*>(p);
     p += up256(size_t(T) * (n / kQ8) * 4);
-    if (int rc = quantize_q8(x, T, n, xq, xd, nullptr, nullptr, s)) return rc;
-    for (int t0 = 0; t0 < T; t0 += tc) {   // chunks in stream order share the dec scratch
+    for (int t0 = 0; t0 < T; t0 += tc) {   // chunks in stream order share the dec scratch; the first quantizes x
         const int tn = T - t0 < tc ? T - t0 : tc;
         if (int rc = dec_hits(hit_ptr + size_t(t0) * K, hit_n + t0, K, xq + size_t(t0) * n, xd + size_t(t0) * (n / kQ8),
-                              n, ff, p, yh + size_t(t0) * K * n, s, tn))
+                              n, ff, p, yh + size_t(t0) * K * n, s, tn, t0 ? nullptr : x, T))
             return rc;
     }
     return kOk;

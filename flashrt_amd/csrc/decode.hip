@@ -36,60 +36,69 @@ namespace {
 // an item's occurrence index j among the live items of its key decides its entry (the one opened by
 // the key's occurrence 4 floor(j / 4)) and its slot in it (j mod 4); entries follow the items that
 // open them, so the list is what a serial pass over the items builds. One workgroup of at least
-// kHitsMaxItems threads (thread i: item i); s_key [kHitsMaxItems] holds the keys, s_live the flags.
+// kHitsMaxItems threads (thread i: item i, with its key and whether it takes part).
 constexpr int kHitsMaxItems = 128;
 constexpr int kGenMaxN = 16384;   // moe_hits rows of any other shape: n and ff at most these
 constexpr int kGenMaxFF = 4096;
 struct GroupLds {
     uint64_t key[kHitsMaxItems];
-    int live[kHitsMaxItems], j[kHitsMaxItems], u[kHitsMaxItems];
+    uint64_t live[kHitsMaxItems / 64];
+    int u[kHitsMaxItems];
     int wtot[2][kHitsMaxItems / 64];
 };
+// Each item's equals as a 128-bit mask: the keys are read uniformly (LDS broadcasts), eight in flight. (A
+// loop with a wait per key and a second one for the opener took 10 us of a 40-item call, all of it latency.)
 template <class BlobOf>
-__device__ __forceinline__ void group_items(GroupLds& G, int N, int K, BlobOf blob_of, DecEntry* __restrict__ ent,
-                                            int32_t* __restrict__ n_ent) {
-    const int i = int(threadIdx.x);
+__device__ __forceinline__ void group_items(GroupLds& G, int N, int K, uint64_t key, bool live, BlobOf blob_of,
+                                            DecEntry* __restrict__ ent, int32_t* __restrict__ n_ent) {
+    static_assert(kHitsMaxItems == 128, "two words of items");
+    const int i = int(threadIdx.x), wave = i >> 6;
     const bool in = i < kHitsMaxItems;
-    const bool live = in && i < N && G.live[i];
-    const uint64_t key = in ? G.key[i] : 0;
-    int j = 0, tot = 0;
-    if (live)
-        for (int q = 0; q < N; ++q) {
-            const bool same = G.live[q] && G.key[q] == key;
-            j += int(same && q < i);
-            tot += int(same);
+    const uint64_t lv = __ballot(live);
+    if (in) {
+        G.key[i] = live ? key : 0;
+        if ((i & 63) == 0) G.live[wave] = lv;
+    }
+    __syncthreads();
+    uint64_t m[2] = {0, 0};
+    for (int w = 0; w < 2; ++w) {
+        const int n = min(N - 64 * w, 64);
+        uint64_t eq = 0;
+        for (int q0 = 0; q0 < n; q0 += 8) {
+            uint64_t k[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) k[q] = G.key[64 * w + q0 + q];
+            uint32_t e8 = 0;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) e8 |= uint32_t(k[q] == key) << q;
+            eq |= uint64_t(e8) << q0;
         }
+        m[w] = eq & G.live[w];
+    }
+    const uint64_t below = (uint64_t(1) << (i & 63)) - 1;
+    const int j = live ? __popcll(m[0] & (wave == 0 ? below : ~uint64_t(0))) + (wave == 1 ? __popcll(m[1] & below) : 0) : 0;
+    const int tot = __popcll(m[0]) + __popcll(m[1]);
     const bool opens = live && j % kDecMaxT == 0;
     const int nt = opens ? min(kDecMaxT, tot - j) : 0;
     // exclusive scans over the items in order: entry index and compact base of each opener
-    const int wave = i >> 6;
     int tu = 0, tb = 0;
     const int su = wave_excl_scan(int(opens), &tu), sb = wave_excl_scan(nt, &tb);
     if (in && (i & 63) == 0) {
         G.wtot[0][wave] = tu;
         G.wtot[1][wave] = tb;
     }
-    if (in) G.j[i] = live ? j : -1;
     __syncthreads();
-    int u0 = 0, b0 = 0;
-    for (int w = 0; w < wave && w < kHitsMaxItems / 64; ++w) {
-        u0 += G.wtot[0][w];
-        b0 += G.wtot[1][w];
-    }
+    const int u0 = wave == 1 ? G.wtot[0][0] : 0, b0 = wave == 1 ? G.wtot[1][0] : 0;
     if (in) G.u[i] = u0 + su;
-    if (i == 0) {
-        int U = 0;
-        for (int w = 0; w < kHitsMaxItems / 64; ++w) U += G.wtot[0][w];
-        *n_ent = U;
-    }
+    if (i == 0) *n_ent = G.wtot[0][0] + G.wtot[0][1];
     __syncthreads();
     if (!live) return;
-    int opener = i;   // the item of this key with occurrence index 4 floor(j / 4)
-    for (int q = 0; q <= i; ++q)
-        if (G.j[q] == j - j % kDecMaxT && G.key[q] == key) {
-            opener = q;
-            break;
-        }
+    uint64_t o0 = m[0], o1 = m[1];   // the opener: the item of this key with occurrence index 4 floor(j / 4)
+    for (int q = j - j % kDecMaxT; q > 0; --q) {
+        if (o0) o0 &= o0 - 1;
+        else o1 &= o1 - 1;
+    }
+    const int opener = o0 ? __builtin_ctzll(o0) : 64 + __builtin_ctzll(o1);
     const int u = G.u[opener], sl = j % kDecMaxT, t = i / K, k = i % K;
     DecEntry& d = ent[u];
     if (opens) {
@@ -107,18 +116,30 @@ __device__ __forceinline__ void group_items(GroupLds& G, int N, int K, BlobOf bl
     d.w[sl] = 1.0f;
 }
 
-// moe_hits: the keys are the blob pointers; items k >= hit_n[t] take no part; no shared expert.
-__global__ void __launch_bounds__(kHitsMaxItems) k_hits_group(const uint8_t* const* __restrict__ hit_ptr,
-                                                              const int32_t* __restrict__ hit_n, int K, int T,
-                                                              DecEntry* __restrict__ ent, int32_t* __restrict__ n_ent) {
+// moe_hits: the keys are the blob pointers; items k >= hit_n[t] take no part; no shared expert. With x
+// (moe_hits' fp32 input, `rows` rows of n): the workgroups past the first write its Q8_0 (xq, xd), eight
+// 32-value blocks each, which nothing in the grouping waits for.
+__global__ void __launch_bounds__(256) k_hits_group(const uint8_t* const* __restrict__ hit_ptr,
+                                                    const int32_t* __restrict__ hit_n, int K, int T,
+                                                    DecEntry* __restrict__ ent, int32_t* __restrict__ n_ent,
+                                                    const float* __restrict__ x, int n_blocks, int8_t* __restrict__ xq,
+                                                    float* __restrict__ xd) {
+    const int i = int(threadIdx.x);
+    if (blockIdx.x > 0) {   // (as k_quant_q8)
+        const int blk = (int(blockIdx.x) - 1) * 8 + (i >> 5), j = i & 31;
+        const bool live = blk < n_blocks;
+        const float v = live ? x[size_t(blk) * kQ8 + j] : 0.0f;
+        const float d = q8_scale(half_max(fabsf(v)));
+        if (!live) return;
+        xq[size_t(blk) * kQ8 + j] = int8_t(q8_code(v, q8_inv(d)));
+        if (j == 0) xd[blk] = f16_round(d);
+        return;
+    }
     __shared__ GroupLds G;
-    const int i = int(threadIdx.x), N = T * K;
-    const int t = i / K, k = i % K;
+    const int N = T * K, t = i / K, k = i % K;
     const bool live = i < N && k < min(hit_n[min(t, T - 1)], K);
-    G.key[i] = live ? reinterpret_cast<uint64_t>(hit_ptr[i]) : 0;
-    G.live[i] = int(live);
-    __syncthreads();
-    group_items(G, N, K, [](uint64_t key) { return reinterpret_cast<const uint8_t*>(key); }, ent, n_ent);
+    const uint64_t key = live ? reinterpret_cast<uint64_t>(hit_ptr[i]) : 0;
+    group_items(G, N, K, key, live, [](uint64_t q) { return reinterpret_cast<const uint8_t*>(q); }, ent, n_ent);
 }
 
 // A verify window's routing and grouping in one workgroup: wave t < T routes token t (topk.hpp, the
@@ -155,7 +176,7 @@ __global__ void __launch_bounds__(512) k_win_route(const float* __restrict__ log
         }
     }
     __syncthreads();
-    const int K1 = K + 1, N = T * K1;
+    const int K1 = shared_blob ? K + 1 : K, N = T * K1;   // (no blob: the shared expert is computed elsewhere)
     const bool live = i < N;   // N <= kHitsMaxItems <= 128: waves 0 and 1
     const int t = i / K1, k = i % K1;
     const int key = live ? (k < K ? s_ids[t][k] : E) : 0;
@@ -266,7 +287,15 @@ __device__ __forceinline__ void gateup_body(const DecEntry& e, int rb, const int
     constexpr int RPW = gu_rpw<NB>();
     constexpr int ROWS = 32 / NW;                       // rows per wave
     constexpr int PASSES = gu_passes<NB, NW>();
-    __shared__ __align__(16) float seqbuf[NW][MT * 128];   // per wave: the block terms of seq_row_sums
+    // The rows' sums over their NB lanes in the CPU path's order (seq_row_sums), GP passes at a time: the
+    // terms of row r, token j, gate or up lie at (2 (r MT + j) + gu) LDF, and a lane each adds them one by
+    // one. One chain of NB dependent adds then serves up to 64 sums; a chain per pass kept two to eight
+    // lanes busy at a time (n = 2560: eight chains of 40). LDF: NB + 4, so that the lanes' 16-byte reads
+    // fall on distinct banks.
+    constexpr int GP = NW > 4 ? 1 : NB <= 40 ? PASSES : (PASSES + 1) / 2;
+    constexpr int SUMS = GP * RPW * MT * 2, LDF = NB + 4;
+    static_assert(SUMS <= 64, "one lane per sum");
+    __shared__ __align__(16) float seqbuf[NW][SUMS * LDF];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int rsub = lane / NB, b = lane % NB;
     const bool live = rsub < RPW;
@@ -366,12 +395,38 @@ __device__ __forceinline__ void gateup_body(const DecEntry& e, int rb, const int
             ag[j] = fg * dg;
             au[j] = fu * du;
         }
-        // the rows' sums over their NB lanes in the CPU path's order: lane 2 RPW j + r holds token j's
-        // row p RPW + r
-        const float2 gu = seq_row_sums<NB, RPW, MT>(ag, au, seqbuf[wave], lane);
-        const int j = lane / (2 * RPW), r = lane % (2 * RPW);
-        if (j < e.ntok && r < RPW && p * RPW + r < ROWS)
-            hrow[j][wave * ROWS + p * RPW + r] = gu.x / (1.0f + expf(-gu.x)) * gu.y;
+        const int pg = p % GP;
+        float* const buf = seqbuf[wave];
+        if (live)
+#pragma unroll
+            for (int j = 0; j < MT; ++j)
+                if (j < e.ntok) {
+                    buf[(2 * ((pg * RPW + rsub) * MT + j)) * LDF + b] = ag[j];
+                    buf[(2 * ((pg * RPW + rsub) * MT + j) + 1) * LDF + b] = au[j];
+                }
+        if (pg != GP - 1 && p != PASSES - 1) continue;
+        // the wave's LDS operations complete in order; the empty asm keeps the compiler from moving the
+        // reads of other lanes' terms above the stores
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        float sum = 0.0f;
+        if (lane < SUMS) {
+            const float4* q = reinterpret_cast<const float4*>(buf + lane * LDF);
+#pragma unroll
+            for (int i = 0; i < NB / 4; ++i) {
+                const float4 v = q[i];
+                sum = sum + v.x;
+                sum = sum + v.y;
+                sum = sum + v.z;
+                sum = sum + v.w;
+            }
+        }
+        asm volatile("" ::: "memory");   // the next group's stores stay after these reads
+        __builtin_amdgcn_wave_barrier();
+        const float up = __shfl(sum, min(lane + 1, 63));
+        const int j = (lane >> 1) % MT, r = (p - pg) * RPW + (lane >> 1) / MT;
+        if (lane < SUMS && (lane & 1) == 0 && j < e.ntok && r < ROWS)
+            hrow[j][wave * ROWS + r] = sum / (1.0f + expf(-sum)) * up;
     }
     __syncthreads();
     // Q8_0 of the 32-row block of h for each token: wave w < ntok, lanes 0..31
@@ -993,7 +1048,8 @@ int dec_moe(const float* logits, const float* gate, int T, int E, int K, const u
 // one launch per window of up to kDecMaxHitsT tokens (the reference's kMaxWindow, moe_fast.cu:38),
 // each distinct expert's rows read once per four of its tokens.
 static int hits_run(const uint8_t* const* hit_ptr, const int32_t* hit_n, int K, const int8_t* xq, const float* xd,
-                    int n, int ff, void* scratch, float* yh, hipStream_t stream, int T, const WinComb& wc) {
+                    int n, int ff, void* scratch, float* yh, hipStream_t stream, int T, const WinComb& wc,
+                    const float* x = nullptr, int x_rows = 0, int8_t* xq_w = nullptr, float* xd_w = nullptr) {
     if (T < 1 || T > kDecMaxHitsT || K < 1 || K > 32 || T * K > kHitsMaxItems)
         return set_error(kErrShape, "moe_hits: T=%d K=%d (T <= %d, T*K <= %d per launch)", T, K, kDecMaxHitsT, kHitsMaxItems);
     const bool tmpl = dec_shape_templated(n, ff);
@@ -1002,7 +1058,8 @@ static int hits_run(const uint8_t* const* hit_ptr, const int32_t* hit_n, int K, 
                          n, ff, kGenMaxN, kGenMaxFF);
     const DecScratch s = dec_carve(scratch, T, K, ff);
     if (hit_ptr) {   // (null: the caller has filled the entry list, dec_window)
-        k_hits_group<<<1, kHitsMaxItems, 0, stream>>>(hit_ptr, hit_n, K, T, s.ent, s.n_ent);
+        const int nb = x ? x_rows * (n / kQ8) : 0;
+        k_hits_group<<<1 + (nb + 7) / 8, 256, 0, stream>>>(hit_ptr, hit_n, K, T, s.ent, s.n_ent, x, nb, xq_w, xd_w);
         timing_mark(stream, "hits_group");
     }
     if (!tmpl) {   // a shape outside the templated set: the runtime-shape kernels
@@ -1027,9 +1084,10 @@ static int hits_run(const uint8_t* const* hit_ptr, const int32_t* hit_n, int K, 
     timing_mark(stream, "dec_gateup");
     return dec_down(s, n, ff, T, K, nullptr, nullptr, yh, stream, nullptr, 0, wc);
 }
-int dec_hits(const uint8_t* const* hit_ptr, const int32_t* hit_n, int K, const int8_t* xq, const float* xd, int n,
-             int ff, void* scratch, float* yh, hipStream_t stream, int T) {
-    return hits_run(hit_ptr, hit_n, K, xq, xd, n, ff, scratch, yh, stream, T, WinComb{});
+// x (or null): fp32 rows whose Q8_0 the call writes to xq / xd first (x_rows of them, from xq's first row)
+int dec_hits(const uint8_t* const* hit_ptr, const int32_t* hit_n, int K, int8_t* xq, float* xd, int n,
+             int ff, void* scratch, float* yh, hipStream_t stream, int T, const float* x, int x_rows) {
+    return hits_run(hit_ptr, hit_n, K, xq, xd, n, ff, scratch, yh, stream, T, WinComb{}, x, x_rows, xq, xd);
 }
 
 // A verify window (T <= 8) after routing: ids / wts [T][K], gate [T], the window's Q8_0 input ->
@@ -1045,6 +1103,12 @@ int dec_window_fits(int T, int K, int ff) {
     // (the window path runs moe_hits over K + 1 slots per token, the shared expert last: K + 1 <= 32)
     return T >= 1 && T <= kDecMaxHitsT && K + 1 <= 32 && T * (K + 1) <= kHitsMaxItems;
 }
+// The shared expert's rows of the window's per-slot outputs: token t's at dec_window_shared() + t (K + 1) n.
+float* dec_window_shared(void* scratch, int T, int K, int n) {
+    uint8_t* p = static_cast<uint8_t*>(scratch) + up256(size_t(T) * (K + 1) * 8) + 256 + up256(size_t(n / 8) * 4);
+    return reinterpret_cast<float*>(p) + size_t(K) * n;
+}
+// shared_blob null: the caller writes the shared expert's rows (dec_window_shared) before this call.
 int dec_window(const float* logits, int E, int32_t* ids, float* wts, uint32_t* counts, const float* gate, int T, int K,
                const uint8_t* arena, size_t stride, const uint8_t* shared_blob, const int8_t* xq, const float* xd, int n,
                int ff, const float* resid, float* out, void* scratch, hipStream_t stream) {

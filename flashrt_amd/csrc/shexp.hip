@@ -76,12 +76,13 @@ __device__ __forceinline__ void q8_pair(const uint8_t* row, int p, uint32_t (&q0
 }
 
 // rows r of W1 (and W2, DUAL) against TT tokens t0 .. : out[t][r] = W1 a_t (DUAL: silu(W1 a_t) * W2 a_t).
-// a: fp32 [T][cols] (dense types) or Q8_0 codes aq [T][cols] with scales ad [T][cols/32] (Q8_0).
+// a: fp32 [T][cols] (dense types; Q8_0 down, which quantizes its h while staging it) or Q8_0 codes aq
+// [T][cols] with scales ad [T][cols/32] (Q8_0 gate / up). out rows are out_ld apart.
 template <int TYPE, bool DUAL>
 __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ W1, const uint8_t* __restrict__ W2,
                                                      int rows, int cols, const float* __restrict__ af,
                                                      const int8_t* __restrict__ aq, const float* __restrict__ ad, int T,
-                                                     float* __restrict__ out) {
+                                                     float* __restrict__ out, size_t out_ld) {
     constexpr bool Q8 = TYPE == FRT_GGML_Q8_0;
     __shared__ __align__(16) float s_af[Q8 ? 1 : kShTT * kShMaxCols];
     __shared__ __align__(16) int8_t s_aq[Q8 ? kShTT * kShMaxCols : 16];
@@ -89,7 +90,18 @@ __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int t0 = blockIdx.y * kShTT, tn = min(kShTT, T - t0);
     // the token tile's activations into LDS
-    if (Q8) {
+    if (Q8 && !DUAL) {   // h to Q8_0, a 32-value block per half wave (as k_quant_q8)
+        const int nb = tn * cols / kQ8, j = tid & 31;
+        for (int i0 = 0; i0 < nb; i0 += kShNT / 32) {
+            const int i = i0 + (tid >> 5);
+            const float v = i < nb ? af[size_t(t0) * cols + size_t(i) * kQ8 + j] : 0.0f;
+            const float d = q8_scale(half_max(fabsf(v)));
+            if (i < nb) {
+                s_aq[i * kQ8 + j] = int8_t(q8_code(v, q8_inv(d)));
+                if (j == 0) s_ad[i] = f16_round(d);
+            }
+        }
+    } else if (Q8) {
         const int nw = tn * cols / 4;
         for (int i = tid; i < nw; i += kShNT)
             reinterpret_cast<uint32_t*>(s_aq)[i] = reinterpret_cast<const uint32_t*>(aq + size_t(t0) * cols)[i];
@@ -170,9 +182,9 @@ __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ 
         const float g = wave_sum_tree(acc1[t]);
         if (DUAL) {
             const float u = wave_sum_tree(acc2[t]);
-            if (lane == 0) out[size_t(t0 + t) * rows + r] = g / (1.0f + expf(-g)) * u;
+            if (lane == 0) out[size_t(t0 + t) * out_ld + r] = g / (1.0f + expf(-g)) * u;
         } else if (lane == 0) {
-            out[size_t(t0 + t) * rows + r] = g;
+            out[size_t(t0 + t) * out_ld + r] = g;
         }
     }
 }
@@ -551,13 +563,13 @@ bool shexp_shape_ok(int n, int ffs) {
 
 // W (rows x cols) against T tokens; DUAL: W1, W2 and the SwiGLU.
 static int shexp_mv(int type, bool dual, const void* W1, const void* W2, int rows, int cols, const float* af,
-                    const int8_t* aq, const float* ad, int T, float* out, hipStream_t stream) {
+                    const int8_t* aq, const float* ad, int T, float* out, size_t out_ld, hipStream_t stream) {
     const dim3 grid((rows + 3) / 4, (T + kShTT - 1) / kShTT);
     const uint8_t* w1 = static_cast<const uint8_t*>(W1);
     const uint8_t* w2 = static_cast<const uint8_t*>(W2);
 #define FRT_SH(TY)                                                                                                  \
-    if (dual) k_shexp_mv<TY, true><<<grid, kShNT, 0, stream>>>(w1, w2, rows, cols, af, aq, ad, T, out);             \
-    else k_shexp_mv<TY, false><<<grid, kShNT, 0, stream>>>(w1, w2, rows, cols, af, aq, ad, T, out);
+    if (dual) k_shexp_mv<TY, true><<<grid, kShNT, 0, stream>>>(w1, w2, rows, cols, af, aq, ad, T, out, out_ld);             \
+    else k_shexp_mv<TY, false><<<grid, kShNT, 0, stream>>>(w1, w2, rows, cols, af, aq, ad, T, out, out_ld);
     switch (type) {
         case FRT_GGML_F32: FRT_SH(FRT_GGML_F32) break;
         case FRT_GGML_F16: FRT_SH(FRT_GGML_F16) break;
@@ -577,7 +589,7 @@ int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16
 constexpr int kShMmMinT = 9;
 
 size_t shexp_ws_bytes(int T, int n, int ffs) {
-    const size_t mv = up256(size_t(T) * ffs * 4) + up256(size_t(T) * ffs) + up256(size_t(T) * (ffs / kQ8) * 4);
+    const size_t mv = up256(size_t(T) * ffs * 4);
     if (T < kShMmMinT) return mv;
     const size_t mm = up256(size_t(T) * n * 6) + up256(size_t(T) * ffs * 6);   // the bf16 planes of x and h
     return mv > mm ? mv : mm;
@@ -616,31 +628,24 @@ static int shexp_run_mm(const void* g, const void* u, const void* d, int n, int 
     return kOk;
 }
 
-// sh [T][n] = the shared expert of type `type` on u [T][n]; uq/ud: u's Q8_0 (Q8_0 type only; may be
-// null, then computed into the workspace's h area first... the caller passes them). ws: shexp_ws_bytes.
+// sh (rows of n, sh_ld apart; n from kShMmMinT tokens on) = the shared expert of type `type` on x [T][n];
+// xq / xd: x's Q8_0 (Q8_0 type only). ws: shexp_ws_bytes.
 int shexp_run(int type, const void* g, const void* u, const void* d, int n, int ffs, const float* x, const int8_t* xq,
-              const float* xd, int T, float* sh, void* ws, hipStream_t stream) {
+              const float* xd, int T, float* sh, size_t sh_ld, void* ws, hipStream_t stream) {
     if (!shexp_type_ok(type)) return set_error(kErrShape, "shared expert: ggml type %d (F32, F16, BF16 or Q8_0)", type);
     if (!shexp_shape_ok(n, ffs)) return set_error(kErrShape, "shared expert: n=%d ffs=%d", n, ffs);
+    if (T >= kShMmMinT && sh_ld != size_t(n)) return set_error(kErrShape, "shared expert: row distance %zu", sh_ld);
     if (T >= kShMmMinT) switch (type) {
         case FRT_GGML_F32: return shexp_run_mm<FRT_GGML_F32>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
         case FRT_GGML_F16: return shexp_run_mm<FRT_GGML_F16>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
         case FRT_GGML_BF16: return shexp_run_mm<FRT_GGML_BF16>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
         default: return shexp_run_mm<FRT_GGML_Q8_0>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
     }
-    uint8_t* p = static_cast<uint8_t*>(ws);
-    float* h = reinterpret_cast<float*>(p);
-    p += up256(size_t(T) * ffs * 4);
-    int8_t* hq = reinterpret_cast<int8_t*>(p);
-    p += up256(size_t(T) * ffs);
-    float* hd = reinterpret_cast<float*>(p);
-    if (type == FRT_GGML_Q8_0) {
-        if (int rc = shexp_mv(type, true, g, u, ffs, n, nullptr, xq, xd, T, h, stream)) return rc;
-        if (int rc = quantize_q8(h, T, ffs, hq, hd, nullptr, nullptr, stream)) return rc;
-        return shexp_mv(type, false, d, nullptr, n, ffs, nullptr, hq, hd, T, sh, stream);
-    }
-    if (int rc = shexp_mv(type, true, g, u, ffs, n, x, nullptr, nullptr, T, h, stream)) return rc;
-    return shexp_mv(type, false, d, nullptr, n, ffs, h, nullptr, nullptr, T, sh, stream);
+    // h [T][ffs] fp32; the down product quantizes it (Q8_0) or takes it as it is
+    float* h = static_cast<float*>(ws);
+    const bool q8 = type == FRT_GGML_Q8_0;
+    if (int rc = shexp_mv(type, true, g, u, ffs, n, q8 ? nullptr : x, xq, xd, T, h, size_t(ffs), stream)) return rc;
+    return shexp_mv(type, false, d, nullptr, n, ffs, h, nullptr, nullptr, T, sh, sh_ld, stream);
 }
 
 int hits_from_ids(const int32_t* ids, int T, int K, const uint8_t* arena, size_t stride, const uint8_t* shared,
