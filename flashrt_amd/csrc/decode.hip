@@ -445,14 +445,17 @@ __device__ __forceinline__ void gateup_body(const DecEntry& e, int rb, const int
 }
 
 // Four waves per workgroup (8 ff rows each): at n <= 2048 three workgroups fit per CU without
-// register spills (12 waves, against 8 for one 8-wave workgroup); wider rows fit two.
+// register spills (12 waves, against 8 for one 8-wave workgroup); wider rows fit two. The entry is read
+// beside the count (the list holds a slot for every item), not after it: 14.2 -> 13.6 us at 8 tokens.
 template <int NB>
 __global__ void __launch_bounds__(256, NB > 32 ? 2 : 3) k_dec_gateup(const DecEntry* __restrict__ ent, const int32_t* __restrict__ n_ent,
                                                     const int8_t* __restrict__ xq, const float* __restrict__ xd, int n,
                                                     int ff, int8_t* __restrict__ hq, float* __restrict__ hd) {
     __shared__ float hrow[kDecMaxT][32];
-    if (int(blockIdx.y) >= *n_ent) return;
+    const int U = *n_ent;
     const DecEntry e = ent[blockIdx.y];
+    asm volatile("" ::"s"(U), "s"(e.blob), "s"(e.ntok));   // (both loads issued before the branch)
+    if (int(blockIdx.y) >= U) return;
     gateup_body<NB, 4>(e, blockIdx.x, xq, xd, n, ff, hq, hd, hrow);
 }
 
@@ -673,12 +676,24 @@ __global__ void __launch_bounds__(256) k_hits_down(const DecEntry* __restrict__ 
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ DecEntry s_ent[kHitsDownEnt];
     const int U = *n_ent, u_lo = int(blockIdx.y) * kHitsDownEnt;
+    // the chunk's slot ranges, read beside the count (the list holds a slot for every item and more)
+    int e_base[kHitsDownEnt], e_n[kHitsDownEnt];
+#pragma unroll
+    for (int u = 0; u < kHitsDownEnt; ++u) {
+        e_base[u] = ent_g[u_lo + u].base;
+        e_n[u] = ent_g[u_lo + u].ntok;
+    }
+#pragma unroll
+    for (int u = 0; u < kHitsDownEnt; ++u) asm volatile("" ::"s"(e_base[u]), "s"(e_n[u]));
     if (u_lo >= U) return;
     const int nu = min(U - u_lo, kHitsDownEnt);
     const int r0 = blockIdx.x * RD, tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const DecEntry* eg = ent_g + u_lo;
-    const int c_lo = eg[0].base, c_hi = eg[nu - 1].base + eg[nu - 1].ntok;   // this chunk's compact slots
+    const int c_lo = e_base[0];   // this chunk's compact slots
+    int c_hi = c_lo;
+#pragma unroll
+    for (int u = 0; u < kHitsDownEnt; ++u) c_hi = u == nu - 1 ? e_base[u] + e_n[u] : c_hi;
     const int nc = c_hi - c_lo;
     int8_t* sh_q = reinterpret_cast<int8_t*>(smem);                       // [nc][ff]
     float* sh_d = reinterpret_cast<float*>(smem + size_t(kHitsDownEnt * kDecMaxT) * ff);   // [nc][ff/32]

@@ -24,8 +24,10 @@ __device__ __forceinline__ void quant32(float v, int j, int8_t* q, float* d) {
     if (j == 0) *d = f16_round(dd);
 }
 
-// ---- router: grid (ceil(rows / W), ceil(T / tok_per_wg)), W = blockDim.x / 64 waves, one router row
-// each (W = 2 for decode windows, so that the 4 MiB of router rows spread over twice as many CUs).
+// ---- router: grid (ceil(rows / W), ceil(T / tok_per_wg)), W = wg_rows router rows per workgroup (2 for
+// decode windows, so that the 4 MiB of router rows spread over twice as many CUs), blockDim.x / 64 / W
+// waves each, which share the row's tokens (two waves from 4 tokens on: staging the tokens, their RMS
+// scales and their dot products are serial per wave, 11.6 us at 8 tokens with one).
 // Rows 0..E-1 are the router (bias optional); row E (when gate_w) is the shared expert's gate.
 // x tiles of TT tokens are staged in LDS with each 64-chain padded by one float (conflict-free).
 // norm: the layer input is u = x * r, r the canonical RMS scale of the token (topk.hpp); u_i is
@@ -37,12 +39,13 @@ __global__ void __launch_bounds__(256) k_router(const float* __restrict__ x, int
                                                 const float* __restrict__ bias, const float* __restrict__ gate_w,
                                                 int E, float* __restrict__ logits, float* __restrict__ gate, int TT,
                                                 int tok_per_wg, int norm, int8_t* __restrict__ xq,
-                                                float* __restrict__ xd) {
+                                                float* __restrict__ xd, int wg_rows) {
     extern __shared__ float xs[];   // [TT][64][L + 1]
     __shared__ float s_r[64];
     const int n = 64 * L;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int row = blockIdx.x * (blockDim.x >> 6) + wave;
+    const int row = blockIdx.x * wg_rows + wave % wg_rows;
+    const int tg = wave / wg_rows, ts = int(blockDim.x >> 6) / wg_rows;   // this wave's tokens: tg, tg + ts, ..
     const bool is_gate = row == E;
     const bool live = row < E || (is_gate && gate_w);
     const float* w = is_gate ? gate_w : W + size_t(row < E ? row : 0) * n;
@@ -67,20 +70,20 @@ __global__ void __launch_bounds__(256) k_router(const float* __restrict__ x, int
         // the previous tile's LDS reads are done (none before the first tile: its x loads then
         // issue right behind the row loads, without a fence waiting for those)
         if (t0 != t_begin) __syncthreads();
-        // x tile into LDS, 4 loads per thread in flight before their LDS writes (clamped indices, no
+        // x tile into LDS, 8 loads per thread in flight before their LDS writes (clamped indices, no
         // branches, which would let the compiler sink each load to its write: past the end a thread
         // rewrites the last element with its own value)
         const int nx = tn * (n / 4);
-        for (int i0 = threadIdx.x; i0 < nx; i0 += 4 * int(blockDim.x)) {
-            float4 v[4];
+        for (int i0 = threadIdx.x; i0 < nx; i0 += 8 * int(blockDim.x)) {
+            float4 v[8];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < 8; ++u) {
                 const int i = min(i0 + u * int(blockDim.x), nx - 1);
                 const int t = i / (n / 4), k = (i % (n / 4)) * 4;
                 v[u] = *reinterpret_cast<const float4*>(x + size_t(t0 + t) * n + k);
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < 8; ++u) {
                 const int i = min(i0 + u * int(blockDim.x), nx - 1);
                 const int t = i / (n / 4), k = (i % (n / 4)) * 4;
                 float* dst = xs + (t * 64 + k / L) * (L + 1) + k % L;   // L % 4 == 0: one chain
@@ -110,7 +113,7 @@ __global__ void __launch_bounds__(256) k_router(const float* __restrict__ x, int
             }
         }
         if (!live) continue;
-        for (int t = 0; t < tn; ++t) {
+        for (int t = tg; t < tn; t += ts) {
             const float* xc = xs + (t * 64 + lane) * (L + 1);
             float acc = 0.0f;
             if (norm) {
@@ -346,14 +349,15 @@ int router_logits(const float* x, int T, const float* W, const float* bias, cons
     const int tok_per_wg = T <= TT ? T : 64;
     if (xq && T > TT) return set_error(kErrShape, "router: fused quantization needs T <= %d", TT);
     const int wg_rows = T <= TT ? 2 : 4;   // decode: 2 rows per workgroup; token tiles: 4
+    const int waves = T <= TT && T >= 4 ? 2 * wg_rows : wg_rows;
     dim3 grid((rows + wg_rows - 1) / wg_rows, (T + tok_per_wg - 1) / tok_per_wg);
 #define FRT_ROUTER_L(LL)                                                                                         \
     case LL:                                                                                                     \
         if (smem > 65536)                                                                                        \
             FRT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_router<LL>),                            \
                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(smem)));                 \
-        launch_timed("router_quant", k_router<LL>, grid, dim3(64 * wg_rows), smem, stream, x, T, W, bias, gate_w, E, \
-                     logits, gate, TT, tok_per_wg, norm, xq, xd);                                                    \
+        launch_timed("router_quant", k_router<LL>, grid, dim3(64 * waves), smem, stream, x, T, W, bias, gate_w, E,   \
+                     logits, gate, TT, tok_per_wg, norm, xq, xd, wg_rows);                                           \
         break;
     switch (L) {
         FRT_ROUTER_L(8) FRT_ROUTER_L(16) FRT_ROUTER_L(24) FRT_ROUTER_L(32) FRT_ROUTER_L(40) FRT_ROUTER_L(48)
