@@ -449,7 +449,11 @@ __device__ __forceinline__ int window_entries(const float* __restrict__ logits, 
 // of its lanes holds one 64-block of one of the RD = 8 rows r0 .. r0 + 7.
 template <int NBF, int BATCH>
 struct DownRegs {
-    static constexpr int RPP = 64 / NBF;   // rows per wave pass
+    // lanes per row: the row's blocks rounded up to a power of two (10 blocks: 16 lanes, 4 rows a pass, as
+    // many passes as 6 rows would take), so that a row's sum is a DPP tree and not NBF shuffles
+    static constexpr int LPR = NBF <= 4 ? 4 : NBF <= 8 ? 8 : 16;
+    static_assert(NBF <= 16, "a row's blocks within 16 lanes");
+    static constexpr int RPP = 64 / LPR;   // rows per wave pass
     static constexpr int RD = 8;           // rows per workgroup
     static constexpr int PASSES = (RD + RPP - 1) / RPP;
     uint4 cd[BATCH][PASSES];
@@ -464,8 +468,8 @@ __device__ __forceinline__ void down_load(const DecEntry* ent, int U, int u0, in
                                           DownRegs<NBF, BATCH>& R) {
     using D = DownRegs<NBF, BATCH>;
     const int lane = threadIdx.x & 63;
-    const int rsub = lane / NBF, b = lane % NBF;
-    const bool live = rsub < D::RPP;
+    const int rsub = lane / D::LPR, b = lane % D::LPR;
+    const bool live = b < NBF;
     const size_t dbase = 2 * mat_bytes(ff, n);
     // The entries' blob pointers in one vector load (lane i < BATCH: entry u0 + 4 i; lane BATCH:
     // entry 0, which stands in for entries past U; the entry array holds at least 4 BATCH entries,
@@ -506,8 +510,8 @@ __device__ __forceinline__ void down_compute1(int U, int u0, const DownRegs<NBF,
                                               const float* sh_d, float* sh_y, int ff) {
     using D = DownRegs<NBF, BATCH>;
     const int lane = threadIdx.x & 63;
-    const int rsub = lane / NBF, b = lane % NBF;
-    const bool live = rsub < D::RPP;
+    const int rsub = lane / D::LPR, b = lane % D::LPR;
+    const bool live = b < NBF;
     float part[BATCH][D::PASSES];
 #pragma unroll
     for (int i = 0; i < BATCH; ++i) {
@@ -551,14 +555,7 @@ __device__ __forceinline__ void down_compute1(int U, int u0, const DownRegs<NBF,
     for (int i = 0; i < BATCH; ++i)
 #pragma unroll
         for (int p = 0; p < D::PASSES; ++p) {
-            float v = part[i][p];
-            if ((NBF & (NBF - 1)) == 0 && NBF <= 16) {
-                v = group_sum<(NBF <= 16 ? NBF : 16)>(v);
-            } else {
-                float acc = 0.0f;
-                for (int q = 0; q < NBF; ++q) acc += __shfl(v, rsub * NBF + q, 64);
-                v = acc;
-            }
+            const float v = group_sum<D::LPR>(part[i][p]);
             const int rl = p * D::RPP + rsub;
             if (u0 + US * i < U && live && b == 0 && rl < D::RD) sh_y[(u0 + US * i) * D::RD + rl] = v;
         }
@@ -571,59 +568,50 @@ __device__ __forceinline__ void down_compute(const DecEntry* ent, int U, int u0,
                                              const int8_t* sh_q, const float* sh_d, float* sh_y, int ff) {
     using D = DownRegs<NBF, BATCH>;
     const int lane = threadIdx.x & 63;
-    const int rsub = lane / NBF, b = lane % NBF;
-    const bool live = rsub < D::RPP;
+    const int rsub = lane / D::LPR, b = lane % D::LPR;
+    const bool live = b < NBF;
 #pragma unroll
     for (int i = 0; i < BATCH; ++i) {
         const int u = u0 + US * i;
         if (u >= U) break;
         const DecEntry& e = ent[u];
+        const int nt = e.ntok, base = e.base, bb = live ? b : 0;
+        for (int j = 0; j < nt; ++j) {   // a token's h block, code sums and scales once for the entry's rows
+            const int c = base + j;
+            const int4* hp = reinterpret_cast<const int4*>(sh_q + size_t(c) * ff + bb * kBlock);
+            int ha[16];
 #pragma unroll
-        for (int p = 0; p < D::PASSES; ++p) {
-            const int rl = p * D::RPP + rsub;
-            const bool ok = (R.ok >> (i * D::PASSES + p)) & 1u;
-            const uint32_t wd[4] = {ok ? R.cd[i][p].x : 0u, ok ? R.cd[i][p].y : 0u, ok ? R.cd[i][p].z : 0u,
-                                    ok ? R.cd[i][p].w : 0u};
-            const float dw = ok ? h2f(uint16_t(R.sd[i][p])) : 0.0f;
-            for (int j = 0; j < e.ntok; ++j) {
-                const int c = e.base + j;
-                float part = 0.0f;
-                if (live && rl < D::RD) {
-                    const int4* hp = reinterpret_cast<const int4*>(sh_q + size_t(c) * ff + b * kBlock);
-                    int ha[16];
+            for (int q = 0; q < 4; ++q) {
+                const int4 v = hp[q];
+                ha[4 * q] = v.x;
+                ha[4 * q + 1] = v.y;
+                ha[4 * q + 2] = v.z;
+                ha[4 * q + 3] = v.w;
+            }
+            const float d0 = sh_d[size_t(c) * (ff / kQ8) + 2 * bb], d1 = sh_d[size_t(c) * (ff / kQ8) + 2 * bb + 1];
+            int s0 = 0, s1 = 0;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int4 v = hp[q];
-                        ha[4 * q] = v.x;
-                        ha[4 * q + 1] = v.y;
-                        ha[4 * q + 2] = v.z;
-                        ha[4 * q + 3] = v.w;
-                    }
-                    int s0 = 0, s1 = 0, q0 = 0, q1 = 0;
+            for (int i2 = 0; i2 < 8; ++i2) s0 = dot4(ha[i2], 0x01010101, s0);
 #pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        q0 = dot4(int(wd[w] & 0x03030303u), ha[w], q0);
-                        q0 = dot4(int((wd[w] >> 2) & 0x03030303u), ha[4 + w], q0);
-                        q1 = dot4(int((wd[w] >> 4) & 0x03030303u), ha[8 + w], q1);
-                        q1 = dot4(int((wd[w] >> 6) & 0x03030303u), ha[12 + w], q1);
-                    }
+            for (int i2 = 8; i2 < 16; ++i2) s1 = dot4(ha[i2], 0x01010101, s1);
 #pragma unroll
-                    for (int i2 = 0; i2 < 8; ++i2) s0 = dot4(ha[i2], 0x01010101, s0);
+            for (int p = 0; p < D::PASSES; ++p) {
+                const int rl = p * D::RPP + rsub;
+                const bool ok = (R.ok >> (i * D::PASSES + p)) & 1u;
+                const uint32_t wd[4] = {ok ? R.cd[i][p].x : 0u, ok ? R.cd[i][p].y : 0u, ok ? R.cd[i][p].z : 0u,
+                                        ok ? R.cd[i][p].w : 0u};
+                const float dw = ok ? h2f(uint16_t(R.sd[i][p])) : 0.0f;
+                int q0 = 0, q1 = 0;
 #pragma unroll
-                    for (int i2 = 8; i2 < 16; ++i2) s1 = dot4(ha[i2], 0x01010101, s1);
-                    const float f = float(q0 - s0) * sh_d[size_t(c) * (ff / kQ8) + 2 * b] +
-                                    float(q1 - s1) * sh_d[size_t(c) * (ff / kQ8) + 2 * b + 1];
-                    part = f * dw;
+                for (int w = 0; w < 4; ++w) {
+                    q0 = dot4(int(wd[w] & 0x03030303u), ha[w], q0);
+                    q0 = dot4(int((wd[w] >> 2) & 0x03030303u), ha[4 + w], q0);
+                    q1 = dot4(int((wd[w] >> 4) & 0x03030303u), ha[8 + w], q1);
+                    q1 = dot4(int((wd[w] >> 6) & 0x03030303u), ha[12 + w], q1);
                 }
-                if ((NBF & (NBF - 1)) == 0 && NBF <= 16) {
-                    part = group_sum<(NBF <= 16 ? NBF : 16)>(part);
-                } else {
-                    // segments of NBF lanes: gather the row's partials from its first lane
-                    float acc = 0.0f;
-                    for (int q = 0; q < NBF; ++q) acc += __shfl(part, rsub * NBF + q, 64);
-                    part = acc;
-                }
-                if (live && b == 0 && rl < D::RD) sh_y[c * D::RD + rl] = part;
+                const float f = float(q0 - s0) * d0 + float(q1 - s1) * d1;
+                const float y = group_sum<D::LPR>(live && rl < D::RD ? f * dw : 0.0f);
+                if (b == 0 && rl < D::RD) sh_y[c * D::RD + rl] = y;
             }
         }
     }
