@@ -249,8 +249,15 @@ __global__ void __launch_bounds__(64) k_pf_place(const int32_t* __restrict__ ids
 // kernels above. What bounds either is launches and latency: 21 -> 9 us for 370 slots. (Longer chunks keep
 // the four kernels: one workgroup would walk them serially, 36 against 24 us at 20480 slots.)
 constexpr int kSmallSlots = 4096;
+// The tokens per tile of a chunk of S slots (k_pf_dispatch1's tn): with few slots there are fewer
+// workgroups than the chip holds, and a 64-token tile's serial K loop (32 stages) sets the time; tiles of
+// 16 tokens are more and shorter, at the price of weights dequantized once per 16 tokens. Layers of 37
+// and 64 tokens (skewed): 78.5 -> 64.1 and 81.3 -> 73.1 us; 93 (even): unchanged; 140: 145.0 -> 146.1 skewed,
+// 190.4 -> 181.7 with 16 hot experts; 200: 162 -> 169; 340: 194 -> 206.
+constexpr int kTile16Slots = 1536;
+static int pf_tile_tokens(int S) { return S <= kTile16Slots ? 16 : kTN; }
 __global__ void __launch_bounds__(1024) k_pf_dispatch1(const int32_t* __restrict__ ids, int S, int K, int E, int id_bits, int T,
-                                                       int shared, int32_t* __restrict__ bounds, int2* __restrict__ tiles,
+                                                       int shared, int tn, int32_t* __restrict__ bounds, int2* __restrict__ tiles,
                                                        int32_t* __restrict__ n_tiles, int32_t* __restrict__ tok_of,
                                                        int32_t* __restrict__ slot_of) {
     extern __shared__ int32_t hist[];
@@ -299,34 +306,40 @@ __global__ void __launch_bounds__(1024) k_pf_dispatch1(const int32_t* __restrict
             hist[w * E + tid] = rows;
             rows += c;
         }
-    // tiles per class (as pf_scan_body counts them) and rows, scanned together
-    const int full = rows / kTN, rest = rows % kTN, kr = rest ? tile_class(rest) : 0;
-    const int v[5] = {rows, int(kr == 1), int(kr == 2), int(kr == 3), full + int(kr == 4)};
+    // tiles per class (as pf_scan_body counts them; tn = 16: all of class 1) and rows, scanned together.
+    // full tiles are of class 4 (tn = 64) or 1, the rest tile of class kr; a class ends with the shared
+    // group's tiles.
+    const int fc = tn == kTN ? 4 : 1;
+    const int full = rows / tn, rest = rows % tn, kr = rest ? tile_class(rest) : 0;
+    const int v[5] = {rows, int(kr == 1) + (fc == 1 ? full : 0), int(kr == 2), int(kr == 3), int(kr == 4) + (fc == 4 ? full : 0)};
     int r[5], tot[5];
     block_excl_scan_v<5>(v, r, tot, ws);
-    const int sfull = shared ? T / kTN : 0, srest = shared ? T % kTN : 0, sk = srest ? tile_class(srest) : 0;
-    int base[5];   // first tile of each class; the shared group's tiles close each class
+    const int sfull = shared ? T / tn : 0, srest = shared ? T % tn : 0, sk = srest ? tile_class(srest) : 0;
+    int base[5], at[5];   // first tile of each class ([0]: their number); this group's first tile of each
     base[4] = 0;
-    base[3] = tot[4] + sfull + int(sk == 4);
-    base[2] = base[3] + tot[3] + int(sk == 3);
-    base[1] = base[2] + tot[2] + int(sk == 2);
+    for (int k = 3; k >= 0; --k) base[k] = base[k + 1] + tot[k + 1] + (fc == k + 1 ? sfull : 0) + int(sk == k + 1);
+    for (int k = 1; k <= 4; ++k) at[k] = base[k] + r[k];
     if (tid < E) {
         bounds[tid] = r[0];
         s_row[tid] = r[0];
-        for (int i = 0; i < full; ++i) tiles[r[4] + i] = make_int2(tid, i * kTN);
+        for (int i = 0; i < full; ++i) tiles[(fc == 4 ? at[4] : at[1]) + i] = make_int2(tid, i * tn);
         if (kr) {
-            const int at = kr == 4 ? r[4] + full : (kr == 3 ? base[3] + r[3] : kr == 2 ? base[2] + r[2] : base[1] + r[1]);
-            tiles[at] = make_int2(tid, full * kTN);
+            const int p = kr == 4 ? at[4] : kr == 3 ? at[3] : kr == 2 ? at[2] : at[1];
+            tiles[p + (kr == fc ? full : 0)] = make_int2(tid, full * tn);
         }
     }
     if (tid == 0) {
         bounds[E] = tot[0];
         if (shared) {
             bounds[E + 1] = tot[0] + T;
-            for (int i = 0; i < sfull; ++i) tiles[tot[4] + i] = make_int2(E, i * kTN);
-            if (sk) tiles[sk == 4 ? tot[4] + sfull : base[sk] + tot[sk]] = make_int2(E, sfull * kTN);
+            const int p = fc == 4 ? base[4] + tot[4] : base[1] + tot[1];
+            for (int i = 0; i < sfull; ++i) tiles[p + i] = make_int2(E, i * tn);
+            if (sk) {
+                const int q = sk == 4 ? base[4] + tot[4] : sk == 3 ? base[3] + tot[3] : sk == 2 ? base[2] + tot[2] : base[1] + tot[1];
+                tiles[q + (sk == fc ? sfull : 0)] = make_int2(E, sfull * tn);
+            }
         }
-        n_tiles[0] = base[1] + tot[1] + int(sk == 1);
+        n_tiles[0] = base[0];
         n_tiles[1] = base[1];
     }
     __syncthreads();
@@ -918,7 +931,7 @@ struct PfWs {
     size_t bytes;
 };
 
-static int pf_max_tiles(int S, int G) { return (S + kTN - 1) / kTN + G; }
+static int pf_max_tiles(int S, int G) { return (S + pf_tile_tokens(S) - 1) / pf_tile_tokens(S) + G; }
 // the gate/up GEMM's K extent: n rounded up to whole pairs of 256-element stretches
 static int pf_np(int n) { return (n + 511) & ~511; }
 
@@ -1015,7 +1028,7 @@ static int pf_dispatch_run(const int32_t* ids, int T, int K, int E, bool shared,
             done = true;
         }
         launch_timed("pf_dispatch1", k_pf_dispatch1, dim3(1), dim3(1024), lds, stream, ids, S, K, E, id_bits, T, shared ? 1 : 0,
-                     bounds, tiles, n_tiles, tok_of, slot_of);
+                     pf_tile_tokens(shared ? S + T : S), bounds, tiles, n_tiles, tok_of, slot_of);
         return kOk;
     }
     launch_timed("pf_hist", k_pf_hist, dim3(nchunk), dim3(256), size_t(E) * 4, stream, ids, S, E, cnt);

