@@ -258,8 +258,9 @@ static DenseWs dense_carve(uint8_t* p0, uint8_t* p, const frt_moe_layer& L, int 
     };
     const int E = L.n_expert, K = L.top_k, n = L.d_model, ff = L.d_ff;
     w.u = reinterpret_cast<float*>(take(size_t(T) * n * 4));
-    w.xq = reinterpret_cast<int8_t*>(take(size_t(T) * n));
-    w.xd = reinterpret_cast<float*>(take(size_t(T) * (n / kQ8) * 4));
+    const size_t Tp = T <= 8 ? size_t(T) : size_t((T + 15) & ~15);   // (from 9 tokens on whole tiles of 16: shexp_code_at)
+    w.xq = reinterpret_cast<int8_t*>(take(Tp * n));
+    w.xd = reinterpret_cast<float*>(take(Tp * (n / kQ8) * 4));
     w.hit_ptr = reinterpret_cast<const uint8_t**>(take(size_t(T) * (K + 1) * 8));
     w.hit_n = reinterpret_cast<int32_t*>(take(size_t(T) * 4));
     w.Y = reinterpret_cast<float*>(take(size_t(T) * (K + 1) * n * 4));

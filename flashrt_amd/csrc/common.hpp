@@ -35,6 +35,17 @@ __host__ __device__ inline int perm256_pos(int K) {
     return 32 * (2 * d + ((k >> 2) & 1)) + 8 * g + 2 * (k & 3) + (k >> 3);
 }
 
+// Q8_0 codes and scales of rows of cols values in the order of the dense shared expert's int8 MFMA operand
+// (shexp.hip k_shexp_mm): per tile of 16 tokens and pair of 32-blocks, lane 16 g + j (g = 0..3) holds codes
+// 8 g .. 8 g + 7 of token j in both blocks; the pair's scales are [2][16]. Offsets of (token t, value k) and
+// (token t, block b).
+__host__ __device__ inline size_t shexp_code_at(int t, int k, int cols) {
+    return ((size_t(t >> 4) * (cols / 64) + (k >> 6)) * 64 + ((k & 31) >> 3) * 16 + (t & 15)) * 16 + ((k >> 5) & 1) * 8 + (k & 7);
+}
+__host__ __device__ inline size_t shexp_scale_at(int t, int b, int cols) {
+    return (size_t(t >> 4) * (cols / 64) + (b >> 1)) * 32 + (b & 1) * 16 + (t & 15);
+}
+
 // C-ABI status codes
 enum Status : int {
     kOk = 0,

@@ -187,7 +187,7 @@ __global__ void k_quant_q8(const float* __restrict__ x, int n_blocks, int8_t* __
 // Same values as k_quant_q8 with xhi / xlo.
 // x [rows][n] -> the pairs [rows][np] (np >= n a multiple of 256; positions n .. np - 1 are zeros),
 // Q8_0 blocks of blk = 32 or 64 values (moe_q2::run's block64). xq / xd (or null; blk 32): the same
-// codes int8 [rows][n] and scales [rows][n / 32].
+// codes and scales in the dense shared expert's order (shexp_code_at, shexp_scale_at).
 struct PairsOut {
     _Float16 *xhi, *xlo;
     int8_t* xq;
@@ -219,8 +219,8 @@ __device__ __forceinline__ void quant_stretch(const float (&v)[4], int row, int 
     }
     const int e = 256 * col + 4 * lane;
     if (o.xq && e < n) {
-        *reinterpret_cast<uint32_t*>(o.xq + size_t(row) * n + e) = codes;
-        if (lane % 8 == 0) o.xd[size_t(row) * (n / kQ8) + e / kQ8] = dr;
+        *reinterpret_cast<uint32_t*>(o.xq + shexp_code_at(row, e, n)) = codes;
+        if (lane % 8 == 0) o.xd[shexp_scale_at(row, e / kQ8, n)] = dr;
     }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0xC07F);   // this wave's LDS writes are done (lgkmcnt(0))

@@ -195,16 +195,20 @@ __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ 
 // its four waves split K in quarters and add their sums in LDS as (q0 + q1) + (q2 + q3), so that a
 // chunk of a few hundred tokens still has several waves per SIMD and no wave runs a long serial K loop.
 // Operands go straight from global memory (each weight row is read by one wave; the activations come
-// from L2) into registers, one K-step ahead; no LDS and no barrier in the K loop.
+// from L2) into registers, one K-step ahead; no LDS and no barrier in the K loop. The activations are kept in
+// the MFMA's own order, a 16-token tile's K-step as 64 lanes x 16 bytes, so that a load's four consecutive
+// lanes read 64 bytes: the L1 takes a clock per 64-byte piece, and in rows (16 tokens x 64 bytes, another
+// token in every lane) a 1 KB load takes 64 clocks instead of 16. The weights stay in the file's rows.
+//   bf16 planes [3][tiles][K / 32][64 lanes][8]: lane 16 g + j holds K 8 g .. 8 g + 7 of token j.
+//   Q8_0 codes [tiles][K / 64][64 lanes][16]: lane 16 g + j holds codes 8 g .. of both blocks of the pair;
+//   scales [tiles][K / 64][2][16].
 //   F32, F16, BF16 weights: the fp32 activations are split exactly into three bf16 planes
 //     (k_split3: 8 + 8 + 8 significant bits by truncation), the weights into one (BF16), two (F16) or
 //     three (F32), and every pair of parts is one v_mfma_f32_16x16x32_bf16 into one fp32 accumulator:
 //     exact products, fp32 sums, as the fmaf chains of k_shexp_mv.
 //   Q8_0 weights: v_mfma_i32_16x16x32_i8 per 32-block, an exact integer dot, then + float(s) * (d_w d_a),
 //     the terms of k_shexp_mv.
-// What bounds it: the L1 reads of the operands (six activation fragments and four weight fragments of
-// 1 KB per 24 matrix instructions), then the matrix cores. Measured (n = 2560, ff = 640; k_shexp_mv
-// before): see kShMmMinT.
+// What bounds it: the L1 reads of the weights (64 clocks per 1 KB), then the matrix cores.
 typedef short bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16v __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -226,16 +230,25 @@ __device__ __forceinline__ void split3(float v, uint32_t& hi, uint32_t& mid, uin
 // the upper halves of two floats' bits as one dword (a below b)
 __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
 
-// planes [3][count] bf16 of count floats (a multiple of 8)
-__global__ void __launch_bounds__(256) k_split3(const float* __restrict__ x, size_t count, uint16_t* __restrict__ planes) {
-    const size_t i = (size_t(blockIdx.x) * 256 + threadIdx.x) * 8;
-    if (i >= count) return;
+// element offset of (token t, value k) in a bf16 plane of rows of cols; planes are up16(T) * cols apart
+__host__ __device__ __forceinline__ size_t plane_at(int t, int k, int cols) {
+    return ((size_t(t >> 4) * (cols / 32) + (k >> 5)) * 64 + ((k & 31) >> 3) * 16 + (t & 15)) * 8 + (k & 7);
+}
+__host__ __device__ __forceinline__ size_t up16(int t) { return size_t((t + 15) & ~15); }
+
+// the planes of x [T][n]: eight values per thread (tokens past T in the last tile are left as they are: their
+// columns of the products are never stored)
+__global__ void __launch_bounds__(256) k_split3(const float* __restrict__ xr, int T, int n, uint16_t* __restrict__ planes) {
+    const size_t e = (size_t(blockIdx.x) * 256 + threadIdx.x) * 8;
+    if (e >= size_t(T) * n) return;
+    const float* x = xr + e;
+    const size_t i = plane_at(int(e / n), int(e % n), n), count = up16(T) * n;
     uint32_t w[3][4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         uint32_t a[3], b[3];
-        split3(x[i + 2 * q], a[0], a[1], a[2]);
-        split3(x[i + 2 * q + 1], b[0], b[1], b[2]);
+        split3(x[2 * q], a[0], a[1], a[2]);
+        split3(x[2 * q + 1], b[0], b[1], b[2]);
 #pragma unroll
         for (int p = 0; p < 3; ++p) w[p][q] = pack_hi(a[p], b[p]);
     }
@@ -276,8 +289,8 @@ struct ShDense {
     }
 };
 
-// out (DUAL): dense types the three planes [3][T][rows] of h = silu(gate) * up, Q8_0 its codes hq [T][rows]
-// and scales hd [T][rows / 32]; else of [T][rows] fp32. aq / ad or ap (planes [3][T][cols]): the input.
+// out (DUAL): dense types the planes of h = silu(gate) * up, Q8_0 its codes hq and scales hd (both as the
+// input's); else of [T][rows] fp32. aq / ad or ap (planes): the input.
 template <int TYPE, bool DUAL, int NC>
 __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1, const uint8_t* __restrict__ W2, int rows,
                                                   int cols, const uint16_t* __restrict__ ap, const int8_t* __restrict__ aq,
@@ -290,9 +303,9 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lg = lane >> 4;
     const int t0 = blockIdx.y * 16 * NC;
     const int r0 = blockIdx.x * (DUAL ? 32 : 64);
-    int tok[NC];
+    size_t tile[NC];   // token tiles; past the end the last again, not written
 #pragma unroll
-    for (int c = 0; c < NC; ++c) tok[c] = min(t0 + 16 * c + li, T - 1);   // past the end: the last token again, not written
+    for (int c = 0; c < NC; ++c) tile[c] = size_t(min(t0 / 16 + c, (T - 1) / 16));
     floatx4 acc[4][NC];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -309,8 +322,8 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
             row[i] = DUAL ? (i < 2 ? W1 : W2) + size_t(r0 + 16 * (i & 1) + li) * rb : W1 + size_t(r0 + 16 * i + li) * rb;
         struct Step {
             uint32_t a[4][5];
-            uint2 b[NC][2];
-            float2 d[NC];
+            uint4 b[NC];
+            float d[NC][2];
         };
         auto load = [&](int st, Step& s) {
 #pragma unroll
@@ -323,10 +336,10 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
             }
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
-                const int8_t* x = aq + size_t(tok[c]) * cols + st * 64 + 8 * lg;
-                s.b[c][0] = *reinterpret_cast<const uint2*>(x);
-                s.b[c][1] = *reinterpret_cast<const uint2*>(x + 32);
-                s.d[c] = *reinterpret_cast<const float2*>(ad + size_t(tok[c]) * (cols / kQ8) + 2 * st);
+                const size_t at = tile[c] * steps + st;
+                s.b[c] = *reinterpret_cast<const uint4*>(aq + (at * 64 + lane) * 16);
+                s.d[c][0] = ad[at * 32 + li];
+                s.d[c][1] = ad[at * 32 + 16 + li];
             }
         };
         auto mac = [&](const Step& s) {
@@ -352,12 +365,12 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
 #pragma unroll
                 for (int c = 0; c < NC; ++c) {
                     const intx4 z = {0, 0, 0, 0};
-                    const intx4 v0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a0, __builtin_bit_cast(long, s.b[c][0]), z, 0, 0, 0);
-                    const intx4 v1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a1, __builtin_bit_cast(long, s.b[c][1]), z, 0, 0, 0);
+                    const intx4 v0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a0, __builtin_bit_cast(long, make_uint2(s.b[c].x, s.b[c].y)), z, 0, 0, 0);
+                    const intx4 v1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a1, __builtin_bit_cast(long, make_uint2(s.b[c].z, s.b[c].w)), z, 0, 0, 0);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        acc[i][c][r] = fmaf(float(v0[r]), w0[r] * s.d[c].x, acc[i][c][r]);
-                        acc[i][c][r] = fmaf(float(v1[r]), w1[r] * s.d[c].y, acc[i][c][r]);
+                        acc[i][c][r] = fmaf(float(v0[r]), w0[r] * s.d[c][0], acc[i][c][r]);
+                        acc[i][c][r] = fmaf(float(v1[r]), w1[r] * s.d[c][1], acc[i][c][r]);
                     }
                 }
             }
@@ -381,10 +394,10 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
         for (int i = 0; i < 4; ++i)
             row[i] = (DUAL ? (i < 2 ? W1 : W2) + size_t(r0 + 16 * (i & 1) + li) * cols * es
                            : W1 + size_t(r0 + 16 * i + li) * cols * es) + 8 * lg * es;
-        const size_t plane = size_t(T) * cols;
+        const size_t plane = up16(T) * cols;
         const uint16_t* xp[NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) xp[c] = ap + size_t(tok[c]) * cols + 8 * lg;
+        for (int c = 0; c < NC; ++c) xp[c] = ap + (tile[c] * (cols / 32) * 64 + lane) * 8;
         struct Step {
             uint32_t a[4][D::words];
             bf16x8 b[NC][3];
@@ -403,7 +416,7 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int p = 0; p < 3; ++p) s.b[c][p] = *reinterpret_cast<const bf16x8*>(xp[c] + p * plane + st * 32);
+                for (int p = 0; p < 3; ++p) s.b[c][p] = *reinterpret_cast<const bf16x8*>(xp[c] + p * plane + size_t(st) * 512);
         };
         auto mac = [&](const Step& s) {
 #pragma unroll
@@ -470,9 +483,9 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
                 uint32_t q = 0;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) q |= uint32_t(uint8_t(int8_t(q8_code(h[i][r], id)))) << (8 * r);
-                *reinterpret_cast<uint32_t*>(hq + size_t(t) * rows + r0 + 16 * i + 4 * lg) = q;
+                *reinterpret_cast<uint32_t*>(hq + shexp_code_at(t, r0 + 16 * i + 4 * lg, rows)) = q;
             }
-            if (lg == 0) hd[size_t(t) * (rows / kQ8) + r0 / 32] = f16_round(d);
+            if (lg == 0) hd[shexp_scale_at(t, r0 / 32, rows)] = f16_round(d);
         }
     } else if (t < T) {
 #pragma unroll
@@ -482,7 +495,7 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
             for (int r = 0; r < 4; ++r) split3(h[i][r], p[r][0], p[r][1], p[r][2]);
 #pragma unroll
             for (int q = 0; q < 3; ++q)
-                *reinterpret_cast<uint2*>(op + (size_t(q) * T + t) * rows + r0 + 16 * i + 4 * lg) =
+                *reinterpret_cast<uint2*>(op + q * up16(T) * rows + plane_at(t, r0 + 16 * i + 4 * lg, rows)) =
                     make_uint2(pack_hi(p[0][q], p[1][q]), pack_hi(p[2][q], p[3][q]));
         }
     }
@@ -591,7 +604,7 @@ constexpr int kShMmMinT = 9;
 size_t shexp_ws_bytes(int T, int n, int ffs) {
     const size_t mv = up256(size_t(T) * ffs * 4);
     if (T < kShMmMinT) return mv;
-    const size_t mm = up256(size_t(T) * n * 6) + up256(size_t(T) * ffs * 6);   // the bf16 planes of x and h
+    const size_t mm = up256(up16(T) * n * 6) + up256(up16(T) * ffs * 6);   // the bf16 planes of x and h
     return mv > mm ? mv : mm;
 }
 
@@ -613,14 +626,13 @@ static int shexp_run_mm(const void* g, const void* u, const void* d, int n, int 
     uint8_t* p = static_cast<uint8_t*>(ws);
     if (TYPE == FRT_GGML_Q8_0) {
         int8_t* hq = reinterpret_cast<int8_t*>(p);
-        float* hd = reinterpret_cast<float*>(p + up256(size_t(T) * ffs));
+        float* hd = reinterpret_cast<float*>(p + up256(up16(T) * ffs));
         shexp_mm<TYPE, true>(wg, wu, ffs, n, nullptr, xq, xd, T, nullptr, nullptr, hq, hd, stream);
         shexp_mm<TYPE, false>(wd, nullptr, n, ffs, nullptr, hq, hd, T, sh, nullptr, nullptr, nullptr, stream);
     } else {
         uint16_t* xp = reinterpret_cast<uint16_t*>(p);
-        uint16_t* hp = reinterpret_cast<uint16_t*>(p + up256(size_t(T) * n * 6));
-        const size_t count = size_t(T) * n;
-        k_split3<<<unsigned((count / 8 + 255) / 256), 256, 0, stream>>>(x, count, xp);
+        uint16_t* hp = reinterpret_cast<uint16_t*>(p + up256(up16(T) * n * 6));
+        k_split3<<<unsigned((size_t(T) * n / 8 + 255) / 256), 256, 0, stream>>>(x, T, n, xp);
         shexp_mm<TYPE, true>(wg, wu, ffs, n, xp, nullptr, nullptr, T, nullptr, hp, nullptr, nullptr, stream);
         shexp_mm<TYPE, false>(wd, nullptr, n, ffs, hp, nullptr, nullptr, T, sh, nullptr, nullptr, nullptr, stream);
     }
@@ -629,7 +641,8 @@ static int shexp_run_mm(const void* g, const void* u, const void* d, int n, int 
 }
 
 // sh (rows of n, sh_ld apart; n from kShMmMinT tokens on) = the shared expert of type `type` on x [T][n];
-// xq / xd: x's Q8_0 (Q8_0 type only). ws: shexp_ws_bytes.
+// xq / xd: x's Q8_0 (Q8_0 type only; from kShMmMinT tokens on in the order of shexp_code_at and
+// shexp_scale_at, for whole tiles of 16 tokens). ws: shexp_ws_bytes.
 int shexp_run(int type, const void* g, const void* u, const void* d, int n, int ffs, const float* x, const int8_t* xq,
               const float* xd, int T, float* sh, size_t sh_ld, void* ws, hipStream_t stream) {
     if (!shexp_type_ok(type)) return set_error(kErrShape, "shared expert: ggml type %d (F32, F16, BF16 or Q8_0)", type);
