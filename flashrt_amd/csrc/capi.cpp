@@ -216,7 +216,8 @@ static bool window_path(const frt_moe_layer& L, int T) {
 
 // ---- the slot path of a layer: the routed experts as per-slot outputs (moe_hits for windows of up to 8
 // tokens, moe_q2::run beyond), the shared expert, then the slot combine. Taken by a layer whose shared
-// expert is given as dense GGUF tensors (frt_moe_layer.shared_dense; shexp.hip), and by windows whose
+// expert is given as dense GGUF tensors (frt_moe_layer.shared_dense; shexp.hip) unless dense_window takes
+// the call, and by windows whose
 // shape is outside the templated decode kernels (n a multiple of 512, ff a multiple of 64 up to 4096:
 // the reference's moe_hits envelope), where the Q2_0 shared expert is moe_hits slot K.
 struct DenseWs {

@@ -1,18 +1,20 @@
 // Prefill MoE: routed (token, slot) pairs sorted by expert, then grouped GEMMs on fp16 MFMA
 // (kernels/cuda/moe_q2.cu:514-548 is the reference's int8 counterpart).
 //
-// Dispatch (moe_q2.cu:83-168 semantics: a stable sort of slots s = t*K + k by ids[s]):
-//   k_pf_hist   per chunk of 256 slots, an LDS histogram of experts (integer atomics only)
-//   k_pf_scan   one workgroup: per-expert column prefix over chunks, bounds, the tile list
-//   k_pf_place  one wave per chunk walks its slots in order, 64 at a time; each lane's rank among
+// Dispatch (moe_q2.cu:83-168 semantics: a stable sort of slots s = t*K + k by ids[s]). Up to 4096 slots
+// and 1024 experts k_pf_dispatch1, one workgroup; beyond:
+//   k_pf_hist     per chunk of 256 slots, an LDS histogram of experts (integer atomics only)
+//   k_pf_colscan  per expert, its column's prefix over the chunks
+//   k_pf_scan     one workgroup: bounds, the tile list
+//   k_pf_place    one wave per chunk walks its slots in order, 64 at a time; each lane's rank among
 //               equal experts in the batch comes from ballots (a wave64 match-any), so the
 //               placement is stable and needs no atomics.
 //   The shared expert, when present, is group E holding every token in order (rows T*K + t, written
 //   by the workgroups of k_pf_place past the chunks).
 //
 // GEMMs (k_pf_gemm, below): Q2_0 weights dequantized exactly to fp16 in registers, activations
-// as exact fp16 (hi, lo) pairs (gate/up) or fp16 (down), fp32 accumulation on MFMA; tiles of 64
-// tokens of one group; the gate/up epilogue applies SwiGLU and the Q8_0 quantization of h.
+// as exact fp16 (hi, lo) pairs (gate/up) or fp16 (down), fp32 accumulation on MFMA; tiles of up to 16
+// or of up to 64 tokens of one group; the gate/up epilogue applies SwiGLU and the Q8_0 quantization of h.
 //   k_pf_combine out[t] = sum_k (in expert order) w * yd[t*K+k] + yd[shared t] * sigmoid(gate)
 #include "common.hpp"
 

@@ -10,9 +10,10 @@
 //     h quantized per 32 as the CPU path does, q8_0 . q8_0 per block as an exact integer dot, then
 //     scaled by d_w d_a); the other types take the fp32 activations.
 //     Taken up to 8 tokens; more go to k_shexp_mm, the same products on the matrix cores.
-//   - the layer with such a shared expert: router logits -> route_topk -> the routed experts as
-//     per-slot outputs (moe_hits for windows of up to 8 tokens, moe_q2::run for prefill chunks) ->
-//     the shared expert -> k_slot_combine (the routed slots in ascending expert id, then the shared
+//   - the layer with such a shared expert: windows of up to 8 tokens of a shape that the decode kernels
+//     are templated for run the window kernels with the shared expert's outputs in slot K; else router
+//     logits -> route_topk -> the routed experts as per-slot outputs (moe_hits for windows of up to 8
+//     tokens, moe_q2::run for prefill chunks) -> the shared expert -> k_slot_combine (the routed slots in ascending expert id, then the shared
 //     expert times sigmoid(gate), then the residual: moe_cpu.cpp:63-80 and moe_ref.cu:90-97).
 #include "common.hpp"
 #include "../../include/flashrt_moe.h"
@@ -208,7 +209,9 @@ __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ 
 //     exact products, fp32 sums, as the fmaf chains of k_shexp_mv.
 //   Q8_0 weights: v_mfma_i32_16x16x32_i8 per 32-block, an exact integer dot, then + float(s) * (d_w d_a),
 //     the terms of k_shexp_mv.
-// What bounds it: the L1 reads of the weights (64 clocks per 1 KB), then the matrix cores.
+// What bounds it: latency at a few hundred tokens. The weights loaded four lanes to a row's 64 bytes and
+// turned through the wave's LDS instead (a quarter of the L1's clocks) changed nothing: a layer of 200 tokens
+// 224 us, of 1024 tokens 449-471 us both ways.
 typedef short bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16v __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));

@@ -146,8 +146,8 @@ int frt_moe_dispatch(void* stream, const int32_t* ids, int T, int K, int E, int3
  * yd [T*K][n]: slot t*K + k gets down(silu(gate x_t) * up x_t) of expert ids[t*K + k], expert e's
  * blob at experts + e * stride. yd_bf16 selects bf16 output. block64: x and h are quantized in Q8
  * blocks of 64 values instead of the CPU path's 32 (moe_q2.cu's AB = 64). Shapes: n and ff multiples
- * of 128 (moe_q2.cu:516-517), ff at most 4096; ff above 1024 takes fp32 yd only (the down GEMM adds
- * up chunks of 1024 in it). FRT_ERR_SHAPE otherwise. */
+ * of 128 (moe_q2.cu:516-517), ff at most 4096; ff above 1024 takes fp32 yd only. FRT_ERR_SHAPE
+ * otherwise. */
 size_t frt_moe_q2_workspace_bytes(int T, int K, int n, int ff, int E);
 int frt_moe_q2_run(const uint8_t* experts, size_t stride, int E, int n, int ff, const float* x, const int32_t* ids,
                    int T, int K, void* yd, void* ws, size_t ws_bytes, void* stream, int block64, int yd_bf16);
@@ -195,9 +195,10 @@ typedef struct frt_moe_layer {
      * linear() in whatever type the file ships). shared_dense = 0 (the default): `shared` is used.
      * shared_type: FRT_GGML_F32, FRT_GGML_F16, FRT_GGML_BF16 or FRT_GGML_Q8_0 (Q8_0 weights take the
      * input and h as Q8_0 activations, per-block integer dots; the others fp32 activations).
-     * shared_ff a multiple of 64, at most 4096. Such a layer runs router -> route_topk -> the routed
-     * experts as per-slot outputs (moe_hits up to 8 tokens, moe_q2::run beyond) -> the shared expert
-     * -> the combine; the persistent single-token kernels take only the Q2_0 blob. */
+     * shared_ff a multiple of 64, at most 4096. Such a layer runs windows of up to 8 tokens on the
+     * window kernels where the shape is one of theirs; else router -> route_topk -> the routed experts
+     * as per-slot outputs (moe_hits up to 8 tokens, moe_q2::run beyond) -> the shared expert -> the
+     * combine. The persistent single-token kernels take only the Q2_0 blob. */
     int shared_dense;
     int shared_type;
     int shared_ff;
