@@ -13,10 +13,13 @@
 //   - the layer with such a shared expert: windows of up to 8 tokens of a shape that the decode kernels
 //     are templated for run the window kernels with the shared expert's outputs in slot K; else router
 //     logits -> route_topk -> the routed experts as per-slot outputs (moe_hits for windows of up to 8
-//     tokens, moe_q2::run for prefill chunks) -> the shared expert -> k_slot_combine (the routed slots in ascending expert id, then the shared
-//     expert times sigmoid(gate), then the residual: moe_cpu.cpp:63-80 and moe_ref.cu:90-97).
+//     tokens, moe_q2::run for prefill chunks) -> the shared expert -> k_slot_combine (the routed slots
+//     in ascending expert id, then the shared expert times sigmoid(gate), then the residual:
+//     moe_cpu.cpp:63-80 and moe_ref.cu:90-97).
 #include "common.hpp"
 #include "../../include/flashrt_moe.h"
+
+#include <type_traits>
 
 namespace frt {
 
@@ -209,6 +212,10 @@ __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ 
 //     exact products, fp32 sums, as the fmaf chains of k_shexp_mv.
 //   Q8_0 weights: v_mfma_i32_16x16x32_i8 per 32-block, an exact integer dot, then + float(s) * (d_w d_a),
 //     the terms of k_shexp_mv.
+// Precision: the products of the leading parts and the small ones have sums of their own, and the leading
+// ones two (even and odd K-steps; Q8_0: a pair's two blocks), added at the end. With one sum for all, every
+// small product rounds the full sum: rms error against float64 2.5e-7 (k_shexp_mv) -> 4.2e-7 (BF16), 6.2e-7
+// (F32) at 2560 / 640; with these 2.0e-7, at no cost (a layer of 200 tokens 224 us, 1024 tokens 469 us both).
 // What bounds it: latency at a few hundred tokens. The weights loaded four lanes to a row's 64 bytes and
 // turned through the wave's LDS instead (a quarter of the L1's clocks) changed nothing: a layer of 200 tokens
 // 224 us, of 1024 tokens 449-471 us both ways.
@@ -309,11 +316,14 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
     size_t tile[NC];   // token tiles; past the end the last again, not written
 #pragma unroll
     for (int c = 0; c < NC; ++c) tile[c] = size_t(min(t0 / 16 + c, (T - 1) / 16));
-    floatx4 acc[4][NC];
+    constexpr int kHi = 2, NA = Q8 ? 2 : kHi + 1;   // sums: see "Precision" above
+    floatx4 acc[NA][4][NC];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int k = 0; k < NA; ++k)
 #pragma unroll
-        for (int c = 0; c < NC; ++c) acc[i][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) acc[k][i][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (Q8) {
         // K-steps of 64: a pair of Q8_0 blocks, 68 bytes of a row. Lane group lg takes codes 8 lg .. 8 lg + 7
         // of each block: bytes 2 + 8 lg (dwords 2 lg .. 2 lg + 2, shifted by two bytes) and 36 + 8 lg.
@@ -372,8 +382,8 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
                     const intx4 v1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a1, __builtin_bit_cast(long, make_uint2(s.b[c].z, s.b[c].w)), z, 0, 0, 0);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        acc[i][c][r] = fmaf(float(v0[r]), w0[r] * s.d[c][0], acc[i][c][r]);
-                        acc[i][c][r] = fmaf(float(v1[r]), w1[r] * s.d[c][1], acc[i][c][r]);
+                        acc[0][i][c][r] = fmaf(float(v0[r]), w0[r] * s.d[c][0], acc[0][i][c][r]);
+                        acc[1][i][c][r] = fmaf(float(v1[r]), w1[r] * s.d[c][1], acc[1][i][c][r]);
                     }
                 }
             }
@@ -421,7 +431,7 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
 #pragma unroll
                 for (int p = 0; p < 3; ++p) s.b[c][p] = *reinterpret_cast<const bf16x8*>(xp[c] + p * plane + size_t(st) * 512);
         };
-        auto mac = [&](const Step& s) {
+        auto mac = [&](const Step& s, auto hi) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 bf16x8 a[D::parts];
@@ -431,27 +441,32 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
 #pragma unroll
                     for (int pa = D::parts - 1; pa >= 0; --pa)   // the small products first
 #pragma unroll
-                        for (int pb = 2; pb >= 0; --pb)
-                            acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16v, a[pa]),
-                                                                                __builtin_bit_cast(bf16v, s.b[c][pb]),
-                                                                                acc[i][c], 0, 0, 0);
+                        for (int pb = 2; pb >= 0; --pb) {
+                            floatx4& t = acc[pa + pb ? kHi : hi][i][c];
+                            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16v, a[pa]),
+                                                                        __builtin_bit_cast(bf16v, s.b[c][pb]), t, 0, 0, 0);
+                        }
             }
         };
         Step a, b;
         if (s0 < s1) load(s0, a);
         for (int st = s0; st < s1; st += 2) {
             load(min(st + 1, s1 - 1), b);
-            mac(a);
+            mac(a, std::integral_constant<int, 0>());
             if (st + 1 < s1) {
                 load(min(st + 2, s1 - 1), a);
-                mac(b);
+                mac(b, std::integral_constant<int, kHi - 1>());
             }
         }
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) part[wave][c][i][lane] = acc[i][c];
+        for (int i = 0; i < 4; ++i) {
+            floatx4 v = acc[0][i][c] + acc[1][i][c];
+            if constexpr (NA > 2) v += acc[2][i][c];
+            part[wave][c][i][lane] = v;
+        }
     __syncthreads();
     if (wave >= NC) return;
     // wave c finishes token column c: lane (token li, rows 16 i + 4 lg + r)
