@@ -262,12 +262,15 @@ static DenseWs dense_carve(uint8_t* p0, uint8_t* p, const frt_moe_layer& L, int 
     const size_t Tp = T <= 8 ? size_t(T) : size_t((T + 15) & ~15);   // (from 9 tokens on whole tiles of 16: shexp_code_at)
     w.xq = reinterpret_cast<int8_t*>(take(Tp * n));
     w.xd = reinterpret_cast<float*>(take(Tp * (n / kQ8) * 4));
-    w.hit_ptr = reinterpret_cast<const uint8_t**>(take(size_t(T) * (K + 1) * 8));
-    w.hit_n = reinterpret_cast<int32_t*>(take(size_t(T) * 4));
-    w.Y = reinterpret_cast<float*>(take(size_t(T) * (K + 1) * n * 4));
-    w.sh = reinterpret_cast<float*>(take(size_t(T) * n * 4));
+    const bool win = dense_window(L, T);
+    if (!win) {   // (the window kernels keep their entries and per-slot outputs, the shared expert's too, in rws)
+        w.hit_ptr = reinterpret_cast<const uint8_t**>(take(size_t(T) * (K + 1) * 8));
+        w.hit_n = reinterpret_cast<int32_t*>(take(size_t(T) * 4));
+        w.Y = reinterpret_cast<float*>(take(size_t(T) * (K + 1) * n * 4));
+        w.sh = reinterpret_cast<float*>(take(size_t(T) * n * 4));
+    }
     w.shws = take(shexp_ws_bytes(T, n, L.shared_ff > 0 ? L.shared_ff : 64));
-    if (dense_window(L, T)) {
+    if (win) {
         w.rws_bytes = dec_window_bytes(T, K, n, ff);
     } else if (dense_small(L, T)) {
         const int S = L.shared_dense ? K : K + 1;

@@ -41,6 +41,27 @@ def test_host_entry_points():
     assert L.frt_moe_dispatch_workspace_bytes(2048, 10, 512) > 0
 
 
+def _layer(E, n, ff, K, dense=None, shared_ff=0, norm=0):
+    """A layer description for the size functions (its pointers are never read)."""
+    d = _lib.FrtMoeLayer(1, 1 << 30, E, 1, 1, 0, 1, n, ff, K, norm)
+    if dense is not None:
+        d.shared_dense, d.shared_type, d.shared_ff = 1, dense, shared_ff
+        d.shared_gate = d.shared_up = d.shared_down = 1
+    return d
+
+
+@pytest.mark.parametrize("n,ff", [(2048, 512), (2560, 640), (4096, 256), (512, 128), (2560, 2048)])
+@pytest.mark.parametrize("K", [1, 10, 15, 31, 32])
+def test_dense_layer_workspace_grows_with_tokens(n, ff, K):
+    """A workspace sized for a longer call of a layer with a dense shared expert holds every shorter one,
+    across the window, slot and grouped paths."""
+    for gtype in (0, 8, 30):
+        for shared_ff in (64, 640, 4096):
+            d = _layer(512, n, ff, K, gtype, shared_ff)
+            b = [_lib.lib().frt_moe_layer_workspace_bytes(C.byref(d), T) for T in range(1, 65)]
+            assert b == sorted(b), (gtype, shared_ff, [T for T in range(1, 64) if b[T - 1] > b[T]])
+
+
 def test_argument_errors_before_device_work():
     """Shape and null-pointer errors are reported with a status and a message, as the reference's
     std::runtime_error would be, without touching a device."""
