@@ -24,28 +24,31 @@ __device__ __forceinline__ void quant32(float v, int j, int8_t* q, float* d) {
     if (j == 0) *d = f16_round(dd);
 }
 
-// ---- router: grid (ceil(rows / W), ceil(T / tok_per_wg)), W = wg_rows router rows per workgroup (2 for
-// decode windows, so that the 4 MiB of router rows spread over twice as many CUs), blockDim.x / 64 / W
-// waves each, which share the row's tokens (two waves from 4 tokens on: staging the tokens, their RMS
-// scales and their dot products are serial per wave, 11.6 us at 8 tokens with one).
+// ---- router: grid (ceil(rows / W), ceil(T / tok_per_wg)), W router rows per workgroup (2 for decode
+// windows, so that the 4 MiB of router rows spread over twice as many CUs), one wave each, or with PAIR
+// two waves, which share the row's tokens: staging the tokens, their RMS scales and their dot products are
+// serial per wave, 11.6 us at 8 tokens of 2048 with one. PAIR is for windows of 4 tokens and 3072 values
+// on. Below, the second wave and the eight loads in flight only add instructions to a kernel of one round
+// of latency (one wave / two: 512 values 3.3 / 3.7 us at 1 token, 3.7 / 4.0 at 4; 1024 values 4.2 / 4.2 at 4,
+// 2048 values 5.1 / 5.4 at 3); so they do in the token tiles of a longer call (4096 values, 8 tokens 10.9 / 11.5).
 // Rows 0..E-1 are the router (bias optional); row E (when gate_w) is the shared expert's gate.
 // x tiles of TT tokens are staged in LDS with each 64-chain padded by one float (conflict-free).
 // norm: the layer input is u = x * r, r the canonical RMS scale of the token (topk.hpp); u_i is
 // formed as a rounded product before its fma, exactly as the CPU oracle does.
 // xq/xd (optional, T <= tok_per_wg): Q8_0 of the experts' input (u when norm, else x), one
 // 32-value block per half-wave spread over the workgroups of grid row 0.
-template <int L>
+template <int L, bool PAIR>
 __global__ void __launch_bounds__(256) k_router(const float* __restrict__ x, int T, const float* __restrict__ W,
                                                 const float* __restrict__ bias, const float* __restrict__ gate_w,
                                                 int E, float* __restrict__ logits, float* __restrict__ gate, int TT,
                                                 int tok_per_wg, int norm, int8_t* __restrict__ xq,
-                                                float* __restrict__ xd, int wg_rows) {
+                                                float* __restrict__ xd) {
     extern __shared__ float xs[];   // [TT][64][L + 1]
     __shared__ float s_r[64];
     const int n = 64 * L;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int row = blockIdx.x * wg_rows + wave % wg_rows;
-    const int tg = wave / wg_rows, ts = int(blockDim.x >> 6) / wg_rows;   // this wave's tokens: tg, tg + ts, ..
+    const int row = PAIR ? blockIdx.x * 2 + (wave & 1) : blockIdx.x * (blockDim.x >> 6) + wave;
+    const int tg = PAIR ? wave >> 1 : 0, ts = PAIR ? 2 : 1;   // this wave's tokens: tg, tg + ts, ..
     const bool is_gate = row == E;
     const bool live = row < E || (is_gate && gate_w);
     const float* w = is_gate ? gate_w : W + size_t(row < E ? row : 0) * n;
@@ -70,20 +73,21 @@ __global__ void __launch_bounds__(256) k_router(const float* __restrict__ x, int
         // the previous tile's LDS reads are done (none before the first tile: its x loads then
         // issue right behind the row loads, without a fence waiting for those)
         if (t0 != t_begin) __syncthreads();
-        // x tile into LDS, 8 loads per thread in flight before their LDS writes (clamped indices, no
+        // x tile into LDS, NV loads per thread in flight before their LDS writes (clamped indices, no
         // branches, which would let the compiler sink each load to its write: past the end a thread
         // rewrites the last element with its own value)
         const int nx = tn * (n / 4);
-        for (int i0 = threadIdx.x; i0 < nx; i0 += 8 * int(blockDim.x)) {
-            float4 v[8];
+        constexpr int NV = PAIR ? 8 : 4;
+        for (int i0 = threadIdx.x; i0 < nx; i0 += NV * int(blockDim.x)) {
+            float4 v[NV];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < NV; ++u) {
                 const int i = min(i0 + u * int(blockDim.x), nx - 1);
                 const int t = i / (n / 4), k = (i % (n / 4)) * 4;
                 v[u] = *reinterpret_cast<const float4*>(x + size_t(t0 + t) * n + k);
             }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < NV; ++u) {
                 const int i = min(i0 + u * int(blockDim.x), nx - 1);
                 const int t = i / (n / 4), k = (i % (n / 4)) * 4;
                 float* dst = xs + (t * 64 + k / L) * (L + 1) + k % L;   // L % 4 == 0: one chain
@@ -349,16 +353,17 @@ int router_logits(const float* x, int T, const float* W, const float* bias, cons
     const int tok_per_wg = T <= TT ? T : 64;
     if (xq && T > TT) return set_error(kErrShape, "router: fused quantization needs T <= %d", TT);
     const int wg_rows = T <= TT ? 2 : 4;   // decode: 2 rows per workgroup; token tiles: 4
-    const int waves = T <= TT && T >= 4 ? 2 * wg_rows : wg_rows;
+    const bool pair = T <= TT && T >= 4 && T * n >= 3072;   // (two waves per row: k_router)
     dim3 grid((rows + wg_rows - 1) / wg_rows, (T + tok_per_wg - 1) / tok_per_wg);
 #define FRT_ROUTER_L(LL)                                                                                         \
-    case LL:                                                                                                     \
+    case LL: {                                                                                                   \
+        auto* k = pair ? k_router<LL, true> : k_router<LL, false>;                                               \
         if (smem > 65536)                                                                                        \
-            FRT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_router<LL>),                            \
+            FRT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k),                                        \
                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(smem)));                 \
-        launch_timed("router_quant", k_router<LL>, grid, dim3(64 * waves), smem, stream, x, T, W, bias, gate_w, E,   \
-                     logits, gate, TT, tok_per_wg, norm, xq, xd, wg_rows);                                           \
-        break;
+        launch_timed("router_quant", k, grid, dim3(64 * wg_rows * (pair ? 2 : 1)), smem, stream, x, T, W, bias, gate_w, E, \
+                     logits, gate, TT, tok_per_wg, norm, xq, xd);                                                    \
+    } break;
     switch (L) {
         FRT_ROUTER_L(8) FRT_ROUTER_L(16) FRT_ROUTER_L(24) FRT_ROUTER_L(32) FRT_ROUTER_L(40) FRT_ROUTER_L(48)
         FRT_ROUTER_L(56) FRT_ROUTER_L(64)

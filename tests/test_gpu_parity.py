@@ -133,6 +133,24 @@ def test_router_logits_bit_exact(F, T, n, with_bias):
     assert np.array_equal(gt.cpu().numpy(), gref)
 
 
+@pytest.mark.parametrize("n", [512, 1024, 4096])
+@pytest.mark.parametrize("T", [1, 3, 4, 5, 6, 8, 16, 17])
+def test_router_logits_small_calls(F, T, n):
+    """Either side of the rule that gives a router row two waves (from 4 tokens and 3072 values on, within
+    one token tile: 16 tokens, 5 at n = 4096): logits and gate bit for bit the oracle's, on an odd row count."""
+    E = 33
+    rng = np.random.default_rng(T * 11 + n)
+    x = rng.standard_normal((T, n)).astype(np.float32)
+    W = (rng.standard_normal((E, n)) * 0.02).astype(np.float32)
+    g = (rng.standard_normal(n) * 0.02).astype(np.float32)
+    lg = torch.full((T, E), float("nan"), dtype=torch.float32, device="cuda")
+    gt = torch.full((T,), float("nan"), dtype=torch.float32, device="cuda")
+    F.router_logits(dev(x), T, dev(W), E, n, lg, gate_w=dev(g), gate=gt)
+    torch.cuda.synchronize()
+    assert np.array_equal(lg.cpu().numpy(), O.router_logits(x, W, None))
+    assert np.array_equal(gt.cpu().numpy(), np.array([O.dot_canon(g, x[t]) for t in range(T)], np.float32))
+
+
 @pytest.mark.parametrize("T,n,with_bias", [(300, 2048, True), (2048, 2048, False), (70, 2560, True), (64, 1024, False),
                                             (100, 512, True), (65, 1536, False), (40, 3584, True)])
 def test_router_logits_gemm_bit_exact(F, T, n, with_bias):
