@@ -94,15 +94,32 @@ __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int t0 = blockIdx.y * kShTT, tn = min(kShTT, T - t0);
     // the token tile's activations into LDS
-    if (Q8 && !DUAL) {   // h to Q8_0, a 32-value block per half wave (as k_quant_q8)
-        const int nb = tn * cols / kQ8, j = tid & 31;
-        for (int i0 = 0; i0 < nb; i0 += kShNT / 32) {
-            const int i = i0 + (tid >> 5);
-            const float v = i < nb ? af[size_t(t0) * cols + size_t(i) * kQ8 + j] : 0.0f;
-            const float d = q8_scale(half_max(fabsf(v)));
-            if (i < nb) {
-                s_aq[i * kQ8 + j] = int8_t(q8_code(v, q8_inv(d)));
-                if (j == 0) s_ad[i] = f16_round(d);
+    if (Q8 && !DUAL) {
+        // h to Q8_0 (the values of k_quant_q8): eight lanes to a block of 32, four values each, four loads in
+        // flight. Every workgroup does this for itself, so it has to be short: a block per half wave and a
+        // load at a time took 28 us of a call at 4 tokens of 512 with a shared expert of 4096 (84 us; a
+        // launch of its own before this one 56 us; this 55 us).
+        const float4* src = reinterpret_cast<const float4*>(af + size_t(t0) * cols);
+        const int nv = tn * cols / 4;   // (a multiple of 16: a block's lanes are all within it or all past it)
+        for (int i0 = 0; i0 < nv; i0 += 4 * kShNT) {
+            float4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = src[min(i0 + u * kShNT + tid, nv - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (i0 + u * kShNT >= nv) break;   // (uniform)
+                const int i = i0 + u * kShNT + tid;
+                float am = fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w)));
+                am = fmaxf(am, __shfl_xor(am, 1));
+                am = fmaxf(am, __shfl_xor(am, 2));
+                am = fmaxf(am, __shfl_xor(am, 4));
+                const float d = q8_scale(am), id = q8_inv(d);
+                const int q[4] = {q8_code(v[u].x, id), q8_code(v[u].y, id), q8_code(v[u].z, id), q8_code(v[u].w, id)};
+                if (i < nv) {
+                    reinterpret_cast<uint32_t*>(s_aq)[i] = uint32_t(uint8_t(int8_t(q[0]))) | uint32_t(uint8_t(int8_t(q[1]))) << 8 |
+                                                           uint32_t(uint8_t(int8_t(q[2]))) << 16 | uint32_t(uint8_t(int8_t(q[3]))) << 24;
+                    if (i % 8 == 0) s_ad[i / 8] = f16_round(d);
+                }
             }
         }
     } else if (Q8) {

@@ -1357,6 +1357,56 @@ def test_layer_dense_shared_expert(F, gtype, T):
     assert err <= H.OUT_REL
 
 
+def _shared_only(F, gtype, T, n, ffs, seed, ff=128, E=16, K=2, weights=None):
+    """A layer whose routed experts have zero scales, so that it gives sigmoid(gate) * shared: its output,
+    and the same in float64 on the weights' exact values (Q8_0: activations and h rounded to codes).
+    weights: a function that changes the float64 gate / up / down matrices' raw bytes in place."""
+    rng = np.random.default_rng(seed)
+    eb = F.expert_bytes(n, ff)
+    stride = (eb + 4095) // 4096 * 4096
+    arena = torch.zeros(E * stride, dtype=torch.uint8, device="cuda")
+    router = torch.from_numpy((rng.standard_normal((E, n)) * 0.02).astype(np.float32)).cuda()
+    gate = (rng.standard_normal(n) * 0.02).astype(np.float32)
+    raw = [H.dense_tensor(gtype, r, c, rng) for r, c in ((ffs, n), (ffs, n), (n, ffs))]
+    if weights is not None:
+        weights(raw)
+    dv = [torch.from_numpy(a).cuda() for a in raw]
+    gate_d = torch.from_numpy(gate).cuda()
+    ml = F.MoeLayer(arena.data_ptr(), stride, E, 0, router, gate_d, n, ff, K)
+    ml.set_shared_dense(gtype, *dv, ffs)
+    x = rng.standard_normal((T, n)).astype(np.float32)
+    out = torch.full((T, n), float("nan"), dtype=torch.float32, device="cuda")
+    ml.forward(torch.from_numpy(x).cuda(), out, T=T)
+    torch.cuda.synchronize()
+    g, u, d = (H.dense_values(gtype, a, r, c) for a, (r, c) in zip(raw, ((ffs, n), (ffs, n), (n, ffs))))
+    xx = x.astype(np.float64)
+    if gtype == H.GGML_Q8_0:
+        q, s = O.quantize_q8(x)
+        xx = (q.reshape(T, n // 32, 32) * s.reshape(T, n // 32, 1).astype(np.float64)).reshape(T, n)
+    with np.errstate(all="ignore"):
+        gg = xx @ g.T
+        h = gg / (1 + np.exp(-gg)) * (xx @ u.T)
+        if gtype == H.GGML_Q8_0:
+            q, s = O.quantize_q8(h.astype(np.float32))
+            h = (q.reshape(T, ffs // 32, 32) * s.reshape(T, ffs // 32, 1).astype(np.float64)).reshape(T, ffs)
+        ref = (h @ d.T) / (1 + np.exp(-(x.astype(np.float64) @ gate)))[:, None]
+    return out.cpu().numpy(), ref
+
+
+@pytest.mark.parametrize("n,ff", [(512, 128), (1024, 256)])
+@pytest.mark.parametrize("ffs", [64, 320, 2112, 4096])
+@pytest.mark.parametrize("T", [1, 4, 5, 8])
+def test_shared_expert_q8_windows(F, T, ffs, n, ff):
+    """A Q8_0 shared expert of a window, whose down product quantizes h for itself: h of two blocks up to
+    4096 values (part of one staging batch up to several, whole ones and a rest), through the slot path
+    (512 / 128) and the window kernels (1024 / 256), against float64. A code of h may move by one step of
+    its block (1/127 of the block's largest value, one of ffs terms): 2e-3."""
+    out, ref = _shared_only(F, H.GGML_Q8_0, T, n, ffs, 7 * T + ffs, ff=ff)
+    err = H.out_rel(out, ref)
+    print(f"T {T} n {n} ffs {ffs}: {err:.2e}")
+    assert err <= 2e-3
+
+
 @pytest.mark.parametrize("gtype", [H.GGML_Q8_0, H.GGML_F16, H.GGML_BF16, H.GGML_F32])
 @pytest.mark.parametrize("T,n,ffs", [(9, 512, 64), (16, 512, 64), (17, 1024, 192), (33, 512, 128), (700, 2560, 640)])
 def test_shared_expert_many_tokens(F, gtype, T, n, ffs):
