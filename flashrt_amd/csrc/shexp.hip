@@ -9,7 +9,8 @@
 //     (h = g / (1 + exp(-g)) * u), or the down product. Q8_0 weights take Q8_0 activations (x and
 //     h quantized per 32 as the CPU path does, q8_0 . q8_0 per block as an exact integer dot, then
 //     scaled by d_w d_a); the other types take the fp32 activations.
-//     Taken up to 8 tokens; more go to k_shexp_mm, the same products on the matrix cores.
+//     More than 8 tokens go to k_shexp_mm, the same products on the matrix cores, save for short calls of
+//     little work (shexp_on_mfma).
 //   - the layer with such a shared expert: windows of up to 8 tokens of a shape that the decode kernels
 //     are templated for run the window kernels with the shared expert's outputs in slot K; else router
 //     logits -> route_topk -> the routed experts as per-slot outputs (moe_hits for windows of up to 8
@@ -633,8 +634,20 @@ static int shexp_mv(int type, bool dual, const void* W1, const void* W2, int row
 int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16* xhi, _Float16* xlo,
                 hipStream_t stream);
 
-// Calls of at least this many tokens run on the matrix cores (k_shexp_mm).
+// Calls of at least this many tokens may run on the matrix cores (k_shexp_mm).
 constexpr int kShMmMinT = 9;
+// Whether T tokens do. F32 and F16 weights cost nine and six products each there and the activations a launch
+// for their planes, and a few workgroups share the work, so that a short call of little work is faster on
+// k_shexp_mv, whose time goes with the tokens. A whole layer, k_shexp_mv / k_shexp_mm in us, F16, shared width x
+// hidden size: 4096 x 512 58 / 91 at 9 tokens, 81 / 92 at 20, 101 / 93 at 32; 4096 x 1024 70 / 108 at 9,
+// 105 / 107 at 20, 117 / 106 at 24; 2048 x 1536 at 24 97 / 91; 2048 x 4096 122 / 147 at 9, 158 / 148 at 16.
+// BF16 and Q8_0, three products and one, are faster on the matrix cores from 9 tokens on (0.64 to 0.85 and 0.65
+// to 0.77 of the time).
+static bool shexp_on_mfma(int type, int T, int n, int ffs) {
+    if (T < kShMmMinT) return false;
+    if (type != FRT_GGML_F32 && type != FRT_GGML_F16) return true;
+    return T > 20 || int64_t(T) * n * ffs >= 72000000;
+}
 
 size_t shexp_ws_bytes(int T, int n, int ffs) {
     const size_t mv = up256(size_t(T) * ffs * 4);
@@ -682,8 +695,9 @@ int shexp_run(int type, const void* g, const void* u, const void* d, int n, int 
               const float* xd, int T, float* sh, size_t sh_ld, void* ws, hipStream_t stream) {
     if (!shexp_type_ok(type)) return set_error(kErrShape, "shared expert: ggml type %d (F32, F16, BF16 or Q8_0)", type);
     if (!shexp_shape_ok(n, ffs)) return set_error(kErrShape, "shared expert: n=%d ffs=%d", n, ffs);
-    if (T >= kShMmMinT && sh_ld != size_t(n)) return set_error(kErrShape, "shared expert: row distance %zu", sh_ld);
-    if (T >= kShMmMinT) switch (type) {
+    const bool mm = shexp_on_mfma(type, T, n, ffs);
+    if (mm && sh_ld != size_t(n)) return set_error(kErrShape, "shared expert: row distance %zu", sh_ld);
+    if (mm) switch (type) {
         case FRT_GGML_F32: return shexp_run_mm<FRT_GGML_F32>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
         case FRT_GGML_F16: return shexp_run_mm<FRT_GGML_F16>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);
         case FRT_GGML_BF16: return shexp_run_mm<FRT_GGML_BF16>(g, u, d, n, ffs, x, xq, xd, T, sh, ws, stream);

@@ -1393,6 +1393,19 @@ def _shared_only(F, gtype, T, n, ffs, seed, ff=128, E=16, K=2, weights=None):
     return out.cpu().numpy(), ref
 
 
+@pytest.mark.parametrize("gtype", [H.GGML_F16, H.GGML_F32])
+@pytest.mark.parametrize("T,n,ffs", [(9, 512, 64), (16, 512, 4096), (20, 512, 4096), (21, 512, 4096), (20, 512, 64), (21, 512, 64),
+                                     (8, 4096, 2048), (9, 4096, 2048)])
+def test_shared_expert_short_calls(F, gtype, T, n, ffs):
+    """F16 and F32 shared experts on either side of the rule that sends a short call to the row kernel (up to
+    20 tokens, fewer than 72 M products), against float64: a root mean square error of at most 2^-20 of the
+    outputs', four times what fp32 sums of these lengths show (2.5e-7)."""
+    out, ref = _shared_only(F, gtype, T, n, ffs, 31 * T + ffs)
+    err = np.sqrt(((out - ref) ** 2).mean() / (ref ** 2).mean())
+    print(f"short type {gtype} T {T} n {n} ffs {ffs}: rms {err:.2e}")
+    assert err <= 2.0 ** -20
+
+
 @pytest.mark.parametrize("n,ff", [(512, 128), (1024, 256)])
 @pytest.mark.parametrize("ffs", [64, 320, 2112, 4096])
 @pytest.mark.parametrize("T", [1, 4, 5, 8])
