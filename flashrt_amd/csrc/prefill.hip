@@ -20,6 +20,7 @@
 
 #include <hip/hip_bf16.h>
 
+#include <algorithm>
 #include <type_traits>
 
 namespace frt {
@@ -934,6 +935,11 @@ struct PfWs {
 };
 
 static int pf_max_tiles(int S, int G) { return (S + pf_tile_tokens(S) - 1) / pf_tile_tokens(S) + G; }
+// The tile list's length in a workspace: never less than a shorter chunk's (whose tiles are of 16 tokens), so
+// that a workspace sized for the longest call holds every other.
+static size_t pf_tile_list(int S, int G) {
+    return size_t(S <= kTile16Slots ? pf_max_tiles(S, G) : std::max(pf_max_tiles(S, G), pf_max_tiles(kTile16Slots, G)));
+}
 // the gate/up GEMM's K extent: n rounded up to whole pairs of 256-element stretches
 static int pf_np(int n) { return (n + 511) & ~511; }
 
@@ -953,7 +959,7 @@ static PfWs pf_carve(void* base, int T, int K, int n, int ff, int E, bool shared
     w.tok_of = reinterpret_cast<int32_t*>(take(size_t(S) * 4));
     w.slot_of = reinterpret_cast<int32_t*>(take(size_t(S) * 4));
     w.n_tiles = reinterpret_cast<int32_t*>(take(8));   // [0] tiles, [1] first tile of one column
-    w.tiles = reinterpret_cast<int2*>(take(size_t(pf_max_tiles(S, G)) * 8));
+    w.tiles = reinterpret_cast<int2*>(take(pf_tile_list(S, G) * 8));
     w.xhi = reinterpret_cast<_Float16*>(take(size_t(T) * pf_np(n) * 2));
     w.xlo = reinterpret_cast<_Float16*>(take(size_t(T) * pf_np(n) * 2));
     w.h16 = reinterpret_cast<_Float16*>(take(size_t(S) * ((ff + 255) & ~255) * 2));
@@ -1112,26 +1118,26 @@ int pf_moe(const uint8_t* arena, size_t stride, int E, const uint8_t* shared_blo
     return kOk;
 }
 
+size_t pf_dispatch_ws_bytes(int T, int K, int E) {
+    const int nchunk = (T * K + kChunk - 1) / kChunk;
+    return up256(size_t(nchunk) * E * 4) + up256(pf_tile_list(T * K, E) * 8) + 256;
+}
 // expose the dispatch alone (tests compare the permutation with the oracle)
 int pf_dispatch(const int32_t* ids, int T, int K, int E, int32_t* bounds, int32_t* tok_of, int32_t* slot_of, void* ws,
                 size_t ws_bytes, hipStream_t stream) {
     if (T < 1 || K < 1 || E < 1 || E > 4096) return set_error(kErrShape, "dispatch: T=%d K=%d E=%d", T, K, E);
     const int nchunk = (T * K + kChunk - 1) / kChunk;
-    const size_t need = up256(size_t(nchunk) * E * 4) + up256(size_t(pf_max_tiles(T * K, E)) * 8) + 256;
+    const size_t need = pf_dispatch_ws_bytes(T, K, E);
     if (ws_bytes < need) return set_error(kErrWorkspace, "dispatch: workspace %zu < %zu", ws_bytes, need);
     uint8_t* p = static_cast<uint8_t*>(ws);
     int32_t* cnt = reinterpret_cast<int32_t*>(p);
     p += up256(size_t(nchunk) * E * 4);
     int2* tiles = reinterpret_cast<int2*>(p);
-    p += up256(size_t(pf_max_tiles(T * K, E)) * 8);
+    p += up256(pf_tile_list(T * K, E) * 8);
     int32_t* n_tiles = reinterpret_cast<int32_t*>(p);
     if (int rc = pf_dispatch_run(ids, T, K, E, false, cnt, bounds, tiles, n_tiles, tok_of, slot_of, stream)) return rc;
     FRT_LAUNCHED("dispatch");
     return kOk;
-}
-size_t pf_dispatch_ws_bytes(int T, int K, int E) {
-    const int nchunk = (T * K + kChunk - 1) / kChunk;
-    return up256(size_t(nchunk) * E * 4) + up256(size_t(pf_max_tiles(T * K, E)) * 8) + 256;
 }
 
 }  // namespace frt

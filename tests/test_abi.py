@@ -62,6 +62,19 @@ def test_dense_layer_workspace_grows_with_tokens(n, ff, K):
             assert b == sorted(b), (gtype, shared_ff, [T for T in range(1, 64) if b[T - 1] > b[T]])
 
 
+@pytest.mark.parametrize("E,K", [(1, 1), (2, 2), (7, 3), (8, 8), (64, 8), (128, 1), (512, 10), (1025, 1)])
+def test_grouped_workspaces_grow_with_tokens(E, K):
+    """The workspaces of the dispatch alone, the grouped expert products and a prefill layer never shrink as the
+    tokens grow, across the tile sizes that the number of slots selects (1536 slots)."""
+    L = _lib.lib()
+    T = range(9, 2 * 1536 // K + 70)
+    d = _layer(E, 512, 128, K)
+    for size in (lambda t: L.frt_moe_dispatch_workspace_bytes(t, K, E), lambda t: L.frt_moe_q2_workspace_bytes(t, K, 128, 128, E),
+                 lambda t: L.frt_moe_layer_workspace_bytes(C.byref(d), t)):
+        b = [size(t) for t in T]
+        assert b == sorted(b), [(t, x, y) for t, x, y in zip(T, b, b[1:]) if x > y]
+
+
 def test_argument_errors_before_device_work():
     """Shape and null-pointer errors are reported with a status and a message, as the reference's
     std::runtime_error would be, without touching a device."""
