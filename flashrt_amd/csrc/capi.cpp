@@ -3,6 +3,7 @@
 
 #include "../../include/flashrt_moe.h"
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -713,9 +714,16 @@ int frt_noalloc_sync_error(void* stream) {
     return err ? 1 : 0;
 }
 
+// the largest of the layers' workspaces (they differ from layer to layer only with dense shared experts)
+static size_t stack_layer_bytes(const frt_moe_layer* layers, int n_layer) {
+    size_t b = frt_moe_layer_workspace_bytes(&layers[0], 1);
+    for (int l = 1; l < n_layer; ++l)
+        if (layers[l].shared_dense || layers[0].shared_dense) b = std::max(b, frt_moe_layer_workspace_bytes(&layers[l], 1));
+    return b;
+}
 size_t frt_moe_stack_workspace_bytes(const frt_moe_layer* layers, int n_layer) {
     if (!layers || n_layer < 1) return 0;
-    return frt_moe_layer_workspace_bytes(&layers[0], 1) + 2 * up256(size_t(layers[0].d_model) * 4);
+    return stack_layer_bytes(layers, n_layer) + 2 * up256(size_t(layers[0].d_model) * 4);
 }
 
 int frt_moe_stack_forward(const frt_moe_layer* layers, int n_layer, const float* x, float* out, int32_t* ids,
@@ -732,13 +740,12 @@ int frt_moe_stack_forward(const frt_moe_layer* layers, int n_layer, const float*
             Ll.stride != L0.stride || Ll.flags != L0.flags)
             return set_error(kErrShape, "moe_stack: layer %d differs in shape, stride or flags from layer 0", l);
     }
-    const size_t need = frt_moe_stack_workspace_bytes(layers, n_layer);
+    const size_t lw = stack_layer_bytes(layers, n_layer), need = lw + 2 * up256(size_t(L0.d_model) * 4);
     if (ws_bytes < need) return set_error(kErrWorkspace, "moe_stack: workspace %zu < %zu", ws_bytes, need);
     const int E = L0.n_expert, K = L0.top_k, n = L0.d_model, ff = L0.d_ff;
     if (E < 1 || E > 1024 || K < 1 || K > 32 || K > E) return set_error(kErrShape, "moe_stack: E=%d K=%d", E, K);
     if (L0.stride < expert_bytes(n, ff)) return set_error(kErrShape, "moe_stack: stride %zu < blob", L0.stride);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const size_t lw = frt_moe_layer_workspace_bytes(&L0, 1);
     float* buf[2] = {reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + lw),
                      reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + lw + up256(size_t(n) * 4))};
     constexpr int kChunk = 64;   // layers of one persistent launch

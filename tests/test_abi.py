@@ -75,6 +75,19 @@ def test_grouped_workspaces_grow_with_tokens(E, K):
         assert b == sorted(b), [(t, x, y) for t, x, y in zip(T, b, b[1:]) if x > y]
 
 
+def test_stack_workspace_holds_every_layer():
+    """A stack whose layers have shared experts of different kinds and widths: its workspace holds the largest
+    layer's, whichever comes first, and the two activation buffers."""
+    L = _lib.lib()
+    kinds = [(None, 0), (8, 64), (8, 640), (0, 4096)]
+    for n, ff, K in ((512, 2048, 15), (2048, 512, 10), (2560, 640, 10)):
+        for a in kinds:
+            for b in kinds:
+                two = (_lib.FrtMoeLayer * 2)(_layer(16, n, ff, K, *a), _layer(16, n, ff, K, *b))
+                one = [L.frt_moe_layer_workspace_bytes(C.byref(d), 1) for d in two]
+                assert L.frt_moe_stack_workspace_bytes(two, 2) == max(one) + 2 * 4 * n, (n, ff, a, b, one)
+
+
 def test_argument_errors_before_device_work():
     """Shape and null-pointer errors are reported with a status and a message, as the reference's
     std::runtime_error would be, without touching a device."""
