@@ -72,6 +72,7 @@ int rmsnorm(const float* x, int T, int n, float* u, hipStream_t stream);
 int router_gemm(const float* x, int T, const float* W, const float* bias, const float* gate_w, int E, int n,
                 float* logits, float* gate, float* part, hipStream_t stream);
 size_t router_gemm_ws_bytes(int T, int E, bool gate);
+int router_gemm_check(int n);
 int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16* xhi, _Float16* xlo,
                 hipStream_t stream);
 int quantize_pairs(const float* x, int rows, int n, int np, int blk, _Float16* xhi, _Float16* xlo, int8_t* xq, float* xd,
@@ -260,7 +261,7 @@ static DenseWs dense_carve(uint8_t* p0, uint8_t* p, const frt_moe_layer& L, int 
     };
     const int E = L.n_expert, K = L.top_k, n = L.d_model, ff = L.d_ff;
     w.u = reinterpret_cast<float*>(take(size_t(T) * n * 4));
-    const size_t Tp = T <= 8 ? size_t(T) : size_t((T + 15) & ~15);   // (from 9 tokens on whole tiles of 16: shexp_code_at)
+    const size_t Tp = T < kShMmMinT ? size_t(T) : size_t((T + 15) & ~15);   // (whole tiles of 16: shexp_code_at)
     w.xq = reinterpret_cast<int8_t*>(take(Tp * n));
     w.xd = reinterpret_cast<float*>(take(Tp * (n / kQ8) * 4));
     const bool win = dense_window(L, T);
@@ -298,8 +299,12 @@ static int dense_layer(const frt_moe_layer& L, const LayerWs& lw, const DenseWs&
     const bool small = dense_small(L, T);
     const int S = dense ? K : K + 1;   // moe_hits slots per token (the Q2_0 shared expert as slot K)
     if (!dense && !small) return set_error(kErrShape, "moe_layer: slot path for T=%d K=%d n=%d ff=%d", T, K, n, ff);
-    if (!small)
+    if (!small) {   // (every shape rule of the kernels below, before the first launch)
         if (int rc = pf_check(T, K, n, ff, E)) return rc;
+        if (int rc = router_gemm_check(n)) return rc;
+        // a shape these take is dense_small's at fewer tokens; xq and xd hold whole tiles only from there on
+        if (T < kShMmMinT) return set_error(kErrShape, "moe_layer: T=%d K=%d n=%d ff=%d", T, K, n, ff);
+    }
     const float* u = x;
     const bool norm = (L.flags & FRT_LAYER_NORM_INPUT) != 0;
     if (!small) {   // the GEMMs' x pairs, and Q8_0 of the input where the shared expert takes it

@@ -35,6 +35,11 @@ __host__ __device__ inline int perm256_pos(int K) {
     return 32 * (2 * d + ((k >> 2) & 1)) + 8 * g + 2 * (k & 3) + (k >> 3);
 }
 
+// A dense shared expert's calls of at least this many tokens may run on the matrix cores (shexp.hip); those of
+// a Q8_0 one do, and take their Q8_0 input in the order below, in whole tiles of 16 tokens, where shorter
+// calls take rows.
+constexpr int kShMmMinT = 9;
+
 // Q8_0 codes and scales of rows of cols values in the order of the dense shared expert's int8 MFMA operand
 // (shexp.hip k_shexp_mm): per tile of 16 tokens and pair of 32-blocks, lane 16 g + j (g = 0..3) holds codes
 // 8 g .. 8 g + 7 of token j in both blocks; the pair's scales are [2][16]. Offsets of (token t, value k) and

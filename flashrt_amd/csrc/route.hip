@@ -745,10 +745,16 @@ int g_router_mfma = 1;   // the prefill router GEMM on the matrix cores (0: the 
 
 size_t router_gemm_ws_bytes(int T, int E, bool gate) { return size_t(kRgSplit) * T * (E + (gate ? 1 : 0)) * 4; }
 
+// the shapes the router GEMM takes (a caller that launches something before it checks them first)
+int router_gemm_check(int n) {
+    if (n % 512 || n < 512 || n > 4096) return set_error(kErrShape, "router_gemm: n=%d (a multiple of 512 up to 4096)", n);
+    return kOk;
+}
+
 // the K-split partial sums of the router GEMM (logits and gate before the combine)
 static int router_gemm_part(const float* x, int T, const float* W, const float* gate_w, int E, int n, float* gate,
                             float* part, hipStream_t stream) {
-    if (n % 512 || n < 512 || n > 4096) return set_error(kErrShape, "router_gemm: n=%d (a multiple of 512 up to 4096)", n);
+    if (int rc = router_gemm_check(n)) return rc;
     if (T < 1 || E < 1 || !part || (gate_w && !gate)) return set_error(kErrShape, "router_gemm: T=%d E=%d", T, E);
     const int E1 = E + (gate_w ? 1 : 0);
     dim3 grid((E1 + 63) / 64, (T + 63) / 64, kRgSplit);

@@ -634,9 +634,7 @@ static int shexp_mv(int type, bool dual, const void* W1, const void* W2, int row
 int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16* xhi, _Float16* xlo,
                 hipStream_t stream);
 
-// Calls of at least this many tokens may run on the matrix cores (k_shexp_mm).
-constexpr int kShMmMinT = 9;
-// Whether T tokens do. F32 and F16 weights cost nine and six products each there and the activations a launch
+// Whether a call of T tokens runs on the matrix cores (k_shexp_mm). F32 and F16 weights cost nine and six products each there and the activations a launch
 // for their planes, and a few workgroups share the work, so that a short call of little work is faster on
 // k_shexp_mv, whose time goes with the tokens. A whole layer, k_shexp_mv / k_shexp_mm in us, F16, shared width x
 // hidden size: 4096 x 512 58 / 91 at 9 tokens, 81 / 92 at 20, 101 / 93 at 32; 4096 x 1024 70 / 108 at 9,

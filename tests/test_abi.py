@@ -100,6 +100,23 @@ def test_argument_errors_before_device_work():
         _lib.check(L.frt_moe_q2_run(None, 0, 512, 2048, 512, None, None, 16, 10, None, None, 0, None, 1, 0))
 
 
+@pytest.mark.parametrize("T", [1, 4, 8, 9, 20])
+@pytest.mark.parametrize("gtype", [0, 8])
+@pytest.mark.parametrize("norm", [0, 1])
+def test_dense_layer_refuses_shapes_before_any_launch(T, gtype, norm):
+    """A layer with a dense shared expert whose n is a multiple of 128 but not of 512: the grouped products
+    would take it, the router does not. The call is refused for its shape before it launches anything (a
+    launch would report FRT_ERR_HIP here, where there is no device)."""
+    L = _lib.lib()
+    d = _layer(16, 640, 128, 2, gtype, 64, norm)
+    n = L.frt_moe_layer_workspace_bytes(C.byref(d), T)
+    ws = C.create_string_buffer(n + 256)
+    before = ws.raw
+    rc = L.frt_moe_layer_forward(C.byref(d), 256, T, None, 256, None, None, None, (C.addressof(ws) + 255) // 256 * 256, n, None)
+    assert rc == -1, (rc, L.frt_last_error())
+    assert ws.raw == before
+
+
 def test_q2_repack_matches_reference_fixture():
     """The product's host repack (frt_q2_repack) reproduces the reference's compiled repack on the
     golden blocks bit for bit (tests/golden/q2_format.npz, 8 rows x 4096), and repack_expert places
