@@ -243,7 +243,8 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef int intx4 __attribute__((ext_vector_type(4)));
 
 // v = hi + mid + lo exactly, each with at most 8 significant bits (truncations: no part overflows);
-// an infinity or a NaN stays in hi alone
+// an infinity or a NaN stays in hi alone (its products with the other operand's zero parts are NaN where
+// the value's own are not: k_shexp_mm forms such sums again, dot_chain)
 __device__ __forceinline__ void split3(float v, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
     const uint32_t b = __float_as_uint(v);
     hi = b & 0xffff0000u;
@@ -316,6 +317,25 @@ struct ShDense {
         for (int p = 0; p < parts; ++p) out[p] = __builtin_bit_cast(bf16x8, make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]));
     }
 };
+
+// Row `row` of weights (TYPE) against token t of the planes, as one chain of fused multiply-adds.
+template <int TYPE>
+__device__ __forceinline__ float dot_chain(const uint8_t* row, const uint16_t* ap, size_t plane, int t, int cols) {
+    float s = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < cols; ++k) {
+        float w;
+        if constexpr (TYPE == FRT_GGML_F32) w = reinterpret_cast<const float*>(row)[k];
+        else if constexpr (TYPE == FRT_GGML_F16) w = h2f(reinterpret_cast<const uint16_t*>(row)[k]);
+        else w = __uint_as_float(uint32_t(reinterpret_cast<const uint16_t*>(row)[k]) << 16);
+        const uint16_t* a = ap + plane_at(t, k, cols);
+        float x = 0.0f;   // lo, mid, hi: exact
+#pragma unroll
+        for (int p = 2; p >= 0; --p) x += __uint_as_float(uint32_t(a[p * plane]) << 16);
+        s = fmaf(w, x, s);
+    }
+    return s;
+}
 
 // out (DUAL): dense types the planes of h = silu(gate) * up, Q8_0 its codes hq and scales hd (both as the
 // input's); else of [T][rows] fp32. aq / ad or ap (planes): the input.
@@ -492,6 +512,27 @@ __global__ void __launch_bounds__(256) k_shexp_mm(const uint8_t* __restrict__ W1
     floatx4 v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = (part[0][c][i][lane] + part[1][c][i][lane]) + (part[2][c][i][lane] + part[3][c][i][lane]);
+    if constexpr (!Q8) {   // an infinity or a NaN among the operands: never a finite sum (split3)
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bad |= !(fabsf(v[i][r]) < INFINITY);
+        if (__builtin_expect(bad && t < T, 0)) {   // (the sums go through LDS so that the loop stays small)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part[0][c][i][lane] = v[i];
+#pragma unroll 1
+            for (int q = 0; q < 16; ++q) {
+                const int i = q >> 2, row = r0 + 16 * (DUAL ? i & 1 : i) + 4 * lg + (q & 3);
+                float* p = reinterpret_cast<float*>(&part[0][c][i][lane]) + (q & 3);
+                if (!(fabsf(*p) < INFINITY))
+                    *p = dot_chain<TYPE>((DUAL && i >= 2 ? W2 : W1) + size_t(row) * cols * (TYPE == FRT_GGML_F32 ? 4 : 2), ap,
+                                         up16(T) * cols, t, cols);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = part[0][c][i][lane];
+        }
+    }
     if constexpr (!DUAL) {
         if (t < T)
 #pragma unroll

@@ -1406,6 +1406,36 @@ def test_shared_expert_short_calls(F, gtype, T, n, ffs):
     assert err <= 2.0 ** -20
 
 
+@pytest.mark.parametrize("gtype", [H.GGML_F16, H.GGML_BF16, H.GGML_F32])
+@pytest.mark.parametrize("case", ["gate", "up", "down", "overflow"])
+def test_shared_expert_nonfinite(F, gtype, case):
+    """An infinite weight of the shared expert, or weights whose h overflows fp32: the outputs of a call on the
+    matrix cores are infinite, NaN and finite where the same tokens' are in a short call (fma chains): an
+    infinity's products with the zero parts of the other operand do not turn it into a NaN."""
+    def plant(raw):
+        view = {H.GGML_F16: np.float16, H.GGML_BF16: np.uint16, H.GGML_F32: np.float32}[gtype]
+        inf = np.uint16(0x7F80) if gtype == H.GGML_BF16 else np.inf
+        if case == "overflow":
+            if gtype == H.GGML_F16:   # (fp16 weights cannot: an infinite down weight of another row instead)
+                raw[2].view(view).reshape(512, 128)[300, 7] = inf
+                return
+            big = np.uint16(0x6951) if gtype == H.GGML_BF16 else np.float32(1.6e25)   # (bf16: 1.58e25)
+            raw[0].view(view).reshape(128, 512)[9, 4] = big
+            raw[1].view(view).reshape(128, 512)[9, 4] = big
+        else:
+            m = ("gate", "up", "down").index(case)
+            raw[m].view(view).reshape(512 if m == 2 else 128, -1)[100, 11] = inf
+    long, _ = _shared_only(F, gtype, 24, 512, 128, 5, weights=plant)
+    short, _ = _shared_only(F, gtype, 8, 512, 128, 5, weights=plant)
+    long = long[:8]
+    assert np.isinf(short).any()
+    assert np.array_equal(np.isnan(long), np.isnan(short))
+    assert np.array_equal(np.isinf(long), np.isinf(short))
+    assert np.array_equal(np.sign(long[np.isinf(long)]), np.sign(short[np.isinf(short)]))
+    ok = np.isfinite(short)
+    assert np.abs(long[ok] - short[ok]).max(initial=0.0) <= 1e-5 * np.abs(short[ok]).max(initial=1.0)
+
+
 @pytest.mark.parametrize("n,ff", [(512, 128), (1024, 256)])
 @pytest.mark.parametrize("ffs", [64, 320, 2112, 4096])
 @pytest.mark.parametrize("T", [1, 4, 5, 8])
