@@ -517,9 +517,8 @@ def test_layer_envelope_decode(F, n, ff):
 
 @pytest.mark.parametrize("n,ff", ENVELOPE)
 def test_moe_q2_run_envelope(F, n, ff):
-    """moe_q2::run at those shapes, T = 200 (ff above 1024: the down GEMM in chunks of 1024 added up in
-    fp32 yd): sampled slots within 2e-3 of the oracle's expert_ffn; bf16 yd with ff above 1024 and ff
-    above 4096 are refused (FRT_ERR_SHAPE)."""
+    """moe_q2::run at those shapes, T = 200 (800 slots, tiles of up to 16 tokens): sampled slots within 2e-3 of
+    the oracle's expert_ffn; bf16 yd with ff above 1024 and ff above 4096 are refused (FRT_ERR_SHAPE)."""
     T, K, E = 200, 4, 12
     w = H.World(cfg=0, n=n, ff=ff, E=E, K=K)
     rng = np.random.default_rng(7 * n + ff)
@@ -744,12 +743,11 @@ def test_moe_q2_run_block64(F, n, ff, T, K, E):
                                          (640, 384, 60, 3, 5), (896, 256, 40, 2, 4), (128, 128, 30, 2, 3),
                                          (1152, 640, 20, 4, 6)])
 def test_moe_q2_run_shapes(F, n, ff, T, K, E):
-    """moe_q2::run at other shapes and tile mixes, every slot against the oracle's expert_ffn:
-    ff = 1024 (four weight stretches per down row block, a 128 KB tile in LDS) with n = 1024 and about
-    27 rows per expert (two-column tiles); only one-column tiles (T = 8, K = 2 over 8 experts); full
-    64-row tiles next to partial ones (T = 200, K = 3 over 4 experts); ff not a multiple of 256 (the
-    h rows padded to whole stretches: 640 = the reference tests' 2560 / 640 shape, with a stretch
-    count that is not a multiple of 4; 128; 384) and n = 512 and 1536; n a multiple of 128 but not of 512
+    """moe_q2::run at other shapes, in tiles of up to 16 tokens (at most 1536 slots), every slot against the
+    oracle's expert_ffn: ff = 1024 (four weight stretches in the down product) with n = 1024 and about 27 rows
+    per expert; groups of a row or two (T = 8, K = 2 over 8 experts) and of about 150 (T = 200, K = 3 over 4
+    experts); ff not a multiple of 256 (the h rows padded to whole stretches: 640 = the reference tests'
+    2560 / 640 shape, 128, 384) and n = 512 and 1536; n a multiple of 128 but not of 512
     (moe_q2.cu:516-517 accepts those: 640, 896, 128, 1152; the activations are padded with zeros to
     a multiple of 512 and the down GEMM's last row block is partial)."""
     w = H.World(cfg=0, n=n, ff=ff, E=E, K=K)
@@ -799,6 +797,58 @@ def test_moe_q2_run_tile_edges(F, n, ff, rep):
     assert err.max() <= max(H.OUT_REL, 0.1 / ff ** 0.5), (err.argmax(), ids[err.argmax()], err.max())
     assert (err > H.OUT_REL).mean() <= 0.005, (err > H.OUT_REL).sum()
     assert np.median(err) <= H.OUT_REL / 4
+
+
+@pytest.mark.parametrize("n,ff,block64,bf16", [(640, 384, True, False), (512, 640, True, True), (1024, 256, False, True),
+                                               (512, 1024, True, False), (1024, 1024, False, True), (512, 2048, False, False),
+                                               (512, 4096, True, False)])
+def test_moe_q2_run_large_tiles(F, n, ff, block64, bf16):
+    """The 17-64-token tiles (chunks of more than 1536 slots: 2148 here) with Q8 blocks of 64, bf16 outputs and
+    rows of 256 to 4096 in the down product: the rows at the edges of every tile and token column of groups of
+    every size class, against the oracle's expert. The bounds are test_moe_q2_run_tile_edges', plus half a
+    step of bf16."""
+    sizes = [1, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 80, 81, 128, 0, 2] * 3
+    rng = np.random.default_rng(n + ff)
+    ids = np.repeat(np.arange(len(sizes)), sizes).astype(np.int32)
+    rng.shuffle(ids)
+    T, E = ids.size, len(sizes)
+    assert T > 1536
+    eb = F.expert_bytes(n, ff)
+    arena = torch.empty(E * eb, dtype=torch.uint8, device="cuda")
+    F.gen.experts(arena, eb, 7, 0, 0, E, n, ff)
+    x = rng.standard_normal((T, n)).astype(np.float32)
+    nb = F.moe_q2.workspace_bytes(T, 1, n, ff, E)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    yd = torch.full((T, n), float("nan"), dtype=torch.bfloat16 if bf16 else torch.float32, device="cuda")
+    F.moe_q2.run(arena.data_ptr(), eb, E, n, ff, torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda(), T, 1, yd, ws, nb,
+                 None, block64, bf16)
+    torch.cuda.synchronize()
+    y, ah = yd.float().cpu().numpy(), arena.cpu().numpy().reshape(E, eb)
+    assert np.isfinite(y).all()
+    rows = []
+    for e in range(E):
+        at = np.nonzero(ids == e)[0]   # (the group's rows in order)
+        rows += [at[i] for i in sorted({0, 1, 15, 16, 31, 32, 47, 48, 63, 64, 79, 80, 127, len(at) - 1}) if 0 <= i < len(at)]
+    step = 2.0 ** -9 if bf16 else 0.0
+    err = np.array([H.out_rel(y[t][None], O.expert_ffn(ah[ids[t]], n, ff, x[t], blk=64 if block64 else 32)) for t in rows])
+    print(f"large tiles n {n} ff {ff} block64 {block64} bf16 {bf16}: {len(rows)} rows, max {err.max():.2e}, "
+          f"median {np.median(err):.2e}, above {(err > H.OUT_REL + step).sum()}")
+    assert err.max() <= max(H.OUT_REL, 0.1 / ff ** 0.5) + step, (err.argmax(), err.max())
+    assert (err > H.OUT_REL + step).mean() <= 0.01
+    assert np.median(err) <= H.OUT_REL / 4 + step
+
+
+@pytest.mark.parametrize("n,ff", [(512, 1024), (512, 2048), (1024, 4096)])
+def test_layer_prefill_large_tiles(F, n, ff):
+    """Whole layers of 400 tokens, K = 4 (2000 slots with the shared group: tiles of up to 64 tokens), at ff of 1024
+    and above: ids bit-exact, weights 1e-6, outputs 2e-3."""
+    w = H.World(cfg=0, n=n, ff=ff, E=16, K=4)
+    x = np.random.default_rng(5 * n + ff).standard_normal((400, n)).astype(np.float32)
+    out, ids, wts = w.gpu_forward(x)
+    ref, rid, rw, _ = w.oracle_forward(x)
+    assert np.array_equal(ids, rid), (n, ff)
+    assert H.w_rel(wts, rw) <= H.W_REL
+    assert H.out_rel(out, ref) <= H.OUT_REL, (n, ff)
 
 
 def test_moe_q2_run_shape_errors(F, w0):
@@ -1451,44 +1501,43 @@ def test_shared_expert_q8_windows(F, T, ffs, n, ff):
 
 
 @pytest.mark.parametrize("gtype", [H.GGML_Q8_0, H.GGML_F16, H.GGML_BF16, H.GGML_F32])
-@pytest.mark.parametrize("T,n,ffs", [(9, 512, 64), (16, 512, 64), (17, 1024, 192), (33, 512, 128), (700, 2560, 640)])
+@pytest.mark.parametrize("T,n,ffs", [(9, 512, 64), (16, 512, 64), (17, 1024, 192), (32, 512, 64), (33, 512, 128), (700, 2560, 640),
+                                     (1025, 2560, 640), (1055, 2560, 640)])
 def test_shared_expert_many_tokens(F, gtype, T, n, ffs):
-    """The dense shared expert on the matrix cores (from 9 tokens): edges of the 16- and 32-token and
-    32-row tiles, one to ten K-steps per wave, against float64 on the weights' exact values. The routed
-    experts have zero scales, so the layer gives sigmoid(gate) * shared. The dense types' products are
-    exact and summed in fp32: n and ffs terms in two products, 4 (n + ffs) 2^-24 of the rows' sizes covers
-    their roundings many times over. Q8_0 rounds h to codes, so a code may move by one step of its block
-    (1/127 of the block's largest value, one of ffs terms): 2e-3."""
-    E, K, ff = 16, 2, 128
-    rng = np.random.default_rng(T + gtype)
-    eb = F.expert_bytes(n, ff)
-    stride = (eb + 4095) // 4096 * 4096
-    arena = torch.zeros(E * stride, dtype=torch.uint8, device="cuda")
-    router = torch.from_numpy((rng.standard_normal((E, n)) * 0.02).astype(np.float32)).cuda()
-    gate = (rng.standard_normal(n) * 0.02).astype(np.float32)
-    raw = [H.dense_tensor(gtype, r, c, rng) for r, c in ((ffs, n), (ffs, n), (n, ffs))]
-    dv = [torch.from_numpy(a).cuda() for a in raw]
-    gate_d = torch.from_numpy(gate).cuda()
-    ml = F.MoeLayer(arena.data_ptr(), stride, E, 0, router, gate_d, n, ff, K)
-    ml.set_shared_dense(gtype, *dv, ffs)
-    x = rng.standard_normal((T, n)).astype(np.float32)
-    out = torch.full((T, n), float("nan"), dtype=torch.float32, device="cuda")
-    ml.forward(torch.from_numpy(x).cuda(), out, T=T)
-    torch.cuda.synchronize()
-    g, u, d = (H.dense_values(gtype, a, r, c) for a, (r, c) in zip(raw, ((ffs, n), (ffs, n), (n, ffs))))
-    xx = x.astype(np.float64)
-    if gtype == H.GGML_Q8_0:
-        q, s = O.quantize_q8(x)
-        xx = (q.reshape(T, n // 32, 32) * s.reshape(T, n // 32, 1).astype(np.float64)).reshape(T, n)
-    gg = xx @ g.T
-    h = gg / (1 + np.exp(-gg)) * (xx @ u.T)
-    if gtype == H.GGML_Q8_0:
-        q, s = O.quantize_q8(h.astype(np.float32))
-        h = (q.reshape(T, ffs // 32, 32) * s.reshape(T, ffs // 32, 1).astype(np.float64)).reshape(T, ffs)
-    ref = (h @ d.T) / (1 + np.exp(-(x.astype(np.float64) @ gate)))[:, None]
-    err = H.out_rel(out.cpu().numpy(), ref)
-    print(f"type {gtype} T {T} n {n} ffs {ffs}: {err:.2e}")
+    """The dense shared expert of more than 8 tokens: edges of the 16- and 32-token and 32-row tiles of the matrix
+    cores (32 tokens from 512 workgroups on: the down product at 700 tokens, both at 1025, whose last workgroups
+    have a token column wholly past the end, and at 1055), one to twenty K-steps per wave, against float64 on the
+    weights' exact values. The dense types' products are exact and summed in fp32: a root mean square error of at most
+    2^-20, four times what such sums show (2.5e-7); a plane or a cross product left out shows 4e-6 and more. Q8_0
+    rounds h to codes, so a code may move by one step of its block (1/127 of the block's largest value, one of ffs
+    terms): 2e-3."""
+    out, ref = _shared_only(F, gtype, T, n, ffs, T + gtype)
+    err, rms = H.out_rel(out, ref), np.sqrt(((out - ref) ** 2).mean() / (ref ** 2).mean())
+    print(f"type {gtype} T {T} n {n} ffs {ffs}: {err:.2e} rms {rms:.2e}")
     assert err <= (2e-3 if gtype == H.GGML_Q8_0 else 4 * (n + ffs) * 2.0 ** -24)
+    assert gtype == H.GGML_Q8_0 or rms <= 2.0 ** -20
+
+
+@pytest.mark.parametrize("gtype", [H.GGML_Q8_0, H.GGML_BF16])
+@pytest.mark.parametrize("n,ff,E,K,T,win", [(2048, 512, 1000, 10, 3, True), (2048, 512, 1024, 16, 7, True), (2560, 640, 64, 10, 8, True),
+                                            (1024, 1024, 128, 31, 4, True), (1024, 256, 31, 31, 1, True),
+                                            (2048, 512, 10, 10, 8, True), (2048, 512, 64, 16, 8, False), (1024, 256, 64, 31, 5, False),
+                                            (4096, 256, 64, 32, 1, False)])
+def test_layer_dense_window_shapes(F, gtype, n, ff, E, K, T, win):
+    """Windows of a layer with a dense shared expert, RMS norm and residual on either side of the rule that sends
+    them to the window kernels (K + 1 <= 32 slots a token, at most 128 in all): more than 512 experts, wide K,
+    ff = 640, experts that all tokens share (two entries each); the path by the kernels that run, ids bit-exact,
+    weights 1e-6, outputs 2e-3."""
+    w = _dense_world(gtype, 192, 40 + gtype, cfg=0, n=n, ff=ff, E=E, K=K, norm_input=True)
+    x = (np.random.default_rng(T + n + K).standard_normal((T, n)) * 2).astype(np.float32)
+    out, ids, wts = w.gpu_forward(x, resid=x)
+    ref, rid, rw, _ = O.moe_layer(w.arena_h, w.stride, w.E, w.dense, w.router_h, w.bias_h, w.gate_h, w.n, w.ff, w.K,
+                                  x, threads=8, norm_input=True)
+    assert np.array_equal(ids, rid)
+    assert H.w_rel(wts, rw) <= H.W_REL
+    assert H.out_rel(out - x, ref) <= H.OUT_REL
+    xd, o = dev(x), torch.empty((T, n), dtype=torch.float32, device="cuda")
+    assert ("win_route" in _kernels(F, lambda: w.layer_obj.forward(xd, o, T=T, resid=xd))) == win
 
 
 def test_layer_dense_shared_expert_stack_norm(F):

@@ -49,6 +49,22 @@ def test_noalloc_matches_workspace_entry(cfg):
         assert not F.noalloc_sync_error()   # no allocation-free call ran out of time
 
 
+@pytest.mark.parametrize("gtype", [H.GGML_Q8_0, H.GGML_F32])
+def test_noalloc_dense_shared_expert(gtype):
+    """A layer with a dense shared expert through both entries: the same bits at 3 tokens and at one."""
+    w = H.World(cfg=0)
+    rng = np.random.default_rng(70 + gtype)
+    raw = [H.dense_tensor(gtype, r, c, rng) for r, c in ((512, w.n), (512, w.n), (w.n, 512))]
+    dv = [torch.from_numpy(a).cuda() for a in raw]
+    w.layer_obj.set_shared_dense(gtype, *dv, 512)
+    for T in (3, 1):
+        x = rng.standard_normal((T, H.N)).astype(np.float32)
+        got, ref = _run(w, x, x, noalloc=True), _run(w, x, x, noalloc=False)
+        for a, b in zip(got, ref):
+            assert np.array_equal(a, b), T
+        assert np.isfinite(got[0]).all()
+
+
 def test_noalloc_largest_decode_workspace_fits():
     """Every decode window the entry point takes (E <= 1024, n <= 4096, ff <= 1024, T <= 4,
     T * K <= 63) has a layer workspace within the static array."""
