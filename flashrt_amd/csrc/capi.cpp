@@ -73,8 +73,7 @@ int router_gemm(const float* x, int T, const float* W, const float* bias, const 
                 float* logits, float* gate, float* part, hipStream_t stream);
 size_t router_gemm_ws_bytes(int T, int E, bool gate);
 int router_gemm_check(int n);
-int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16* xhi, _Float16* xlo,
-                hipStream_t stream);
+int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, hipStream_t stream);
 int quantize_pairs(const float* x, int rows, int n, int np, int blk, _Float16* xhi, _Float16* xlo, int8_t* xq, float* xd,
                    hipStream_t stream);
 int router_gemm_topk(const float* x, int T, const float* W, const float* bias, const float* gate_w, int E, int n,
@@ -219,9 +218,8 @@ static bool window_path(const frt_moe_layer& L, int T) {
 // ---- the slot path of a layer: the routed experts as per-slot outputs (moe_hits for windows of up to 8
 // tokens, moe_q2::run beyond), the shared expert, then the slot combine. Taken by a layer whose shared
 // expert is given as dense GGUF tensors (frt_moe_layer.shared_dense; shexp.hip) unless dense_window takes
-// the call, and by windows whose
-// shape is outside the templated decode kernels (n a multiple of 512, ff a multiple of 64 up to 4096:
-// the reference's moe_hits envelope), where the Q2_0 shared expert is moe_hits slot K.
+// the call, and by windows whose shape is outside the templated decode kernels (n a multiple of 512, ff a
+// multiple of 64 up to 4096: the reference's moe_hits envelope), where the Q2_0 shared expert is moe_hits slot K.
 struct DenseWs {
     float* u;                  // the layer input (normalised with FRT_LAYER_NORM_INPUT)
     int8_t* xq;
@@ -346,7 +344,7 @@ static int dense_layer(const frt_moe_layer& L, const LayerWs& lw, const DenseWs&
             return rc;
         }
         if (small)
-            if (int rc = quantize_q8(u, T, n, w.xq, w.xd, nullptr, nullptr, s)) return rc;
+            if (int rc = quantize_q8(u, T, n, w.xq, w.xd, s)) return rc;
     }
     timing_mark(s, "router");
     if (small)   // (the GEMM path selected already)
@@ -569,7 +567,7 @@ int frt_router_widen(void* stream, const void* src, int type, size_t count, floa
 
 int frt_quantize_q8(void* stream, const float* x, int rows, int n, int8_t* xq, float* xd) {
     if (!x || !xq || !xd) return set_error(kErrNull, "quantize_q8: null pointer");
-    return quantize_q8(x, rows, n, xq, xd, nullptr, nullptr, static_cast<hipStream_t>(stream));
+    return quantize_q8(x, rows, n, xq, xd, static_cast<hipStream_t>(stream));
 }
 
 int frt_quantize_pairs(void* stream, const float* x, int rows, int n, int block, uint16_t* xhi, uint16_t* xlo) {

@@ -249,14 +249,18 @@ __global__ void __launch_bounds__(64) k_pf_place(const int32_t* __restrict__ ids
 // 1024 (a thread per expert). Wave w ranks its slots in order by ballots against its own histogram
 // (hist [16][E]), the histograms are summed over the waves per expert, one scan gives the groups' first
 // rows and the tiles, and each slot goes to its place: the same bounds, tiles and rows as the four
-// kernels above. What bounds either is launches and latency: 21 -> 9 us for 370 slots. (Longer chunks keep
+// kernels above. What bounds either is launches and latency: 21 -> 6 us for 370 slots. (Longer chunks keep
 // the four kernels: one workgroup would walk them serially, 36 against 24 us at 20480 slots.)
 constexpr int kSmallSlots = 4096;
 // The tokens per tile of a chunk of S slots (k_pf_dispatch1's tn): with few slots there are fewer
 // workgroups than the chip holds, and a 64-token tile's serial K loop (32 stages) sets the time; tiles of
 // 16 tokens are more and shorter, at the price of weights dequantized once per 16 tokens. Layers of 37
-// and 64 tokens (skewed): 78.5 -> 64.1 and 81.3 -> 73.1 us; 93 (even): unchanged; 140: 145.0 -> 146.1 skewed,
-// 190.4 -> 181.7 with 16 hot experts; 200: 162 -> 169; 340: 194 -> 206.
+// and 64 tokens (skewed) of 10 out of 512 experts: 78.5 -> 64.1 and 81.3 -> 73.1 us; 93 (even): unchanged; 140:
+// 145.0 -> 146.1 skewed, 190.4 -> 181.7 with 16 hot experts; 200: 162 -> 169; 340: 194 -> 206. With few experts
+// each weight is dequantized up to four times as often, but there are fewer tiles still. The expert products
+// alone, tiles of 64 -> of 16, 8 experts (the same within 5% with 16): 160 slots 51.5 -> 32.7 us (2048 / 512),
+// 62.7 -> 37.5 (2560 / 640); 512 slots 56.3 -> 39.6, 68.9 -> 46.3; 1024 slots 60.3 -> 53.7, 74.4 -> 64.8, but at 1024 /
+// 1024 46.1 -> 47.4; 1536 slots 63.1 -> 59.9, 79.0 -> 83.4, 50.5 -> 55.2: the line for few experts lies near it too.
 constexpr int kTile16Slots = 1536;
 static int pf_tile_tokens(int S) { return S <= kTile16Slots ? 16 : kTN; }
 __global__ void __launch_bounds__(1024) k_pf_dispatch1(const int32_t* __restrict__ ids, int S, int K, int E, int id_bits, int T,
@@ -963,7 +967,7 @@ static PfWs pf_carve(void* base, int T, int K, int n, int ff, int E, bool shared
     w.xhi = reinterpret_cast<_Float16*>(take(size_t(T) * pf_np(n) * 2));
     w.xlo = reinterpret_cast<_Float16*>(take(size_t(T) * pf_np(n) * 2));
     w.h16 = reinterpret_cast<_Float16*>(take(size_t(S) * ((ff + 255) & ~255) * 2));
-    // (fp32 when ff > 1024: the down GEMM's chunks are added up in it)
+    // (fp32 when ff > 1024: pf_moe)
     w.yd = own_yd ? reinterpret_cast<_Float16*>(take(size_t(S) * n * (ff > 1024 ? 4 : 2))) : nullptr;
     w.bytes = size_t(p - static_cast<uint8_t*>(base));
     return w;
@@ -980,8 +984,8 @@ int norm_pairs(const float* x, int rows, int n, int np, float* u, _Float16* xhi,
 
 int pf_check(int T, int K, int n, int ff, int E) {
     if (T < 1 || K < 1 || K > 32 || E < 1 || E > 4096 || K > E) return set_error(kErrShape, "prefill: T=%d K=%d E=%d", T, K, E);
-    // n and ff multiples of 128 (moe_q2.cu:516-517); gate/up: slices of 128 ff rows; down: the tile's
-    // h (ff rounded up to 256) in LDS in chunks of at most 1024
+    // n and ff multiples of 128 (moe_q2.cu:516-517): gate/up takes slices of 128 ff rows, and a row's 64-blocks
+    // come in pairs
     if (n % 128 || n < 128 || n > 65536 || ff % 128 || ff < 128 || ff > 4096)
         return set_error(kErrShape, "prefill: n=%d ff=%d (n and ff multiples of 128; ff at most 4096)", n, ff);
     return kOk;
@@ -1011,6 +1015,7 @@ template <typename OutT>
 static int pf_expert_gemms(const uint8_t* arena, size_t stride, int E, const uint8_t* shared_blob, int n, int ff,
                            int blk, const PfWs& w, int mt, OutT* ydf, hipStream_t stream) {
     const int ffp = (ff + 255) / 256 * 256;   // h row length
+    // (the kernels take any ff: 16-bit outputs of longer sums are refused as a matter of precision)
     if (ffp > 1024 && !std::is_same<OutT, float>::value)
         return set_error(kErrShape, "prefill: ff=%d above 1024 needs fp32 per-slot outputs", ff);
     if (int rc = pf_gemm<false>("pf_gateup", arena, stride, E, shared_blob, n, pf_np(n), ff, blk,
@@ -1102,7 +1107,7 @@ int pf_moe(const uint8_t* arena, size_t stride, int E, const uint8_t* shared_blo
     if (int rc = pf_check(T, K, n, ff, E)) return rc;
     const PfWs w = pf_carve(ws, T, K, n, ff, E, true, true);
     if (w.bytes > ws_bytes) return set_error(kErrWorkspace, "prefill: workspace %zu < %zu", ws_bytes, w.bytes);
-    if (ff > 1024) {   // fp32 per-slot outputs
+    if (ff > 1024) {   // fp32 per-slot outputs: fp16 ones would be a precision less than these layers have
         if (int rc = pf_experts(arena, stride, E, shared_blob, n, ff, x, ids, T, K, w.yd, 0, 32, w, pairs_done, stream)) return rc;
         launch_timed("pf_combine", k_pf_combine<float>, dim3((n + 1023) / 1024, T), dim3(256), 0, stream,
                      (const float*)w.yd, ids, wts, gate, T, K, n, 1, resid, out);

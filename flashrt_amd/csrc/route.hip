@@ -155,11 +155,8 @@ __global__ void __launch_bounds__(256) k_rmsnorm(const float* __restrict__ x, in
 }
 
 // ---- Q8_0 of activations: one wave per 2 blocks of 32 (quant/q2_0/q2_0.cpp:93-108).
-// xq int8 [rows][n] natural order, xd [rows][n/32]. With xhi (and xlo): the activations a = q * d as
-// fp16 in the prefill GEMM's operand order (perm256_pos), [rows][n]: xhi = fp16(a) and
-// xlo = fp16(a - xhi), an exact pair (a has at most 7 + 11 significant bits).
-__global__ void k_quant_q8(const float* __restrict__ x, int n_blocks, int8_t* __restrict__ xq, float* __restrict__ xd,
-                           _Float16* __restrict__ xhi, _Float16* __restrict__ xlo, int n) {
+// xq int8 [rows][n] natural order, xd [rows][n/32].
+__global__ void k_quant_q8(const float* __restrict__ x, int n_blocks, int8_t* __restrict__ xq, float* __restrict__ xd) {
     const int gw = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;   // global wave
     const int lane = threadIdx.x & 63;
     const int blk = gw * 2 + (lane >> 5);
@@ -172,23 +169,15 @@ __global__ void k_quant_q8(const float* __restrict__ x, int n_blocks, int8_t* __
     const float id = q8_inv(d);
     const int q = q8_code(v, id);
     if (!live) return;
-    if (xq) xq[size_t(blk) * kQ8 + j] = int8_t(q);
-    const float dr = f16_round(d);
-    if (xd && j == 0) xd[blk] = dr;
-    if (xhi) {
-        const size_t e = size_t(blk) * kQ8 + j;   // element index in the row-major [rows][n]
-        const size_t pos = (e & ~size_t(255)) + perm256_pos(int(e & 255));
-        const float a = float(q) * dr;
-        const _Float16 hi = _Float16(a);
-        xhi[pos] = hi;
-        if (xlo) xlo[pos] = _Float16(a - float(hi));
-    }
+    xq[size_t(blk) * kQ8 + j] = int8_t(q);
+    if (j == 0) xd[blk] = f16_round(d);
 }
 
 // ---- Q8_0 of activations into the prefill GEMM's exact (hi, lo) fp16 pairs, perm256_pos order: one
 // wave per 256-element stretch, 4 consecutive elements per lane (8 lanes per Q8_0 block of 32). The
 // pairs go through LDS so that each lane then writes 4 consecutive positions (8 bytes) of each.
-// Same values as k_quant_q8 with xhi / xlo.
+// The values a = q d of k_quant_q8: xhi = fp16(a) and xlo = fp16(a - xhi), an exact pair (a has at most 7 + 11
+// significant bits).
 // x [rows][n] -> the pairs [rows][np] (np >= n a multiple of 256; positions n .. np - 1 are zeros),
 // Q8_0 blocks of blk = 32 or 64 values (moe_q2::run's block64). xq / xd (or null; blk 32): the same
 // codes and scales in the dense shared expert's order (shexp_code_at, shexp_scale_at).
@@ -420,13 +409,11 @@ int norm_pairs(const float* x, int rows, int n, int np, float* u, _Float16* xhi,
     return kOk;
 }
 
-int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16* xhi, _Float16* xlo,
-                hipStream_t stream) {
+int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, hipStream_t stream) {
     if (rows < 1 || n % 64) return set_error(kErrShape, "quantize_q8: n=%d not a multiple of 64", n);
     const int nb = rows * (n / kQ8);
-    if (xhi && xlo && !xq && !xd && n % 256 == 0) return quantize_pairs(x, rows, n, n, 32, xhi, xlo, nullptr, nullptr, stream);
     const int waves = (nb + 1) / 2;
-    launch_timed("pf_quant_x", k_quant_q8, dim3((waves + 3) / 4), dim3(256), 0, stream, x, nb, xq, xd, xhi, xlo, n);
+    launch_timed("pf_quant_x", k_quant_q8, dim3((waves + 3) / 4), dim3(256), 0, stream, x, nb, xq, xd);
     FRT_LAUNCHED("quantize_q8");
     return kOk;
 }

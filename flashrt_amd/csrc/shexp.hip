@@ -217,7 +217,8 @@ __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ 
 // its four waves split K in quarters and add their sums in LDS as (q0 + q1) + (q2 + q3), so that a
 // chunk of a few hundred tokens still has several waves per SIMD and no wave runs a long serial K loop.
 // Operands go straight from global memory (each weight row is read by one wave; the activations come
-// from L2) into registers, one K-step ahead; no LDS and no barrier in the K loop. The activations are kept in
+// from L2) into registers, one K-step ahead; no barrier in the K loop, and LDS only for a wave's own Q8_0 block
+// scales, from the lanes that load them to those that use them. The activations are kept in
 // the MFMA's own order, a 16-token tile's K-step as 64 lanes x 16 bytes, so that a load's four consecutive
 // lanes read 64 bytes: the L1 takes a clock per 64-byte piece, and in rows (16 tokens x 64 bytes, another
 // token in every lane) a 1 KB load takes 64 clocks instead of 16. The weights stay in the file's rows.
@@ -226,8 +227,8 @@ __global__ void __launch_bounds__(kShNT) k_shexp_mv(const uint8_t* __restrict__ 
 //   scales [tiles][K / 64][2][16].
 //   F32, F16, BF16 weights: the fp32 activations are split exactly into three bf16 planes
 //     (k_split3: 8 + 8 + 8 significant bits by truncation), the weights into one (BF16), two (F16) or
-//     three (F32), and every pair of parts is one v_mfma_f32_16x16x32_bf16 into one fp32 accumulator:
-//     exact products, fp32 sums, as the fmaf chains of k_shexp_mv.
+//     three (F32), and every pair of parts is one v_mfma_f32_16x16x32_bf16: exact products, fp32 sums (three,
+//     see Precision), as the fmaf chains of k_shexp_mv.
 //   Q8_0 weights: v_mfma_i32_16x16x32_i8 per 32-block, an exact integer dot, then + float(s) * (d_w d_a),
 //     the terms of k_shexp_mv.
 // Precision: the products of the leading parts and the small ones have sums of their own, and the leading
@@ -671,9 +672,6 @@ static int shexp_mv(int type, bool dual, const void* W1, const void* W2, int row
     FRT_LAUNCHED("shared expert");
     return kOk;
 }
-
-int quantize_q8(const float* x, int rows, int n, int8_t* xq, float* xd, _Float16* xhi, _Float16* xlo,
-                hipStream_t stream);
 
 // Whether a call of T tokens runs on the matrix cores (k_shexp_mm). F32 and F16 weights cost nine and six products each there and the activations a launch
 // for their planes, and a few workgroups share the work, so that a short call of little work is faster on

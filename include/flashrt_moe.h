@@ -144,7 +144,8 @@ int frt_moe_dispatch(void* stream, const int32_t* ids, int T, int K, int E, int3
 
 /* ---- prefill grouped expert GEMM (kernels/cuda/moe_q2.h:20-30 moe_q2::workspace_bytes, run).
  * yd [T*K][n]: slot t*K + k gets down(silu(gate x_t) * up x_t) of expert ids[t*K + k], expert e's
- * blob at experts + e * stride. yd_bf16 selects bf16 output. block64: x and h are quantized in Q8
+ * blob at experts + e * stride (both multiples of 16: blobs are read in pieces of 16 bytes; an arena's
+ * are multiples of 4096). yd_bf16 selects bf16 output. block64: x and h are quantized in Q8
  * blocks of 64 values instead of the CPU path's 32 (moe_q2.cu's AB = 64). Shapes: n and ff multiples
  * of 128 (moe_q2.cu:516-517), ff at most 4096; ff above 1024 takes fp32 yd only. FRT_ERR_SHAPE
  * otherwise. */

@@ -62,6 +62,16 @@ def test_dense_layer_workspace_grows_with_tokens(n, ff, K):
             assert b == sorted(b), (gtype, shared_ff, [T for T in range(1, 64) if b[T - 1] > b[T]])
 
 
+def test_noalloc_scratch_holds_dense_windows():
+    """Every window the allocation-free entry takes (T <= 4, T * K <= 63) of a layer with the widest dense shared
+    expert fits its static scratch."""
+    L = _lib.lib()
+    worst = max((L.frt_moe_layer_workspace_bytes(C.byref(_layer(1024, n, ff, K, gtype, 4096, 1)), T), n, ff, K, gtype, T)
+                for n in (512, 2560, 4096) for ff in (256, 640, 1024) for gtype in (0, 8) for T in (1, 2, 3, 4)
+                for K in range(1, 33) if T * K <= 63)
+    assert 0 < worst[0] <= L.frt_noalloc_scratch_bytes(), worst
+
+
 @pytest.mark.parametrize("E,K", [(1, 1), (2, 2), (7, 3), (8, 8), (64, 8), (128, 1), (512, 10), (1025, 1)])
 def test_grouped_workspaces_grow_with_tokens(E, K):
     """The workspaces of the dispatch alone, the grouped expert products and a prefill layer never shrink as the
