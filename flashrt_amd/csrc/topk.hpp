@@ -135,13 +135,42 @@ __device__ __forceinline__ int lanes_below(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0));
 }
 
+// The K best of the lanes' V values each (lane l: experts V l ..) in rank order by K rounds of wave maxima over
+// the lanes' sorted lists; take(k, logit, id) runs in every lane. The ids are distinct: a lane whose list is used
+// up takes no further part (its -inf would tie with other lanes' -inf logits, masked experts, and give its last
+// id again, which the windows' grouping cannot take).
+template <int V, class F>
+__device__ __forceinline__ void topk_rounds(float (&v)[V], int K, F take) {
+    const int lane = threadIdx.x & 63;
+    int id[V], left = V;
+#pragma unroll
+    for (int i = 0; i < V; ++i) id[i] = V * lane + i;
+    sort_desc<V>(v, id);
+    for (int k = 0; k < K; ++k) {
+        const float m = wave_max(v[0]);   // (a used-up list's v[0] is -inf)
+        const uint64_t b = __ballot(left > 0 && v[0] == m);
+        const int win = __ffsll((long long)b) - 1;   // ties: the lowest lane, whose ids are the lowest
+        const int sel = __builtin_amdgcn_readlane(id[0], win);
+        if (lane == win) {
+#pragma unroll
+            for (int i = 0; i + 1 < V; ++i) {
+                v[i] = v[i + 1];
+                id[i] = id[i + 1];
+            }
+            v[V - 1] = -INFINITY;
+            --left;
+        }
+        take(k, m, sel);
+    }
+}
+
 // Top-K (K <= 64) of one token's E <= 64 V logits by one wave. cand: 64 floats + 64 ints of LDS
 // scratch for this wave. On return lane k < K holds the k-th selection (sel_id, sel_l) in rank
 // order; mx is the largest logit and se this lane's share of sum_e exp(l_e - mx).
 // Method: lane l holds experts V l .. V l + V - 1. The K best lane maxima (bitonic sort of the 64
 // lane maxima) are K distinct logits, so every member of the top K ranks at or above the K-th of
 // them; the (few) logits that do are compacted and sorted. Should more than 64 tie there (coarse,
-// heavily tied logits), K rounds of wave maxima over the lanes' sorted lists do the selection.
+// heavily tied logits), topk_rounds does the selection.
 template <int V>
 __device__ __forceinline__ void topk_select(const float* __restrict__ l, int E, int K, float* cand_v, int* cand_id,
                                            int& sel_id, float& sel_l, float& mx, float& se) {
@@ -219,31 +248,14 @@ __device__ __forceinline__ void topk_select(const float* __restrict__ l, int E, 
         sel_id = lane < K ? cand_id[lane] : 0;
         return;
     }
-    // heavily tied logits: K rounds over the lanes' sorted lists
-    int id[V];
-#pragma unroll
-    for (int i = 0; i < V; ++i) id[i] = V * lane + i;
-    sort_desc<V>(v, id);
     sel_id = 0;
     sel_l = 0.0f;
-    for (int k = 0; k < K; ++k) {
-        const float m = wave_max(v[0]);
-        const uint64_t b = __ballot(v[0] == m);
-        const int win = __ffsll((long long)b) - 1;
-        const int sel = __builtin_amdgcn_readlane(id[0], win);
-        if (lane == win) {
-#pragma unroll
-            for (int i = 0; i + 1 < V; ++i) {
-                v[i] = v[i + 1];
-                id[i] = id[i + 1];
-            }
-            v[V - 1] = -INFINITY;
-        }
+    topk_rounds<V>(v, K, [&](int k, float m, int sel) {
         if (lane == k) {
             sel_id = sel;
             sel_l = m;
         }
-    }
+    });
 }
 
 // The K weights from a selection (lane k holds the k-th), moe_ref.cu:146-164: p = exp(l - mx) / S
@@ -370,8 +382,8 @@ __device__ __forceinline__ int topk_wave_fast(const float* __restrict__ l, int E
 //   2. the logits that rank at or above tv are the candidates (at least K, typically a few more);
 //      wave 0 compacts them into LDS; each candidate's rank among them is again split over the
 //      group; ranks < K are the selection, written in rank order to sel_v / sel_id.
-//   (More than 64 candidates, only with coarse heavily tied logits: wave 0 selects by K rounds of
-//   wave maxima, as topk_select does.)
+//   (More than 64 candidates, only with coarse heavily tied logits: wave 0 selects by topk_rounds, as
+//   topk_select does.)
 // Every wave of the workgroup must call this the same number of times (it holds __syncthreads);
 // a group with no token passes active = false. mx (the largest logit) comes back in every wave of
 // the group.
@@ -487,30 +499,13 @@ __device__ __forceinline__ void topk_group4(const float* __restrict__ l, int E, 
         }
     } else {
         __syncthreads();
-        if (active && q == 0) {   // heavily tied logits: K rounds over the lanes' sorted lists
-            int id[V];
-#pragma unroll
-            for (int i = 0; i < V; ++i) id[i] = V * lane + i;
-            sort_desc<V>(v, id);
-            for (int k = 0; k < K; ++k) {
-                const float m = wave_max(v[0]);
-                const uint64_t b = __ballot(v[0] == m);
-                const int win = __ffsll((long long)b) - 1;
-                const int sel = __builtin_amdgcn_readlane(id[0], win);
-                if (lane == win) {
-#pragma unroll
-                    for (int i = 0; i + 1 < V; ++i) {
-                        v[i] = v[i + 1];
-                        id[i] = id[i + 1];
-                    }
-                    v[V - 1] = -INFINITY;
-                }
+        if (active && q == 0)
+            topk_rounds<V>(v, K, [&](int k, float m, int sel) {
                 if (lane == 0) {
                     S.sel_v[k] = m;
                     S.sel_id[k] = sel;
                 }
-            }
-        }
+            });
     }
     __syncthreads();
 }

@@ -1140,6 +1140,47 @@ def test_decode_routing_edge_logits(F, case):
         assert H.out_rel(out, ref) <= H.OUT_REL, (case, T)
 
 
+SINGLE_TOKEN_ROUTES = [(1, 0), (8, 0), (1, 1)]   # options (route_waves, decode_xcd): the single token's routings
+
+
+@pytest.mark.parametrize("E,K,finite", [(512, 10, 1), (512, 10, 9), (512, 32, 3), (1000, 32, 1), (40, 32, 5)])
+@pytest.mark.parametrize("shared", ["q2", "dense"])
+def test_routing_few_finite_logits(F, E, K, finite, shared):
+    """Fewer finite logits than selections (-inf biases: masked experts), through every routing kernel: the rest of
+    the selection are the lowest masked ids, each once (one lane of the selection holds only 8 or 16 of them),
+    with weight 0: ids and weights the oracle's, outputs 2e-3 up to 8 tokens. The grouped products of 24 tokens sum
+    h in another order, so that a code of h may move a step, and few experts carry the output: the bound of a
+    single expert's rows there (test_moe_q2_run_tile_edges)."""
+    b = np.full(E, -np.inf, np.float32)
+    b[np.random.default_rng(E + K).permutation(E)[:finite]] = np.arange(finite) * 0.5
+    kw = dict(cfg=0, n=1024, ff=256, E=E, K=K, bias=b)
+    w = H.World(**kw) if shared == "q2" else _dense_world(H.GGML_Q8_0, 64, 3, **kw)
+    w.router_w.zero_()
+    w.router_h[:] = 0.0
+    for T in (1, 2, 3, 4, 5, 8, 24):
+        print(f"E {E} K {K} finite {finite} {shared} T {T}", flush=True)
+        x = np.random.default_rng(T).standard_normal((T, w.n)).astype(np.float32)
+        ref, rid, rw, _ = O.moe_layer(w.arena_h, w.stride, E, w.shared_h if shared == "q2" else w.dense, w.router_h, b,
+                                      w.gate_h, w.n, w.ff, K, x, threads=8)
+        nz = rw != 0
+        for waves, xcd in SINGLE_TOKEN_ROUTES if T == 1 and shared == "q2" else SINGLE_TOKEN_ROUTES[:1]:
+            try:
+                F.set_option("route_waves", waves)
+                F.set_option("decode_xcd", xcd)
+                out, ids, wts = w.gpu_forward(x)
+            finally:
+                F.set_option("route_waves", 1)
+                F.set_option("decode_xcd", 0)
+            assert np.array_equal(ids, rid), (T, waves, xcd)
+            assert np.array_equal(wts[~nz], rw[~nz]) and H.w_rel(wts[nz], rw[nz]) <= H.W_REL, (T, waves, xcd)
+            assert H.out_rel(out, ref) <= (H.OUT_REL if T <= 8 else max(H.OUT_REL, 0.1 / w.ff ** 0.5)), (T, waves, xcd)
+    ids = torch.full((4, K), -1, dtype=torch.int32, device="cuda")
+    wts = torch.empty((4, K), dtype=torch.float32, device="cuda")
+    F.moe_route_topk(None, dev(np.tile(b, (4, 1))), 4, E, K, ids, wts)
+    torch.cuda.synchronize()
+    assert np.array_equal(ids.cpu().numpy(), O.route_topk(np.tile(b, (4, 1)), K)[0])
+
+
 def test_layer_errors(F, w0):
     x = torch.zeros((1, H.N), dtype=torch.float32, device="cuda")
     out = torch.zeros((1, H.N), dtype=torch.float32, device="cuda")
