@@ -271,7 +271,7 @@ __global__ void __launch_bounds__(kNT1) k_dec1(Dec1Args a_byval) {
     }
     }
     __syncthreads();
-    if (R.many) {   // more than 64 candidates (heavily tied logits): four waves select, as window_entries
+    if (R.many) {   // more than 64 candidates (heavily tied logits) or a NaN: four waves select, as window_entries
         float mx;
         topk_group4<V>(s_lg, E, K, wave & 3, wave < 4, R.tk[0], mx);
         if (wave == 0) {

@@ -374,7 +374,7 @@ __global__ void __launch_bounds__(kNT2) k_dec2(Dec2Args a_byval) {
     }
     FRT_D2_STAMP(11);
     __syncthreads();
-    if (R.many) {   // more than 64 candidates (heavily tied logits): four waves select, as window_entries
+    if (R.many) {   // more than 64 candidates (heavily tied logits) or a NaN: four waves select, as window_entries
         float mx;
         topk_group4<V>(s_lg, E, K, wave & 3, wave < 4, R.tk[0], mx);
         if (wave == 0) {

@@ -84,7 +84,7 @@ struct DecComb {
 
 struct WinLds {
     DecEntry ent[64];
-    int32_t many;   // the one-wave selection of a single token found more than 64 candidates
+    int32_t many;   // the one-wave selection of a single token found more than 64 candidates or a NaN
     int32_t ids[kDecMaxT][32];
     float w[kDecMaxT][32];
     DecComb comb;
@@ -105,8 +105,8 @@ struct WinLds {
 //   3. only this workgroup's entry (blockIdx.y) is written, with the rank in slot[0] (w[0]: the
 //      selected logit; the weight is formed later, single_weights, while the weight rows load); the
 //      ids and logits in rank order go to L.ids and L.w.
-// More than 64 candidates (heavily tied logits) sets L.many and writes nothing else; the caller
-// then runs the four-wave path. gl is the shared gate logit in lane 0. ALL: every entry is written
+// More than 64 candidates (heavily tied logits), fewer than K or a NaN among them (topk_wave_fast) sets L.many
+// and writes nothing else; the caller then runs the four-wave path. gl is the shared gate logit in lane 0. ALL: every entry is written
 // (the persistent single-token layer, where each workgroup needs the whole list).
 template <int V, bool ALL = false>
 __device__ __forceinline__ void route1_wave(const float (&v)[V], int E, int K, float gl,
@@ -126,7 +126,7 @@ __device__ __forceinline__ void route1_wave(const float (&v)[V], int E, int K, f
     for (int i = 0; i < V; ++i) c += int(key[i] != 0u && key[i] >= t1);
     int C;
     int pos = wave_excl_scan(c, &C);
-    if (C > 64) {
+    if (C > 64 || C < K) {
         if (lane == 0) L.many = 1;
         return;
     }
@@ -141,6 +141,10 @@ __device__ __forceinline__ void route1_wave(const float (&v)[V], int E, int K, f
     const bool cl = lane < C;
     const float cv = cl ? S.cand_v[lane] : 0.0f;
     const int ci = cl ? S.cand_id[lane] : 0x7fffffff;
+    if (__ballot(cv != cv)) {
+        if (lane == 0) L.many = 1;
+        return;
+    }
     // rank among the candidates: those ahead by logit, or equal and lower id (= lower slot); each
     // candidate's logit broadcast from its lane (no LDS round trip per step); float order with
     // -0 == +0 is the keys' order
@@ -195,8 +199,7 @@ __device__ __forceinline__ void route1_wave(const float (&v)[V], int E, int K, f
 //      lower bound on the K-th largest key of all E (a wave with K keys >= t puts K keys >= t in all);
 //   2. each wave compacts its keys >= T (every member of the top K) into LDS in ascending id;
 //   3. wave 0 takes the candidates, in ascending id, one per lane, and ranks them by logit (ties: the
-//      lower id, the lower position) as route1_wave does; more than 64 candidates (heavily tied
-//      logits) sets L.many.
+//      lower id, the lower position) as route1_wave does, and sets L.many where it does.
 // Every wave of the workgroup calls it (it holds barriers). A wave may start as soon as its own
 // lanes' logits are in s_lg (each lane reads only the word at its expert); s_lg[E] (the shared gate
 // logit) is read by wave 0 after the first barrier.
@@ -239,13 +242,13 @@ __device__ __forceinline__ void route_8waves(const float* s_lg, int E, int K, co
         }
         C += cw;
     }
-    if (C > 64) {
-        if (lane == 0) L.many = 1;
-        return;
-    }
     const bool cl = lane < C;
     const float cv = cl ? Q.v[sw][si] : 0.0f;
     const int ci = cl ? Q.id[sw][si] : 0x7fffffff;
+    if (C > 64 || C < K || __ballot(cv != cv)) {
+        if (lane == 0) L.many = 1;
+        return;
+    }
     int rank = 0;   // candidates ahead: higher logit, or equal and lower id (= lower position)
     for (int j = 0; j < C; ++j) {
         const float o = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cv), j));

@@ -106,8 +106,8 @@ __device__ __forceinline__ int wave_excl_scan(int c, int* total) {
 }
 
 // Order key of a logit: unsigned comparison of keys is float comparison of logits, with -0 and +0
-// equal (for finite and infinite values; NaN is not a logit). Key 0 is below every logit and marks
-// an empty lane.
+// equal (for finite and infinite values; a NaN's key is above +inf's or below -inf's, by its sign, and callers
+// leave a selection that meets one to topk_rounds). Key 0 is below every logit and marks an empty lane.
 __device__ __forceinline__ uint32_t logit_key(float f) {
     uint32_t u = __builtin_bit_cast(uint32_t, f);
     u = u == 0x80000000u ? 0u : u;
@@ -136,15 +136,18 @@ __device__ __forceinline__ int lanes_below(uint64_t m) {
 }
 
 // The K best of the lanes' V values each (lane l: experts V l ..) in rank order by K rounds of wave maxima over
-// the lanes' sorted lists; take(k, logit, id) runs in every lane. The ids are distinct: a lane whose list is used
-// up takes no further part (its -inf would tie with other lanes' -inf logits, masked experts, and give its last
-// id again, which the windows' grouping cannot take).
+// the lanes' sorted lists; take(k, logit, id) runs in every lane. A NaN ranks with -inf. The ids are distinct
+// whatever the logits hold: a lane whose list is used up takes no further part (its -inf would tie with other
+// lanes' -inf logits, masked experts, and give its last id again, which the windows' grouping cannot take).
 template <int V, class F>
 __device__ __forceinline__ void topk_rounds(float (&v)[V], int K, F take) {
     const int lane = threadIdx.x & 63;
     int id[V], left = V;
 #pragma unroll
-    for (int i = 0; i < V; ++i) id[i] = V * lane + i;
+    for (int i = 0; i < V; ++i) {
+        id[i] = V * lane + i;
+        v[i] = v[i] == v[i] ? v[i] : -INFINITY;
+    }
     sort_desc<V>(v, id);
     for (int k = 0; k < K; ++k) {
         const float m = wave_max(v[0]);   // (a used-up list's v[0] is -inf)
@@ -170,7 +173,7 @@ __device__ __forceinline__ void topk_rounds(float (&v)[V], int K, F take) {
 // Method: lane l holds experts V l .. V l + V - 1. The K best lane maxima (bitonic sort of the 64
 // lane maxima) are K distinct logits, so every member of the top K ranks at or above the K-th of
 // them; the (few) logits that do are compacted and sorted. Should more than 64 tie there (coarse,
-// heavily tied logits), topk_rounds does the selection.
+// heavily tied logits), or fewer than K rank there (NaN among the logits), topk_rounds does the selection.
 template <int V>
 __device__ __forceinline__ void topk_select(const float* __restrict__ l, int E, int K, float* cand_v, int* cand_id,
                                            int& sel_id, float& sel_l, float& mx, float& se) {
@@ -215,7 +218,7 @@ __device__ __forceinline__ void topk_select(const float* __restrict__ l, int E, 
     }
     int C;
     int pos = wave_excl_scan(c, &C);
-    if (C <= 64) {
+    if (C <= 64 && C >= K) {
 #pragma unroll
         for (int i = 0; i < V; ++i) {
             const int e = V * lane + i;
@@ -303,7 +306,8 @@ __device__ __forceinline__ int topk_wave(const float* __restrict__ l, int E, int
 // a lower bound on the K-th largest lane maximum (ballot counts over the keys' upper 12 bits) makes
 // every member of the top K a candidate; the candidates, compacted in ascending id, are ranked by
 // logit (ties: lower id first) and scattered by rank. The weights are topk_weight_sel's (the max is
-// the rank-0 logit). More than 64 candidates (heavily tied logits) falls back to topk_wave.
+// the rank-0 logit). More than 64 candidates (heavily tied logits) falls back to topk_wave; so do a NaN among
+// them and fewer than K of them (a NaN's key is above every logit's, or below, or 0).
 // cand_v / cand_id: 128 entries each (64 candidates and one junk slot per lane).
 template <int V>
 __device__ __forceinline__ int topk_wave_fast(const float* __restrict__ l, int E, int K, int32_t* ids, float* wts,
@@ -336,20 +340,26 @@ __device__ __forceinline__ int topk_wave_fast(const float* __restrict__ l, int E
     for (int i = 0; i < V; ++i) c += int(key[i] != 0u && key[i] >= t1);
     int C;
     int pos = wave_excl_scan(c, &C);
-    if (C > 64) return topk_wave<V>(l, E, K, ids, wts, cand_v, cand_id);
-#pragma unroll
-    for (int i = 0; i < V; ++i) {   // branch-free compaction: a non-candidate goes to junk slot 64 + lane
-        const bool is_c = key[i] != 0u && key[i] >= t1;
-        const int slot = is_c ? pos : 64 + lane;
-        cand_v[slot] = v[i];
-        cand_id[slot] = V * lane + i;
-        pos += int(is_c);
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
     const bool cl = lane < C;
-    const float cv = cl ? cand_v[lane] : 0.0f;
-    const int ci = cl ? cand_id[lane] : 0x7fffffff;
+    float cv = 0.0f;
+    int ci = 0x7fffffff;
+    bool ok = C <= 64 && C >= K;
+    if (ok) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) {   // branch-free compaction: a non-candidate goes to junk slot 64 + lane
+            const bool is_c = key[i] != 0u && key[i] >= t1;
+            const int slot = is_c ? pos : 64 + lane;
+            cand_v[slot] = v[i];
+            cand_id[slot] = V * lane + i;
+            pos += int(is_c);
+        }
+        __builtin_amdgcn_s_waitcnt(0);
+        __builtin_amdgcn_wave_barrier();
+        cv = cl ? cand_v[lane] : 0.0f;
+        ci = cl ? cand_id[lane] : 0x7fffffff;
+        ok = __ballot(cv != cv) == 0;
+    }
+    if (!ok) return topk_wave<V>(l, E, K, ids, wts, cand_v, cand_id);
     int rank = 0;   // candidates ahead: higher logit, or equal and lower id (= lower slot)
     for (int j = 0; j < C; ++j) {
         const float o = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cv), j));
@@ -382,8 +392,8 @@ __device__ __forceinline__ int topk_wave_fast(const float* __restrict__ l, int E
 //   2. the logits that rank at or above tv are the candidates (at least K, typically a few more);
 //      wave 0 compacts them into LDS; each candidate's rank among them is again split over the
 //      group; ranks < K are the selection, written in rank order to sel_v / sel_id.
-//   (More than 64 candidates, only with coarse heavily tied logits: wave 0 selects by topk_rounds, as
-//   topk_select does.)
+//   (More than 64 candidates, only with coarse heavily tied logits, or fewer than K, with NaN among
+//   the logits: wave 0 selects by topk_rounds, as topk_select does.)
 // Every wave of the workgroup must call this the same number of times (it holds __syncthreads);
 // a group with no token passes active = false. mx (the largest logit) comes back in every wave of
 // the group.
@@ -443,8 +453,8 @@ __device__ __forceinline__ void topk_group4(const float* __restrict__ l, int E, 
     if (active) S.part[q][lane] = cnt;
     __syncthreads();
     const int rank = S.part[0][lane] + S.part[1][lane] + S.part[2][lane] + S.part[3][lane];
-    const int kl = __ffsll((long long)__ballot(rank == K - 1)) - 1;
-    const int l0 = __ffsll((long long)__ballot(rank == 0)) - 1;
+    const int kl = (__ffsll((long long)__ballot(rank == K - 1)) - 1) & 63;   // (no such lane: NaN among the maxima)
+    const int l0 = (__ffsll((long long)__ballot(rank == 0)) - 1) & 63;
     const float tv = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lm), kl));
     const int tid = __builtin_amdgcn_readlane(li, kl);
     mx = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lm), l0));
@@ -466,7 +476,7 @@ __device__ __forceinline__ void topk_group4(const float* __restrict__ l, int E, 
         }
     }
     __syncthreads();
-    if (C <= 64) {
+    if (C <= 64 && C >= K) {
         const float cv = lane < C ? S.cand_v[lane] : -INFINITY;
         const int ci = lane < C ? S.cand_id[lane] : 0x7fffffff;
         // this wave's 16 candidates as four 16-byte LDS reads of each array (same address in every

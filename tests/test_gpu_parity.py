@@ -1181,6 +1181,50 @@ def test_routing_few_finite_logits(F, E, K, finite, shared):
     assert np.array_equal(ids.cpu().numpy(), O.route_topk(np.tile(b, (4, 1)), K)[0])
 
 
+@pytest.mark.parametrize("E,K", [(512, 10), (1000, 32), (40, 10)])
+@pytest.mark.parametrize("bits", [0x7FC00000, 0xFFC00000, 0xFFFFFFFF])
+@pytest.mark.parametrize("shared", ["q2", "dense"])
+def test_routing_nan_logits(F, E, K, bits, shared):
+    """NaN logits rank with -inf: a token of NaN selects K distinct experts in range and leaves the other tokens of
+    its call as they are (the bounds of test_routing_few_finite_logits); experts whose logit alone is NaN (a NaN
+    bias) are not selected."""
+    some = np.random.default_rng(E).permutation(E)[:20]
+    for bias_nan in (False, True):
+        b = np.zeros(E, np.float32)
+        if bias_nan:
+            b.view(np.uint32)[some] = bits
+        kw = dict(cfg=0, n=1024, ff=256, E=E, K=K, bias=b)
+        w = H.World(**kw) if shared == "q2" else _dense_world(H.GGML_Q8_0, 64, 3, **kw)
+        for T in (1, 2, 3, 4, 5, 8, 24):
+            print(f"E {E} K {K} bits {bits:x} {shared} bias {bias_nan} T {T}", flush=True)
+            x = np.random.default_rng(T).standard_normal((T, w.n)).astype(np.float32)
+            if not bias_nan:
+                x.view(np.uint32)[T // 2] = bits
+            xd, out = dev(x), torch.empty((T, w.n), dtype=torch.float32, device="cuda")
+            ids = torch.full((T, K), -1, dtype=torch.int32, device="cuda")
+            cnt = torch.zeros(E, dtype=torch.int32, device="cuda")
+            lg = O.router_logits(x, w.router_h, b)
+            ref = np.argsort(-np.where(np.isnan(lg), -np.inf, lg), axis=1, kind="stable")[:, :K]
+            for waves, xcd in SINGLE_TOKEN_ROUTES if T == 1 and shared == "q2" else SINGLE_TOKEN_ROUTES[:1]:
+                ids.fill_(-1)
+                cnt.zero_()
+                try:
+                    F.set_option("route_waves", waves)
+                    F.set_option("decode_xcd", xcd)
+                    w.layer_obj.forward(xd, out, T=T, ids=ids, counts=cnt)
+                finally:
+                    F.set_option("route_waves", 1)
+                    F.set_option("decode_xcd", 0)
+                assert np.array_equal(ids.cpu().numpy(), ref), (T, waves, xcd)
+                assert np.array_equal(cnt.cpu().numpy(), np.bincount(ref.reshape(-1), minlength=E)), (T, waves, xcd)
+            out = out.cpu().numpy()
+            if not bias_nan and T > 1:
+                ok = np.arange(T) != T // 2
+                r = O.moe_layer(w.arena_h, w.stride, E, w.shared_h if shared == "q2" else w.dense, w.router_h, b,
+                                w.gate_h, w.n, w.ff, K, x[ok], threads=8)[0]
+                assert H.out_rel(out[ok], r) <= (H.OUT_REL if T <= 8 else max(H.OUT_REL, 0.1 / w.ff ** 0.5)), T
+
+
 def test_layer_errors(F, w0):
     x = torch.zeros((1, H.N), dtype=torch.float32, device="cuda")
     out = torch.zeros((1, H.N), dtype=torch.float32, device="cuda")
