@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """bench.py — flashrt's MoE-layer hot path on one MI355X.
 
-Headline (BASELINE.json configs[2]): a 48-layer stack of the Q2_0 512-expert top-10 MoE layer
+Headline: a 48-layer stack of the Q2_0 512-expert top-10 MoE layer
 (hidden 2048, expert ff 512, shared expert ff 512), all experts resident in HBM, decode at bs=1.
 A step is one token through the 48 layers (x_{l+1} = x_l + moe_l(rms_norm(x_l)), the pre-MoE
 RMS norm without weight keeping the chained residual stream bounded); each step's input is a
@@ -11,7 +11,7 @@ the experts. The 48 layers of one step are captured once as a HIP graph and repl
 Also measured in the same run:
   - per-kernel durations (hipEvents on the launch stream, eager run) and the roofline of the
     dominant kernel: algorithmic expert bytes per launch / its average duration vs 8 TB/s;
-  - configs[3]: one layer, 2048-token prefill (bf16 inputs, Zipf(1.2) prior): tokens/s and the
+  - one layer, 2048-token prefill (bf16 inputs, Zipf(1.2) prior): tokens/s and the
     grouped GEMM kernels' MFMA utilisation against the 2.5 PFLOP/s dense fp16 peak;
   - cpu_baseline: the reference's own CPU MoE (moe_cpu over its CpuPool, AVX-512 VNNI; built from
     its sources into oracle/_ref) on a bounded sample of the same workload on this host.
@@ -176,7 +176,7 @@ def run_stack(args, F, torch):
 # ---------------------------------------------------------------- config 3: 2K prefill
 
 def build_layer(F, torch, cfg, bias_np=None):
-    """One layer of BASELINE configs[cfg]: its own arena (E experts), shared expert, router, gate."""
+    """One layer of the generator's configuration cfg: its own arena (E experts), shared expert, router, gate."""
     eb = F.expert_bytes(N, FF)
     stride = (eb + 4095) // 4096 * 4096
     g = F.gen
@@ -238,7 +238,7 @@ def time_prefill_layer(F, torch, ml, x, reps):
 
 
 def run_prefill(args, F, torch):
-    """one layer, 2048 bf16 tokens, Zipf(1.2) popularity."""
+    """One layer, 2048 bf16 tokens, Zipf(1.2) popularity."""
     ml = build_layer(F, torch, 3, F.gen.zipf_bias(3, 0, E, ZIPF_PREFILL, PREFILL_ALPHA))
     x = torch.empty((2048, N), dtype=torch.float32, device="cuda")
     F.gen.normal(x, 3, 0, F.gen.X_TENSOR, 1.0, round_bf16=True)
@@ -248,7 +248,7 @@ def run_prefill(args, F, torch):
 
 
 def run_mixed(args, F, torch):
-    """configs[4]: one launch of 8192 bf16 prefill tokens plus 16 uncorrelated fp32 decode tokens;
+    """One launch of 8192 bf16 prefill tokens plus 16 uncorrelated fp32 decode tokens;
     +2.8 on the logits of 16 seeded hot experts puts about 90% of the selections on them."""
     hot = np.random.default_rng(4).permutation(E)[:16]
     bias = np.zeros(E, np.float32)
@@ -263,8 +263,8 @@ def run_mixed(args, F, torch):
 
 
 def run_windows(args, F, torch, st):
-    """configs[0] (T = 1) and configs[1] (T = 3, pairwise cosine 0.8) as single-layer calls, and the
-    other verify-window sizes T = 2, 5, 8: configs[0]-shaped layers (no prior, no input norm) over
+    """A single token (T = 1) and a window of T = 3 (pairwise cosine 0.8) as single-layer calls, and the
+    other verify-window sizes T = 2, 5, 8: layers of the benchmark shape (no prior, no input norm) over
     the 48 layers of the stack's arena, one call per layer captured as a graph and replayed, so that
     every call streams its experts from HBM as a lone layer call would. Per T: us per call and the
     HBM rate on the bytes the call must read (its distinct routed experts + shared + router)."""
@@ -485,9 +485,9 @@ def main():
                     help="first run 3 plain device copies of MIB MiB (scales the HBM byte counters of a profile)")
     ap.add_argument("--timing-steps", type=int, default=3, help="decode steps in the per-kernel timing pass")
     ap.add_argument("--no-prefill", action="store_true")
-    ap.add_argument("--no-windows", action="store_true", help="skip configs[0]/[1] and the other window sizes")
+    ap.add_argument("--no-windows", action="store_true", help="skip the single-layer calls of 1, 3 and other window sizes")
     ap.add_argument("--window-reps", type=int, default=8, help="replays of the 48-call graph per window size")
-    ap.add_argument("--no-mixed", action="store_true", help="skip configs[4]")
+    ap.add_argument("--no-mixed", action="store_true", help="skip the mixed prefill + decode launch")
     ap.add_argument("--decode-grid", type=int, default=0, help="workgroups of a persistent decode call (0: one per CU)")
     ap.add_argument("--decode-xcd", type=int, default=0,
                     help="1: persistent single-token calls split each layer by XCD (decode2.hip) where the shape "

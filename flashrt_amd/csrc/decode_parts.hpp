@@ -106,8 +106,8 @@ struct WinLds {
 //      selected logit; the weight is formed later, single_weights, while the weight rows load); the
 //      ids and logits in rank order go to L.ids and L.w.
 // More than 64 candidates (heavily tied logits), fewer than K or a NaN among them (topk_wave_fast) sets L.many
-// and writes nothing else; the caller then runs the four-wave path. gl is the shared gate logit in lane 0. ALL: every entry is written
-// (the persistent single-token layer, where each workgroup needs the whole list).
+// and writes nothing else; the caller then runs the four-wave path. gl is the shared gate logit in lane 0. ALL:
+// every entry is written (the persistent single-token layer, where each workgroup needs the whole list).
 template <int V, bool ALL = false>
 __device__ __forceinline__ void route1_wave(const float (&v)[V], int E, int K, float gl,
                                             const uint8_t* __restrict__ arena, size_t stride,

@@ -1,4 +1,4 @@
-// Decode windows of 2-4 tokens (speculative verify batches, configs[1]) as ONE persistent launch.
+// Decode windows of 2-4 tokens (speculative verify batches) as ONE persistent launch.
 //
 // The window path of decode.hip runs a window as four launches (router + Q8_0, routing and grouping
 // in one workgroup, gate/up per entry, down + combine). This kernel runs the same steps in one grid
@@ -38,10 +38,11 @@ namespace {
 constexpr int kNTW = kNTP;          // threads per workgroup
 constexpr int kNWW = kNTW / 64;     // waves per workgroup
 // The kernel is written for windows of up to 8 tokens (the reference's kMaxWindow; entries of at most
-// 4 tokens, k_win_route's split) and takes those of 2-4 tokens. Measured on configs[1]-like windows (same box, the four-launch path
-// beside it): T = 2 26.2 -> 23.5 us, T = 3 29.1 -> 25.8; but T = 5 35.9 -> 37.0 and T = 8 46.4 -> 47.7
-// (at T = 8 each workgroup runs about 5 gate/up units one after another, where the four-launch
-// path spreads them over 3 workgroups of 4 waves per CU), so larger windows keep the four launches.
+// 4 tokens, k_win_route's split) and takes those of 2-4 tokens. Measured on windows of correlated tokens at
+// 2048 / 512, 512 experts (same session, the four-launch path beside it): T = 2 26.2 -> 23.5 us, T = 3 29.1 ->
+// 25.8; but T = 5 35.9 -> 37.0 and T = 8 46.4 -> 47.7 (at T = 8 each workgroup runs about 5 gate/up units one
+// after another, where the four-launch path spreads them over 3 workgroups of 4 waves per CU), so larger windows
+// keep the four launches.
 constexpr int kWUseT = 4;
 constexpr int kWLgStride = 4;       // words between two published logits (as k_dec1)
 // logit and h words per thread to wait for, for windows of at most MT tokens: T (E + 1) logits,
@@ -417,7 +418,7 @@ __global__ void __launch_bounds__(kNTW) k_decw(DecwArgs a_byval) {
         }
         __syncthreads();   // s_h is free for the next unit
     };
-    // a window has more units than workgroups (about 21 entries x ff / 32 at configs[1], 5 units per
+    // a window has more units than workgroups (about 21 entries x ff / 32 at three tokens of 2048 / 512, 5 units per
     // workgroup at T = 8): two register sets in turn, unit i + 1's rows in flight while unit i computes
     {
         GuRegs g0, g1;

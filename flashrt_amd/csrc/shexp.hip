@@ -673,9 +673,9 @@ static int shexp_mv(int type, bool dual, const void* W1, const void* W2, int row
     return kOk;
 }
 
-// Whether a call of T tokens runs on the matrix cores (k_shexp_mm). F32 and F16 weights cost nine and six products each there and the activations a launch
-// for their planes, and a few workgroups share the work, so that a short call of little work is faster on
-// k_shexp_mv, whose time goes with the tokens. A whole layer, k_shexp_mv / k_shexp_mm in us, F16, shared width x
+// Whether a call of T tokens runs on the matrix cores (k_shexp_mm). F32 and F16 weights cost nine and six
+// products each there and the activations a launch for their planes, and a few workgroups share the work, so that
+// a short call of little work is faster on k_shexp_mv, whose time goes with the tokens. A whole layer, k_shexp_mv / k_shexp_mm in us, F16, shared width x
 // hidden size: 4096 x 512 58 / 91 at 9 tokens, 81 / 92 at 20, 101 / 93 at 32; 4096 x 1024 70 / 108 at 9,
 // 105 / 107 at 20, 117 / 106 at 24; 2048 x 1536 at 24 97 / 91; 2048 x 4096 122 / 147 at 9, 158 / 148 at 16.
 // BF16 and Q8_0, three products and one, are faster on the matrix cores from 9 tokens on (0.64 to 0.85 and 0.65

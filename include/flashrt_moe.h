@@ -267,8 +267,8 @@ int frt_moe_layer_forward_noalloc(const frt_moe_layer* L, const float* x, int T,
 int frt_noalloc_sync_error(void* stream);
 
 /* ---- a stack of single-token MoE layers (no reference counterpart as one call: the engine calls
- * moe_block_fast once per layer, arch/qwen4exp/forward.cu:214-217; BASELINE config 2 is a stack of
- * MoE layers chained by the residual). x_0 = x, x_{l+1} = x_l + moe_l(x_l) with each layer's own
+ * moe_block_fast once per layer, arch/qwen4exp/forward.cu:214-217; here a stack of MoE layers
+ * chained by the residual). x_0 = x, x_{l+1} = x_l + moe_l(x_l) with each layer's own
  * flags (all layers share E, K, d_model, d_ff, stride and flags), out = x_{n_layer} [d_model].
  * ids/wts [n_layer][K] optional. Runs as one persistent launch per 64 layers ("decode_fused", the
  * default), else as n_layer calls of frt_moe_layer_forward; both give identical results. The last

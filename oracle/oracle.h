@@ -1,7 +1,7 @@
 /* CPU ORACLE — test infrastructure only.
  *
- * A clean-room restatement of flashrt's CPU MoE path, used as the checker for the HIP
- * library. Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may load it;
+ * A clean-room restatement of flashrt's CPU MoE path, which the tests hold the HIP library
+ * against. Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may load it;
  * the product path (flashrt_amd) never does.
  *
  * Every function cites the reference file:line whose semantics it restates. Parity status of
@@ -80,7 +80,7 @@ void orc_moe_cpu(int n, int ff, const uint8_t* const* blobs, const int* ntok, co
  * logits (canonical router) -> routing -> misses grouped per expert (<= 4 tokens each, token
  * order, experts ascending) -> moe_cpu -> + shared expert * sigmoid(gate logit) (moe_ref.cu:90-97).
  * Routed expert e of the layer is at arena + e*stride. The shared expert is a Q2_0 blob of the
- * same shape (the BASELINE configuration's choice). Outputs: out [T][n], ids/wts [T][K].
+ * same shape. Outputs: out [T][n], ids/wts [T][K].
  * norm_input: the layer runs on u = orc_rmsnorm(x) instead of x. */
 void orc_moe_layer(const uint8_t* arena, size_t stride, int E, const uint8_t* shared_blob, const float* router_w,
                    const float* router_bias, const float* gate_w, int n, int ff, int K, const float* x, int T,

@@ -1,7 +1,7 @@
 """Shared test helpers: one MoE layer's synthetic weights on the GPU and the same bytes on the host
 for the CPU oracle, plus the tolerances the parity tests use.
 
-Tolerances (from the north star in BASELINE.json):
+Tolerances:
   expert ids and the dispatch permutation: bit-exact;
   routing weights: relative error <= 1e-6;
   layer outputs: per token, max_i |gpu_i - ref_i| / max_i |ref_i| <= 2e-3 (fp32 accumulation).
@@ -15,7 +15,7 @@ from oracle import oracle as O
 W_REL = 1e-6
 OUT_REL = 2e-3
 
-# BASELINE.json configuration shapes
+# the benchmark layer's shape
 N, FF, E, K = 2048, 512, 512, 10
 # Zipf prior strengths of configs 2 and 3 (s) and config 3's alpha, chosen so that a 2048-token
 # chunk gives per-expert counts from 0 up to a few hundred
@@ -34,7 +34,7 @@ def w_rel(gpu: np.ndarray, ref: np.ndarray) -> float:
 
 
 class World:
-    """Layer `layer` of BASELINE config `cfg` (n, ff, E, K as given): expert arena, shared expert,
+    """Layer `layer` of the generator's configuration `cfg` (n, ff, E, K as given): expert arena, shared expert,
     router and gate weights generated on the GPU by flashrt_amd.gen, and host copies."""
 
     def __init__(self, cfg: int, layer: int = 0, n: int = N, ff: int = FF, E: int = E, K: int = K,

@@ -906,7 +906,7 @@ def test_layer_prefill_config3_all_rows(F):
     assert np.array_equal(ids, rid)
     g, r = out.astype(np.float64), ref.astype(np.float64)
     e = np.abs(g - r).max(axis=1) / np.abs(r).max(axis=1)
-    print(f"configs[3] all rows: median {np.median(e):.2e}, p99 {np.quantile(e, 0.99):.2e}, max {e.max():.2e}")
+    print(f"prefill of 2048 tokens, all rows: median {np.median(e):.2e}, p99 {np.quantile(e, 0.99):.2e}, max {e.max():.2e}")
     assert np.median(e) <= 5e-4 and np.quantile(e, 0.99) <= 1e-3
     assert e.max() <= H.OUT_REL
 
